@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace gj {
 
@@ -52,15 +53,50 @@ __device__ __forceinline__ int group_popc(uint64_t mask, int gbase) {
     return __popc(group_bits<G>(mask, gbase));
   }
 }
-// index (0-based, within the group) of the lowest set bit, or -1
-template <int G>
-__device__ __forceinline__ int group_ffs(uint64_t mask, int gbase) {
-  if constexpr (G == 64) {
-    return mask ? __ffsll(static_cast<unsigned long long>(mask)) - 1 : -1;
-  } else {
-    const uint32_t b = group_bits<G>(mask, gbase);
-    return b ? __ffs(b) - 1 : -1;
-  }
+// Quads: groups of four neighbouring lanes.  A quad-permute rides on an ordinary VALU
+// instruction (DPP), where a cross-lane read through the LDS crossbar (shfl) is an LDS
+// operation with its latency and a shared port.
+constexpr int kQuad = 4;
+template <int Ctrl>
+__device__ __forceinline__ uint32_t quad_perm32(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), Ctrl, 0xF, 0xF, true));
+}
+// the value of the quad's lane R, in all four lanes
+template <int R>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
+  return quad_perm32<R * 0x55>(v);
+}
+template <int R>
+__device__ __forceinline__ uint64_t quad_bcast(uint64_t v) {
+  const uint32_t lo = quad_bcast<R>(static_cast<uint32_t>(v));
+  const uint32_t hi = quad_bcast<R>(static_cast<uint32_t>(v >> 32));
+  return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+__device__ __forceinline__ uint32_t quad_sum(uint32_t v) {
+  v += quad_perm32<0xB1>(v);  // lanes 1 0 3 2
+  v += quad_perm32<0x4E>(v);  // lanes 2 3 0 1
+  return v;
+}
+__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
+  v |= quad_perm32<0xB1>(v);
+  v |= quad_perm32<0x4E>(v);
+  return v;
+}
+// A 16-byte register value left as it is: what a round that loads nothing compares.  (A
+// plain uninitialised variable would let the compiler assume anything of the result; a
+// zeroed one costs its moves on every step.)
+__device__ __forceinline__ u32x4 any_u32x4() {
+  u32x4 v;
+  asm volatile("" : "=v"(v));
+  return v;
+}
+// f(R) for R = 0 .. 3 as compile-time constants (the permute's control must be one)
+template <class F>
+__device__ __forceinline__ void quad_rounds(F&& f) {
+  f(std::integral_constant<int, 0>{});
+  f(std::integral_constant<int, 1>{});
+  f(std::integral_constant<int, 2>{});
+  f(std::integral_constant<int, 3>{});
 }
 
 // Streaming (non-temporal) load of one probe key.
@@ -80,8 +116,7 @@ struct Piece {
   K k[kKeys];
 };
 template <class K>
-__device__ __forceinline__ Piece<K> load_piece(const K* p) {
-  const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+__device__ __forceinline__ Piece<K> piece_of(u32x4 v) {
   Piece<K> r;
   if constexpr (sizeof(K) == 8) {
     r.k[0] = (static_cast<uint64_t>(v.y) << 32) | v.x;
@@ -94,14 +129,9 @@ __device__ __forceinline__ Piece<K> load_piece(const K* p) {
   }
   return r;
 }
-// Same, for the tail of a column: keys at or beyond `valid` are replaced by `fill`.
 template <class K>
-__device__ __forceinline__ Piece<K> load_piece_guarded(const K* p, int valid, K fill) {
-  Piece<K> r;
-  if (valid >= Piece<K>::kKeys) return load_piece(p);
-#pragma unroll
-  for (int j = 0; j < Piece<K>::kKeys; ++j) r.k[j] = (j < valid) ? p[j] : fill;
-  return r;
+__device__ __forceinline__ Piece<K> load_piece(const K* p) {
+  return piece_of<K>(*reinterpret_cast<const u32x4*>(p));
 }
 
 template <class K>

@@ -60,74 +60,126 @@ struct BSearchDev {
 };
 
 // ---------------------------------------------------------------------------
-// Cooperative 128-byte node search in groups of G = 8 lanes (8 x 16 B = one
-// 128-byte line).  Each lane owns one probe; the group serves its G probes
-// in G rounds: in round r all G lanes fetch their 16-byte slice of the node
-// of lane (gbase + r), and a ballot counts the keys below that lane's probe.
-// All G loads of a level are issued before any compare, so a level costs one
-// memory latency.  This is the CDNA form of Harmonia's leader rotation
-// (src/harmonia.cuh:561-599) with one full line per load instruction.  NB is the
-// node size in bytes (G = NB / 16 lanes per group): 128 by default, 64 or 256 for
-// the B-tree's other node sizes.
+// Cooperative search of NB-byte sorted lines (tree nodes, column lines, key lines)
+// by quads.  Each lane owns one probe; a quad serves its four probes in four rounds:
+// in round r its lanes fetch the line of lane r's probe, a quarter each, and each lane
+// counts its own keys below that probe.  All four rounds' loads are issued
+// before any compare, so a line step costs one memory latency.  The counts of the
+// four rounds sit in the bytes of one register, so two quad additions sum all of them
+// and lane r takes byte r.
+//
+// What bounds it: with every line in L2 the search is bound by VALU issue.  The form
+// before this one (groups of 8 lanes, probe and node fetched through the LDS crossbar,
+// one ballot, shift and population count per key) took about 230 instructions per line
+// step and 64 probes; this one takes about 75.  2^24 probes, plain driver, before and
+// after: B-tree over 2^20 u32 keys 449 -> 229 us, 2^20 u64 470 -> 322, 2^22 u64 557 -> 402;
+// hash over 2^14 u32 keys 179 -> 159; RadixSpline over 2^16 u64 keys 382 -> 337.  Beyond
+// L2 the bound is 55 G lines/s whatever the search (2^26 u64 keys: B-tree 3.12 -> 2.92 ms
+// per 2^26 probes).
 // ---------------------------------------------------------------------------
-template <class K, int G, int NB = 128>
-__device__ __forceinline__ uint32_t group_count_less(const K* level_base, uint64_t my_node, K my_x, int gbase,
-                                                     int gl) {
-  constexpr int NK = NB / static_cast<int>(sizeof(K));
-  constexpr int KPL = NK / G;
-  static_assert(KPL == Piece<K>::kKeys, "one 16-byte piece per lane");
-  Piece<K> pc[G];
+template <class K, int NB>
+struct QuadLine {
+  static constexpr int kPiece = Piece<K>::kKeys;               // keys per 16-byte piece
+  static constexpr int kPieces = NB / (16 * kQuad);            // pieces per lane
+  static constexpr int kLaneKeys = kPiece * kPieces;           // consecutive keys per lane
+  static constexpr int kKeys = NB / static_cast<int>(sizeof(K));
+  static_assert(kPieces >= 1 && kKeys < 128, "a round's count must fit its byte");
+  Piece<K> pc[kPieces];
+
+  // lane_base: the array of lines plus this lane's first key
+  __device__ __forceinline__ void load(const K* lane_base, uint64_t line) {
+    const K* p = lane_base + line * kKeys;
 #pragma unroll
-  for (int r = 0; r < G; ++r) {
-    const uint64_t nd = shfl64(my_node, gbase + r);
-    pc[r] = load_piece(level_base + nd * NK + gl * KPL);
+    for (int t = 0; t < kPieces; ++t) pc[t] = load_piece(p + t * kPiece);
   }
-  // each round's probe is fetched from its lane when compared (while the lines are in
-  // flight), so only the G lines stay live across the level: 108 -> 64 VGPRs for u64
-  // keys, 4 -> 8 waves per SIMD
-  uint32_t result = 0;
+  // whatever the registers hold, for the rounds that then load nothing and whose count is
+  // not looked at; all of a step's calls come before its loads, whose registers these are
+  __device__ __forceinline__ void any() {
 #pragma unroll
-  for (int r = 0; r < G; ++r) {
-    const K xr = shfl(my_x, gbase + r);
-    int cnt = 0;
-#pragma unroll
-    for (int j = 0; j < KPL; ++j) cnt += group_popc<G>(ballot(pc[r].k[j] < xr), gbase);
-    if (gl == r) result = static_cast<uint32_t>(cnt);
+    for (int t = 0; t < kPieces; ++t) pc[t] = piece_of<K>(any_u32x4());
   }
-  return result;
+  __device__ __forceinline__ uint32_t below(K x) const {
+    uint32_t c = 0;
+#pragma unroll
+    for (int t = 0; t < kPieces; ++t)
+#pragma unroll
+      for (int j = 0; j < kPiece; ++j) c += pc[t].k[j] < x ? 1u : 0u;
+    return c;
+  }
+  __device__ __forceinline__ bool holds(K x) const {
+    bool e = false;
+#pragma unroll
+    for (int t = 0; t < kPieces; ++t)
+#pragma unroll
+      for (int j = 0; j < kPiece; ++j) e |= pc[t].k[j] == x;
+    return e;
+  }
+};
+
+// The four probes of the lane's quad.
+template <class K>
+struct QuadProbes {
+  K x[kQuad];
+  __device__ __forceinline__ explicit QuadProbes(K mine) {
+    quad_rounds([&](auto r) { x[r] = quad_bcast<r>(mine); });
+  }
+};
+
+// Rank of each lane's probe in the line its quad loaded for it: keys below it, and
+// whether the line holds it.
+template <class K, int NB>
+__device__ __forceinline__ uint32_t quad_below(const QuadLine<K, NB> (&ln)[kQuad], const QuadProbes<K>& q, int ql) {
+  uint32_t c = 0;
+#pragma unroll
+  for (int r = 0; r < kQuad; ++r) c |= ln[r].below(q.x[r]) << (8 * r);
+  return (quad_sum(c) >> (8 * ql)) & 0xFFu;
+}
+template <class K, int NB>
+__device__ __forceinline__ bool quad_holds(const QuadLine<K, NB> (&ln)[kQuad], const QuadProbes<K>& q, int ql) {
+  uint32_t e = 0;
+#pragma unroll
+  for (int r = 0; r < kQuad; ++r) e |= ln[r].holds(q.x[r]) ? 1u << r : 0u;
+  return (quad_or(e) >> ql) & 1u;
 }
 
-// Equality search of each lane's probe in its NB-byte column chunk.
-template <class K, int G, int NB = 128>
-__device__ __forceinline__ uint32_t group_find_equal(const K* col, uint64_t n, uint64_t my_chunk, K my_x,
-                                                     bool my_live, int gbase, int gl) {
-  constexpr int NK = NB / static_cast<int>(sizeof(K));
-  constexpr int KPL = NK / G;
-  Piece<K> pc[G];
-#pragma unroll
-  for (int r = 0; r < G; ++r) {
-    const uint64_t chunk = shfl64(my_chunk, gbase + r);
-    const uint64_t start = chunk * NK + static_cast<uint64_t>(gl * KPL);
-    const int valid = (start >= n) ? 0 : ((n - start) >= static_cast<uint64_t>(KPL) ? KPL : static_cast<int>(n - start));
-    pc[r] = load_piece_guarded(col + start, valid, key_max<K>());
+// Keys below each lane's probe in line `line` of `base` (whole lines).
+template <class K, int NB>
+__device__ __forceinline__ uint32_t quad_count_less(const K* base, uint32_t line, const QuadProbes<K>& q, int ql) {
+  QuadLine<K, NB> ln[kQuad];
+  const K* lane_base = base + ql * QuadLine<K, NB>::kLaneKeys;
+  quad_rounds([&](auto r) { ln[r].load(lane_base, quad_bcast<r>(line)); });
+  return quad_below(ln, q, ql);
+}
+
+// The partial last line of a column of n keys holds fewer keys than a quad reads: the lane
+// walks it by itself, from position `at`.
+template <class K>
+__device__ __forceinline__ uint32_t tail_below(const K* col, uint64_t n, uint64_t at, K x, bool& eq) {
+  uint32_t b = 0;
+  while (at + b < n && col[at + b] < x) ++b;
+  eq = at + b < n && col[at + b] == x;
+  return b;
+}
+
+// Position of each lane's probe in its NB-byte chunk of the column, or not found.
+template <class K, int NB>
+__device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, uint32_t chunk, bool live, K x,
+                                                    const QuadProbes<K>& q, int ql) {
+  using L = QuadLine<K, NB>;
+  const uint64_t at = static_cast<uint64_t>(chunk) * L::kKeys;
+  const bool tail = chunk >= n / L::kKeys;  // the column's partial last chunk
+  const uint32_t whole = tail ? 0u : chunk;
+  uint32_t below = 0;
+  bool eq = false;
+  if (n >= static_cast<uint64_t>(L::kKeys)) {  // kernel-uniform: there is a whole chunk to read
+    L ln[kQuad];
+    const K* lane_base = col + ql * L::kLaneKeys;
+    quad_rounds([&](auto r) { ln[r].load(lane_base, quad_bcast<r>(whole)); });
+    below = quad_below(ln, q, ql);
+    eq = quad_holds(ln, q, ql);
   }
-  // as in group_count_less, each round's probe is fetched again when compared; the owning
-  // lane forms the match position from its own chunk.  Slots past the column's end hold the
-  // key_max fill: the lowest matching slot is taken (the column's keys are unique, so a
-  // real match precedes any fill) and a position past the end reads as not found.
-  uint64_t pos = ~0ull;
-#pragma unroll
-  for (int r = 0; r < G; ++r) {
-    const K xr = shfl(my_x, gbase + r);
-    int best = NK;
-#pragma unroll
-    for (int j = 0; j < KPL; ++j) {
-      const int f = group_ffs<G>(ballot(pc[r].k[j] == xr), gbase);
-      if (f >= 0 && f * KPL + j < best) best = f * KPL + j;
-    }
-    if (gl == r && best < NK) pos = my_chunk * NK + static_cast<uint64_t>(best);
-  }
-  return (my_live && pos < n) ? static_cast<uint32_t>(pos) : kNotFound;
+  if (tail && live) below = tail_below(col, n, at, x, eq);
+  return (live && eq) ? static_cast<uint32_t>(at + below) : kNotFound;
 }
 
 // ---------------------------------------------------------------------------
@@ -146,7 +198,6 @@ template <class K, int NB = 128>
 struct BTreeDev {
   static_assert(NB == 64 || NB == 128 || NB == 256, "B-tree nodes of 64, 128 or 256 bytes");
   static constexpr int NK = NB / static_cast<int>(sizeof(K));
-  static constexpr int G = NB / 16;  // lanes per node search, 16 bytes each
   const K* col;
   uint64_t n;
   const K* nodes;  // all inner levels, top level first, NK keys per node
@@ -159,35 +210,24 @@ struct BTreeDev {
   __host__ __device__ size_t lds_bytes() const { return lds_nodes * NB; }
   __device__ void stage(uint8_t* lds) const { stage_to_lds(lds, nodes, lds_nodes * NB); }
 
-  __device__ __forceinline__ void descend(uint64_t& node, bool& live, uint32_t c, uint32_t lvl) const {
-    const uint64_t child = node * NK + c;
+  __device__ __forceinline__ void descend(uint32_t& node, bool& live, uint32_t c, uint32_t lvl) const {
+    const uint64_t child = static_cast<uint64_t>(node) * NK + c;
     live = live && (c < static_cast<uint32_t>(NK)) && (child < level_cnt[lvl + 1]);
-    node = live ? child : 0;
-  }
-
-  // Walks the inner levels; returns the column chunk of the probe (or live = false).
-  __device__ __forceinline__ uint64_t find_chunk(K x, bool& live, const uint8_t* lds, int gbase, int gl) const {
-    uint64_t node = 0;
-    uint32_t lvl = 0;
-    const K* lds_nodes_p = reinterpret_cast<const K*>(lds);
-    for (; lvl < lds_levels; ++lvl) {
-      const uint32_t c = group_count_less<K, G, NB>(lds_nodes_p + level_off[lvl] * NK, node, x, gbase, gl);
-      descend(node, live, c, lvl);
-    }
-    for (; lvl < levels; ++lvl) {
-      const uint32_t c = group_count_less<K, G, NB>(nodes + level_off[lvl] * NK, node, x, gbase, gl);
-      descend(node, live, c, lvl);
-    }
-    return node;
+    node = live ? static_cast<uint32_t>(child) : 0u;
   }
 
   __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
-    const int ln = lane();
-    const int gbase = ln & ~(G - 1);
-    const int gl = ln & (G - 1);
+    const int ql = lane() & (kQuad - 1);
+    const QuadProbes<K> q(x);
     bool live = active;
-    const uint64_t chunk = find_chunk(x, live, lds, gbase, gl);
-    return group_find_equal<K, G, NB>(col, n, chunk, x, live, gbase, gl);
+    uint32_t node = 0;  // fewer than 2^32 / NK chunks, hence nodes of any level
+    uint32_t lvl = 0;
+    const K* lds_nodes_p = reinterpret_cast<const K*>(lds);
+    for (; lvl < lds_levels; ++lvl)
+      descend(node, live, quad_count_less<K, NB>(lds_nodes_p + level_off[lvl] * NK, node, q, ql), lvl);
+    for (; lvl < levels; ++lvl)
+      descend(node, live, quad_count_less<K, NB>(nodes + level_off[lvl] * NK, node, q, ql), lvl);
+    return quad_find_equal<K, NB>(col, n, node, live, x, q, ql);
   }
 };
 

@@ -164,74 +164,29 @@ struct HarmoniaDev {
 // ---------------------------------------------------------------------------
 // Last-mile window search shared by RadixSpline and the learned models.
 // Each lane's probe has a predicted position `pred` and a window [lo, hi) of
-// the column that holds the key if it is present.  Groups of kWinG = 4 lanes
-// read whole 128-byte lines (32 B per lane); a group serves its 4 probes in 4
-// rounds.  A round starts at the line holding pred and walks one line left or
-// right until the line brackets the probe or leaves the window.  The search
-// runs in phases: in each phase every unresolved round of every group requests
-// its next line before any line is examined, so a wave pays one memory latency
-// per phase (one, occasionally two or three) rather than one per walking round.
+// the column that holds the key if it is present.  Quads read whole 128-byte
+// lines (QuadLine); a quad serves its 4 probes in 4 rounds.  A round starts at
+// the line holding pred and walks one line left or right until the line brackets
+// the probe or leaves the window.  The search runs in phases: in each phase every
+// unresolved round of every quad requests its next line before any line is
+// examined, so a wave pays one memory latency per phase (one, occasionally two or
+// three) rather than one per walking round.
 //
-// A round's line is sorted, so the group only needs two facts about it for the
-// owning lane: how many of its keys are below the probe (`below`, which is the
-// in-line offset of the probe's lower bound) and whether the key at that offset
-// equals the probe.  The owning lane alone holds its probe's state (line,
-// window, direction), which keeps the registers per lane, and hence the waves
-// per SIMD, where a latency-bound search needs them.  Positions are 32-bit
-// (n < 2^32); keys at or past n read as the all-ones fill, which sorts last.
+// A round's line is sorted, so the owning lane only needs how many of its keys are
+// below the probe (the in-line offset of the probe's lower bound) and whether the
+// line holds it.  The owning lane alone holds its probe's state (line, window,
+// direction), which keeps the registers per lane, and hence the waves per SIMD,
+// where a latency-bound search needs them.  Positions are 32-bit (n < 2^32).
 // ---------------------------------------------------------------------------
-constexpr int kWinG = 4;
-
-template <class K>
-struct LineProbe {
-  static constexpr int LK = 128 / static_cast<int>(sizeof(K));  // keys per line
-  static constexpr int KPL = LK / kWinG;                         // keys per lane (32 bytes)
-  K k[KPL];
-  __device__ __forceinline__ void load(const K* col, uint64_t n, uint32_t line, int gl) {
-    load(col, n, 0u, gl, static_cast<uint64_t>(line));
-  }
-  // line given as 64 bits (the line copies of the lines layout can exceed 2^32 slots)
-  __device__ __forceinline__ void load(const K* col, uint64_t n, uint32_t, int gl, uint64_t line) {
-    const uint64_t start = line * LK + static_cast<uint64_t>(gl * KPL);
-    if (start + KPL <= n) {
-      const u32x4 a = *reinterpret_cast<const u32x4*>(col + start);
-      const u32x4 b = *reinterpret_cast<const u32x4*>(col + start + KPL / 2);
-      if constexpr (sizeof(K) == 8) {
-        k[0] = (static_cast<uint64_t>(a.y) << 32) | a.x;
-        k[1] = (static_cast<uint64_t>(a.w) << 32) | a.z;
-        k[2] = (static_cast<uint64_t>(b.y) << 32) | b.x;
-        k[3] = (static_cast<uint64_t>(b.w) << 32) | b.z;
-      } else {
-        k[0] = a.x; k[1] = a.y; k[2] = a.z; k[3] = a.w;
-        k[4] = b.x; k[5] = b.y; k[6] = b.z; k[7] = b.w;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < KPL; ++j) k[j] = (start + j < n) ? col[start + j] : key_max<K>();
-    }
-  }
-  // keys of the group's line below x, and whether the line holds x
-  __device__ __forceinline__ void eval(K x, int gbase, uint32_t& below, bool& eq) const {
-    below = 0;
-    bool e = false;
-#pragma unroll
-    for (int j = 0; j < KPL; ++j) {
-      below += static_cast<uint32_t>(group_popc<kWinG>(ballot(k[j] < x), gbase));
-      e |= group_bits<kWinG>(ballot(k[j] == x), gbase) != 0;
-    }
-    eq = e;
-  }
-};
-
 template <class K>
 __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n, uint32_t my_pred, uint32_t my_lo,
                                                         uint32_t my_hi, K my_x, bool my_live) {
-  using LP = LineProbe<K>;
-  constexpr int G = kWinG;
-  constexpr uint32_t LK = LP::LK;
-  const int ln = lane();
-  const int gbase = ln & ~(G - 1);
-  const int gl = ln & (G - 1);
+  using L = QuadLine<K, 128>;
+  constexpr uint32_t LK = L::kKeys;
+  const int ql = lane() & (kQuad - 1);
+  const QuadProbes<K> q(my_x);
+  const K* lane_base = col + ql * L::kLaneKeys;
+  const uint32_t whole = static_cast<uint32_t>(n / LK);  // whole lines of the column
   bool open = my_live && my_lo < my_hi;
   uint32_t line = 0, found = kNotFound;
   if (open) {
@@ -240,33 +195,23 @@ __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n
   }
   const uint32_t first_line = my_lo / LK, last_line = open ? (my_hi - 1) / LK : 0u;
   int dir = 0;  // 0: first line, -1 walking left, +1 walking right
-  for (;;) {
-    const uint64_t open_mask = ballot(open);
-    if (open_mask == 0) break;  // wave-uniform exit
-    LP pc[G];
-#pragma unroll
-    for (int r = 0; r < G; ++r) {
-      const uint32_t l = shfl32(line, gbase + r);
-      if ((open_mask >> (gbase + r)) & 1ull) pc[r].load(col, n, l, gl);
-    }
-    uint32_t below = 0;
-    bool eq = false;
-#pragma unroll
-    for (int r = 0; r < G; ++r) {
-      if (!((open_mask >> (gbase + r)) & 1ull)) continue;
-      uint32_t b;
-      bool e;
-      pc[r].eval(shfl(my_x, gbase + r), gbase, b, e);
-      if (gl == r) {
-        below = b;
-        eq = e;
-      }
-    }
+  while (ballot(open) != 0) {  // wave-uniform exit
+    const bool tail = open && line >= whole;  // the column's partial last line
+    const uint32_t rounds = quad_or(open && !tail ? 1u << ql : 0u);
+    L ln[kQuad];
+    quad_rounds([&](auto r) { ln[r].any(); });
+    quad_rounds([&](auto r) {
+      const uint32_t l = quad_bcast<r>(line);
+      if ((rounds >> r) & 1u) ln[r].load(lane_base, l);
+    });
+    uint32_t below = quad_below(ln, q, ql);
+    bool eq = quad_holds(ln, q, ql);
+    if (tail) below = tail_below(col, n, static_cast<uint64_t>(line) * LK, my_x, eq);
     if (open) {
       const uint32_t base = line * LK;
       const uint32_t a = my_lo > base ? my_lo - base : 0u;               // window slots of this line: [a, c)
       const uint32_t c = my_hi - base < LK ? my_hi - base : LK;
-      if (eq && static_cast<uint64_t>(base) + below < n) {
+      if (eq) {
         found = base + below;  // the line holds x at its lower-bound offset
         open = false;
       } else if (below >= c && dir >= 0 && line < last_line) {
@@ -281,35 +226,6 @@ __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n
     }
   }
   return found;
-}
-
-// Number of the 16 u64 keys of line `my_line` (of `lines`) that are below each
-// lane's probe, for the lanes with my_live; whole-wave call (4-lane groups, one
-// 128-byte line per round, all rounds' lines requested before any is examined).
-template <class K>
-__device__ __forceinline__ uint32_t group_line_count(const uint64_t* lines, uint32_t my_line, K my_x, bool my_live) {
-  using LP = LineProbe<uint64_t>;
-  constexpr int G = kWinG;
-  const int ln = lane();
-  const int gbase = ln & ~(G - 1);
-  const int gl = ln & (G - 1);
-  const uint64_t live_mask = ballot(my_live);
-  LP pc[G];
-#pragma unroll
-  for (int r = 0; r < G; ++r) {
-    const uint32_t l = shfl32(my_line, gbase + r);
-    if ((live_mask >> (gbase + r)) & 1ull) pc[r].load(lines, ~0ull, l, gl);
-  }
-  uint32_t below = 0;
-#pragma unroll
-  for (int r = 0; r < G; ++r) {
-    if (!((live_mask >> (gbase + r)) & 1ull)) continue;
-    uint32_t b;
-    bool e;
-    pc[r].eval(shfl64(static_cast<uint64_t>(my_x), gbase + r), gbase, b, e);
-    if (gl == r) below = b;
-  }
-  return below;
 }
 
 // ---------------------------------------------------------------------------
@@ -589,7 +505,10 @@ struct LearnedDev {
       }
     }
     if (num_splits && ballot(split) != 0) {  // wave-uniform
-      const uint32_t t = group_line_count<K>(seps, split ? m.start : 0u, x, split);
+      // separators below the probe in its leaf's line (the lanes without a split read line 0)
+      const uint32_t t = quad_count_less<uint64_t, 128>(seps, split ? m.start : 0u,
+                                                        QuadProbes<uint64_t>(static_cast<uint64_t>(x)),
+                                                        lane() & (kQuad - 1));
       if (split) {
         m = subs[static_cast<uint64_t>(m.start) * kSplitWays + (t < kSplitWays ? t : kSplitWays - 1)];
         use_tree = __builtin_isnan(m.slope);
@@ -735,67 +654,47 @@ struct LinesDev {
     return group_line_walk(t, x, live);
   }
 
-  // Groups of kWinG lanes read whole lines (32 bytes per lane, lane 0 holding the
-  // header) and serve their probes in kWinG rounds; every open round requests its
-  // line before any line is examined, so a wave pays one memory latency per step.
+  // Quads read whole lines (QuadLine; lane 0's first piece starts with the header) and
+  // serve their probes in four rounds; every open round requests its line before any line
+  // is examined, so a wave pays one memory latency per step.  Slots past a line's count
+  // hold key_max, which no probe exceeds, so `below` needs no count, and a line's keys are
+  // all below the probe and the line is full exactly when below = CAP.
   __device__ __forceinline__ uint32_t group_line_walk(uint64_t my_line, K my_x, bool my_live) const {
-    using LP = LineProbe<K>;
-    constexpr int G = kWinG;
-    constexpr uint32_t KPL = LP::KPL;
-    static_assert(LP::LK == SLOTS, "a line probe covers one line");
-    const int ln = lane();
-    const int gbase = ln & ~(G - 1);
-    const int gl = ln & (G - 1);
-    const uint64_t all = num_lines * SLOTS;
+    using L = QuadLine<K, 128>;
+    static_assert(L::kKeys == SLOTS, "a quad line covers one line");
+    const int ql = lane() & (kQuad - 1);
+    const QuadProbes<K> q(my_x);
+    const K* lane_base = lines + ql * L::kLaneKeys;
     bool open = my_live;
-    uint64_t line = my_line < num_lines ? my_line : num_lines - 1;
+    // fewer than 2^32 lines (targets and line bases are 32-bit at build)
+    uint32_t line = static_cast<uint32_t>(my_line < num_lines ? my_line : num_lines - 1);
+    const uint32_t last = static_cast<uint32_t>(num_lines - 1);
     uint32_t found = kNotFound;
-    for (;;) {
-      const uint64_t open_mask = ballot(open);
-      if (open_mask == 0) break;  // wave-uniform exit
-      LP pc[G];
+    while (ballot(open) != 0) {  // wave-uniform exit
+      const uint32_t rounds = quad_or(open ? 1u << ql : 0u);
+      L ln[kQuad];
+      quad_rounds([&](auto r) { ln[r].any(); });
+      quad_rounds([&](auto r) {
+        const uint32_t l = quad_bcast<r>(line);
+        if ((rounds >> r) & 1u) ln[r].load(lane_base, l);
+      });
+      uint32_t base = 0;
+      quad_rounds([&](auto r) {
+        const uint32_t b = quad_bcast<0>(static_cast<uint32_t>(ln[r].pc[0].k[0]));  // the header's first row id
+        base = ql == r ? b : base;
 #pragma unroll
-      for (int r = 0; r < G; ++r) {
-        const uint64_t l = shfl64(line, gbase + r);
-        if ((open_mask >> (gbase + r)) & 1ull) pc[r].load(lines, all, static_cast<uint32_t>(0), gl, l);
-      }
-      uint32_t below = 0, count = 0, base = 0;
-      bool eq = false;
-#pragma unroll
-      for (int r = 0; r < G; ++r) {
-        if (!((open_mask >> (gbase + r)) & 1ull)) continue;
-        uint64_t w0;
-        if constexpr (sizeof(K) == 8) {
-          w0 = static_cast<uint64_t>(pc[r].k[0]);
-        } else {
-          w0 = (static_cast<uint64_t>(pc[r].k[1]) << 32) | static_cast<uint64_t>(pc[r].k[0]);
-        }
-        const uint64_t hdr = shfl64(w0, gbase);  // group lane 0 holds the header
-        const uint32_t c = static_cast<uint32_t>(hdr >> 32);
-        const K xr = shfl(my_x, gbase + r);
-        uint32_t b = 0;
-        bool e = false;
-#pragma unroll
-        for (uint32_t j = 0; j < KPL; ++j) {
-          const uint32_t slot = static_cast<uint32_t>(gl) * KPL + j;
-          const bool valid = slot >= HDR && slot < HDR + c;
-          b += static_cast<uint32_t>(group_popc<G>(ballot(valid && pc[r].k[j] < xr), gbase));
-          e |= group_bits<G>(ballot(valid && pc[r].k[j] == xr), gbase) != 0;
-        }
-        if (gl == r) {
-          below = b;
-          eq = e;
-          count = c;
-          base = static_cast<uint32_t>(hdr);
-        }
-      }
+        for (uint32_t h = 0; h < HDR; ++h)
+          ln[r].pc[0].k[h] = ql == 0 ? key_max<K>() : ln[r].pc[0].k[h];  // the header is no key
+      });
+      const uint32_t below = quad_below(ln, q, ql);
+      const bool eq = quad_holds(ln, q, ql);
       if (open) {
-        if (eq) {
-          found = base + below;
-          open = false;
-        } else if (below == count && count == CAP && line + 1 < num_lines) {
+        if (below == CAP && line < last) {
           ++line;  // a full line below the probe: keys pushed on from it sit in the next line
         } else {
+          // a live probe equal to the key_max fill is the column's last key, and is met in
+          // its own line (behind full lines only), where the rank is its slot
+          if (eq && below < CAP) found = base + below;
           open = false;
         }
       }
@@ -811,8 +710,8 @@ struct LinesDev {
 // empty = all-ones key.
 // An entry is 16 bytes {u64 key, u32 row id, pad}.  The reference reads one entry per
 // 16-byte load and steps on (ld.global.cs of a longlong2, :62), so a wave waits for its
-// longest probe run, one dependent load per slot.  Here groups of kWinG lanes read whole
-// 128-byte lines of 8 entries (32 bytes per lane) and serve their probes in kWinG
+// longest probe run, one dependent load per slot.  Here quads read whole
+// 128-byte lines of 8 entries (32 bytes per lane) and serve their probes in four
 // rounds, every open round requesting its line before any line is examined: a probe
 // resolves within the line of its home slot unless its run passes the line's end.
 // Tables below 8 slots take the entry-by-entry walk.
@@ -827,7 +726,7 @@ static_assert(sizeof(HashEntry) == 16, "16-byte entry");
 template <class K>
 struct HashDev {
   static constexpr uint32_t kLineEntries = 8;
-  static constexpr uint32_t kEntriesPerLane = kLineEntries / kWinG;  // 2
+  static constexpr uint32_t kEntriesPerLane = kLineEntries / kQuad;  // 2
   const HashEntry* table;
   uint64_t mask;  // capacity - 1
 
@@ -851,63 +750,55 @@ struct HashDev {
     const uint64_t k = static_cast<uint64_t>(x);
     const bool live = active && k != ~0ull;  // all-ones is the empty marker, never a stored key
     if (mask < kLineEntries - 1) return lookup_entries(k, live);  // wave-uniform
-    constexpr int G = kWinG;
-    const int ln = lane();
-    const int gbase = ln & ~(G - 1);
-    const int gl = ln & (G - 1);
+    const int ql = lane() & (kQuad - 1);
     uint64_t slot = live ? key_hash<K>(k) & mask : 0;
     uint64_t lines_left = (mask + 1) / kLineEntries;  // a table without an empty slot ends the walk
+    const QuadProbes<uint64_t> q(k);
+    const u32x4* lane_base = reinterpret_cast<const u32x4*>(table) + ql * kEntriesPerLane;
     bool open = live;
     uint32_t found = kNotFound;
-    for (;;) {
-      const uint64_t open_mask = ballot(open);
-      if (open_mask == 0) break;  // wave-uniform exit
-      u32x4 e[G][kEntriesPerLane];
+    while (ballot(open) != 0) {  // wave-uniform exit
+      const uint32_t rounds = quad_or(open ? 1u << ql : 0u);
+      const uint32_t line = static_cast<uint32_t>(slot / kLineEntries);  // at most 2^33 slots
+      const uint32_t off = static_cast<uint32_t>(slot) & (kLineEntries - 1);
+      u32x4 e[kQuad][kEntriesPerLane];
 #pragma unroll
-      for (int r = 0; r < G; ++r) {
-        const uint64_t sr = shfl64(slot, gbase + r);
-        if ((open_mask >> (gbase + r)) & 1ull) {
-          const u32x4* p = reinterpret_cast<const u32x4*>(table + (sr & ~static_cast<uint64_t>(kLineEntries - 1)) +
-                                                          static_cast<uint64_t>(gl) * kEntriesPerLane);
+      for (int r = 0; r < kQuad; ++r)
 #pragma unroll
-          for (uint32_t t = 0; t < kEntriesPerLane; ++t) e[r][t] = p[t];
+        for (uint32_t t = 0; t < kEntriesPerLane; ++t) e[r][t] = any_u32x4();
+      quad_rounds([&](auto r) {
+        const uint64_t l = quad_bcast<r>(line);
+        if ((rounds >> r) & 1u) {
+#pragma unroll
+          for (uint32_t t = 0; t < kEntriesPerLane; ++t) e[r][t] = lane_base[l * kLineEntries + t];
         }
-      }
-      bool hit = false, stop = false;
-      uint32_t value = 0;
-#pragma unroll
-      for (int r = 0; r < G; ++r) {
-        if (!((open_mask >> (gbase + r)) & 1ull)) continue;
-        const uint64_t kr = shfl64(k, gbase + r);
-        const uint32_t off = static_cast<uint32_t>(shfl64(slot, gbase + r)) & (kLineEntries - 1);
-        uint32_t v = 0;
-        bool m = false, em = false;
+      });
+      uint32_t flags = 0;     // bit r: round r's key is here; bit 4 + r: an empty slot from its home on
+      uint32_t v[kQuad];
+      quad_rounds([&](auto r) {
+        const uint32_t o = quad_bcast<r>(off);
+        v[r] = 0;
 #pragma unroll
         for (uint32_t t = 0; t < kEntriesPerLane; ++t) {
-          const uint32_t j = static_cast<uint32_t>(gl) * kEntriesPerLane + t;  // entry in the line
           const uint64_t ek = (static_cast<uint64_t>(e[r][t].y) << 32) | e[r][t].x;
-          const bool at = j >= off;
-          if (at && ek == kr) {
-            m = true;
-            v = e[r][t].z;
-          }
-          em |= at && ek == ~0ull;
+          // a key sits in one slot only, so a match needs no look at the home slot
+          const bool m = ek == q.x[r];
+          v[r] = m ? e[r][t].z : v[r];
+          flags |= m ? 1u << r : 0u;
+          flags |= (ek == ~0ull && static_cast<uint32_t>(ql) * kEntriesPerLane + t >= o) ? 16u << r : 0u;
         }
-        // a present key comes before every empty slot of its run, so a match decides
-        const uint32_t mb = group_bits<G>(ballot(m), gbase);
-        const uint32_t eb = group_bits<G>(ballot(em), gbase);
-        const uint32_t vr = shfl32(v, gbase + (mb ? __ffs(mb) - 1 : 0));
-        if (gl == r) {
-          hit = mb != 0;
-          stop = hit || eb != 0;
-          value = vr;
-        }
-      }
+      });
+      flags = quad_or(flags) >> ql;
+      // lane r takes round r's value: one lane of the quad holds it, the others zero
+      const uint32_t a = ((ql & 1) ? v[1] : v[0]) | quad_perm32<0xB1>((ql & 1) ? v[0] : v[1]);
+      const uint32_t b = ((ql & 1) ? v[3] : v[2]) | quad_perm32<0xB1>((ql & 1) ? v[2] : v[3]);
+      const uint32_t value = ((ql & 2) ? b : a) | quad_perm32<0x4E>((ql & 2) ? a : b);
       if (open) {
-        if (hit) {
+        // a present key comes before every empty slot of its run, so a match decides
+        if (flags & 1u) {
           found = value;
           open = false;
-        } else if (stop || --lines_left == 0) {
+        } else if ((flags & 16u) || --lines_left == 0) {
           open = false;
         } else {
           slot = ((slot | (kLineEntries - 1)) + 1) & mask;  // the next line's first entry
