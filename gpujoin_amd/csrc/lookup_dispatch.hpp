@@ -20,6 +20,23 @@ inline unsigned lookup_block(const gj_lookup_params& p) {
   return b;
 }
 
+// Blocks of a driver whose waves take steps of `per_block` items per workgroup, without a
+// caller's grid_blocks: one step per wave.  The hardware then hands a workgroup's place to
+// the next one as soon as it is free, where a grid of resident workgroups that each stride
+// over the input ends with the slowest one and runs its waves in lockstep: 2^24 probes of
+// 2^20 u32 keys (learned, column layout) 260 -> 218 us, 2^28 of 2^26 u64 keys (lines)
+// 5.49 -> 5.29 ms.  Every workgroup stages the descriptor's LDS image, though, so above
+// kStageStep bytes of it a wave takes one more step for each (Harmonia's 15.9 KB at 2^20
+// u64 keys: 575 us with one step, 529 with four, 570 strided).  Never fewer workgroups
+// than fit on the chip at once, if there is a step for each.
+constexpr uint64_t kStageStep = 8192;
+inline uint64_t cover_blocks(uint64_t items, uint64_t per_block, size_t stage_bytes, uint64_t resident) {
+  const uint64_t cover = ceil_div(items, per_block);
+  const uint64_t steps = 1 + stage_bytes / kStageStep;
+  const uint64_t blocks = std::max<uint64_t>(ceil_div(cover, steps), std::min<uint64_t>(cover, resident));
+  return std::min<uint64_t>(std::max<uint64_t>(blocks, 1), 0x7FFFFFFFull);
+}
+
 template <class Dev, class K>
 void launch_plain(const Dev& d, const K* probes, uint64_t m, uint32_t* out, const gj_lookup_params& p, hipStream_t s,
                   int cu) {
@@ -27,9 +44,9 @@ void launch_plain(const Dev& d, const K* probes, uint64_t m, uint32_t* out, cons
   const unsigned block = lookup_block(p);
   const size_t lds = d.lds_bytes();
   const void* fn = reinterpret_cast<const void*>(&lookup_plain_kernel<Dev, K>);
-  uint64_t blocks = p.grid_blocks ? p.grid_blocks : static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu;
-  blocks = std::min<uint64_t>(blocks, ceil_div(m, block));
-  blocks = std::max<uint64_t>(blocks, 1);
+  const uint64_t blocks = p.grid_blocks
+                              ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(m, block)))
+                              : cover_blocks(m, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
   hipLaunchKernelGGL((lookup_plain_kernel<Dev, K>), dim3(static_cast<unsigned>(blocks)), dim3(block), lds, s, d,
                      probes, m, out);
   GJ_HIP_CHECK(hipGetLastError());
@@ -60,10 +77,10 @@ void launch_tuples(const Dev& d, const K* keys, const uint64_t* d_total, uint64_
   const unsigned block = lookup_block(p);
   const size_t lds = d.lds_bytes();
   const void* fn = reinterpret_cast<const void*>(&lookup_tuples_kernel<Dev, K>);
-  uint64_t blocks = p.grid_blocks ? p.grid_blocks : static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu;
-  blocks = std::min<uint64_t>(blocks, ceil_div(total_max, block));
+  uint64_t blocks = p.grid_blocks
+                        ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(total_max, block)))
+                        : cover_blocks(total_max, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
   if (blocks >= 8) blocks = blocks / 8 * 8;  // whole XCD rounds for the XCD-major chunk map
-  blocks = std::max<uint64_t>(blocks, 1);
   hipLaunchKernelGGL((lookup_tuples_kernel<Dev, K>), dim3(static_cast<unsigned>(blocks)), dim3(block), lds, s, d,
                      keys, d_total, total_max, res);
   GJ_HIP_CHECK(hipGetLastError());
@@ -78,9 +95,9 @@ void launch_bws(const Dev& d, const K* probes, uint64_t m, uint32_t* out, const 
   const unsigned block = lookup_block(p);
   const size_t lds = (d.lds_bytes() + 15) / 16 * 16 + kBwsTile * (sizeof(K) + sizeof(uint32_t));
   const void* fn = reinterpret_cast<const void*>(&lookup_bws_kernel<Dev, K, kBwsTile>);
-  uint64_t blocks = p.grid_blocks ? p.grid_blocks : static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu;
-  blocks = std::min<uint64_t>(blocks, ceil_div(m, kBwsTile));
-  blocks = std::max<uint64_t>(blocks, 1);
+  const uint64_t blocks =
+      p.grid_blocks ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(m, kBwsTile)))
+                    : cover_blocks(m, kBwsTile, 0, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
   hipLaunchKernelGGL((lookup_bws_kernel<Dev, K, kBwsTile>), dim3(static_cast<unsigned>(blocks)), dim3(block), lds, s,
                      d, probes, m, out);
   GJ_HIP_CHECK(hipGetLastError());
