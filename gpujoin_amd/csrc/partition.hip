@@ -13,15 +13,11 @@
 //
 // Kernels (no cooperative launch, no device-wide barrier):
 //   hist     one block per contiguous chunk, LDS histogram of 2^radix_bits u32 bins
-//   colscan  one wave per partition: column prefix over the blocks and the partition total
-//   starts   one block: aligned exclusive prefix over partitions -> partition starts
-//   scatter  one block per chunk (the same chunks as hist), three variants:
-//            write-combining (LDS carry buffers, whole aligned segments; unordered,
-//              or stable where two blocks fit per CU)
-//            register tiles with per-wave cursors (stable; fan-outs the
-//              write-combining buffers do not fit)
-//            one store per item at an LDS-atomic slot (unordered, where the
-//              write-combining buffers do not fit)
+//   colscan  column prefix over the blocks and the partition totals, 64 partitions a block
+//   starts   one block: aligned exclusive prefix over partitions -> partition starts, and
+//            the padding behind every partition
+//   scatter  one block per chunk (the same chunks as hist): tiles sorted by partition in
+//            LDS, stable or in any order, then stored run by run
 #include <algorithm>
 
 #include "common.hpp"
@@ -29,10 +25,7 @@
 
 namespace gj {
 
-constexpr int kPartBlock = 256;
-constexpr int kPartWaves = kPartBlock / kWave;
-constexpr int kPartItems = 16;                        // items per lane per tile
-constexpr int kPartTile = kPartBlock * kPartItems;    // 4096 items
+constexpr int kPartTile = 4096;  // chunks are whole multiples of this many items (histogram rows are sized by it)
 constexpr uint32_t kMaxRadixBits = 16;
 
 __host__ __device__ __forceinline__ uint32_t part_align(int key_bytes) { return 128u / static_cast<uint32_t>(key_bytes); }
@@ -112,36 +105,76 @@ __global__ __launch_bounds__(1024) void part_hist_kernel(const K* __restrict__ k
   for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x) hist[c * fan + p] = h[p];
 }
 
-// hist[b][p] <- sum_{b' < b} hist[b'][p]; count[p] <- total.  One wave per
-// partition scans its column 64 rows at a time (wave prefix sum by shuffles).
-__global__ __launch_bounds__(256) void part_colscan_kernel(uint32_t* __restrict__ hist, uint32_t blocks, uint32_t fan,
-                                                           uint64_t* __restrict__ count) {
-  const uint32_t p = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-  if (p >= fan) return;  // wave-uniform
-  const int ln = lane();
-  uint64_t carry = 0;
-  for (uint32_t b0 = 0; b0 < blocks; b0 += kWave) {
-    const uint32_t b = b0 + static_cast<uint32_t>(ln);
-    const uint32_t v = b < blocks ? hist[static_cast<uint64_t>(b) * fan + p] : 0u;
-    uint32_t x = v;
+// Column scan of one segment's histogram rows [r0, r1): hist[r][p] becomes the sum of the
+// rows before r, count[p] the total.  A workgroup takes 64 partitions and cuts the rows
+// into one span per wave: each lane sums its partition over the wave's span (a row of 64
+// counts is one coalesced 256-byte read, kColIn rows in flight), the spans' sums meet in
+// LDS, and a second walk over the span writes the prefixes.  (One wave per partition
+// reading a row per lane touched 64 lines per load: 14.5 us for 245 rows of 1024
+// partitions, now 5.)
+constexpr int kColIn = 8;
+constexpr uint32_t kColThreads = 1024;
+__device__ __forceinline__ void scan_columns(uint32_t* __restrict__ hist, uint64_t r0, uint64_t r1, uint32_t p0,
+                                             uint32_t fan, uint64_t* __restrict__ count) {
+  constexpr uint32_t kWaves = kColThreads / kWave;
+  __shared__ uint32_t part[kWaves][kWave];
+  const uint32_t w = threadIdx.x / kWave;
+  const uint32_t p = p0 + static_cast<uint32_t>(lane());
+  const uint64_t per = (r1 - r0 + kWaves - 1) / kWaves;
+  const uint64_t a = std::min<uint64_t>(r1, r0 + w * per), b = std::min<uint64_t>(r1, a + per);
+  uint32_t sum = 0;
+  for (uint64_t r = a; r < b; r += kColIn) {
+    uint32_t v[kColIn];
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const uint32_t y = __shfl_up(x, off, kWave);
-      if (ln >= off) x += y;
-    }
-    if (b < blocks) hist[static_cast<uint64_t>(b) * fan + p] = static_cast<uint32_t>(carry) + x - v;
-    carry += __shfl(x, kWave - 1, kWave);
+    for (int u = 0; u < kColIn; ++u) v[u] = (r + u < b && p < fan) ? hist[(r + u) * fan + p] : 0u;
+#pragma unroll
+    for (int u = 0; u < kColIn; ++u) sum += v[u];
   }
-  if (ln == 0) count[p] = carry;
+  part[w][lane()] = sum;
+  __syncthreads();
+  uint32_t run = 0, total = 0;
+#pragma unroll
+  for (uint32_t v = 0; v < kWaves; ++v) {
+    const uint32_t x = part[v][lane()];
+    run += v < w ? x : 0u;
+    total += x;
+  }
+  if (w == 0 && p < fan) count[p] = total;
+  for (uint64_t r = a; r < b; r += kColIn) {
+    uint32_t v[kColIn];
+#pragma unroll
+    for (int u = 0; u < kColIn; ++u) v[u] = (r + u < b && p < fan) ? hist[(r + u) * fan + p] : 0u;
+#pragma unroll
+    for (int u = 0; u < kColIn; ++u) {
+      if (r + u < b && p < fan) hist[(r + u) * fan + p] = run;
+      run += v[u];
+    }
+  }
+}
+
+__global__ __launch_bounds__(kColThreads) void part_colscan_kernel(uint32_t* __restrict__ hist, uint32_t blocks,
+                                                                   uint32_t fan, uint64_t* __restrict__ count) {
+  scan_columns(hist, 0, blocks, blockIdx.x * kWave, fan, count);
+}
+
+// The same per segment of the segmented pass (grid: segments x ceil(fan / 64)).
+__global__ __launch_bounds__(kColThreads) void seg_colscan_wide_kernel(uint32_t* __restrict__ hist,
+                                                                       const uint64_t* __restrict__ chunk0,
+                                                                       uint32_t fan, uint64_t* __restrict__ count) {
+  const uint32_t per = (fan + kWave - 1) / kWave;
+  const uint32_t h = blockIdx.x / per;
+  scan_columns(hist, chunk0[h], chunk0[h + 1], (blockIdx.x % per) * kWave, fan, count + static_cast<uint64_t>(h) * fan);
 }
 
 // start[p] = align_up(start[p-1] + count[p-1], align); one block of 1024 threads.
 // Each thread owns `per` consecutive partitions and reads their counts kScanBatch at a
 // time, loads first (a thread's loads do not depend on one another, so a batch is in
 // flight together: at fan-out 2^16, 64 counts per thread, one at a time took 115 µs).
+// start2 (optional): a second copy of start[0 .. fan).
 constexpr uint32_t kScanBatch = 8;
 __global__ __launch_bounds__(1024) void part_scan_starts_kernel(const uint64_t* __restrict__ count, uint32_t fan,
-                                                                uint32_t align, uint64_t* __restrict__ start) {
+                                                                uint32_t align, uint64_t* __restrict__ start,
+                                                                uint64_t* __restrict__ start2) {
   __shared__ uint64_t s[1024];
   const uint32_t per = (fan + blockDim.x - 1) / blockDim.x;
   const uint32_t p0 = threadIdx.x * per;
@@ -175,7 +208,10 @@ __global__ __launch_bounds__(1024) void part_scan_starts_kernel(const uint64_t* 
 #pragma unroll
     for (uint32_t u = 0; u < kScanBatch; ++u) {
       const uint32_t p = p0 + q + u;
-      if (q + u < per && p < fan) start[p] = run;
+      if (q + u < per && p < fan) {
+        start[p] = run;
+        if (start2) start2[p] = run;
+      }
       run += (c[u] + align - 1) / align * align;
     }
   }
@@ -267,13 +303,13 @@ __global__ __launch_bounds__(kScanThreads) void part_span_starts_kernel(const ui
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanThreads - 1) start[fan] = off + s[kScanThreads - 1];
 }
 
-// start[0 .. fan] from count[0 .. fan) (start[fan] = padded total); sums: kScanSumsBytes
-// of scratch, used above kOneBlockScanMax partitions.
-inline void launch_scan_starts(const uint64_t* count, uint64_t fan, uint32_t align, uint64_t* start, uint64_t* sums,
-                               hipStream_t s) {
+// start[0 .. fan] from count[0 .. fan) (start[fan] = padded total), copied to start2 when
+// given; sums: kScanSumsBytes of scratch, used above kOneBlockScanMax partitions.
+inline void launch_scan_starts(const uint64_t* count, uint64_t fan, uint32_t align, uint64_t* start, uint64_t* start2,
+                               uint64_t* sums, hipStream_t s) {
   if (fan <= kOneBlockScanMax) {
     hipLaunchKernelGGL(part_scan_starts_kernel, dim3(1), dim3(1024), 0, s, count, static_cast<uint32_t>(fan), align,
-                       start);
+                       start, start2);
     GJ_HIP_CHECK(hipGetLastError());
     return;
   }
@@ -285,326 +321,136 @@ inline void launch_scan_starts(const uint64_t* count, uint64_t fan, uint32_t ali
   hipLaunchKernelGGL(part_span_starts_kernel, dim3(static_cast<unsigned>(spans)), dim3(kScanThreads), 0, s, count,
                      static_cast<uint32_t>(fan), align, sums, start);
   GJ_HIP_CHECK(hipGetLastError());
+  if (start2) GJ_HIP_CHECK(hipMemcpyAsync(start2, start, fan * 8, hipMemcpyDeviceToDevice, s));
 }
 
 // Marks the padding slots after every partition (fewer than `align` each) with payload
-// 0xFFFFFFFF and key_max; one thread per partition, grid stride (a batch of windows has
-// up to 2^18 partitions).
+// 0xFFFFFFFF and key_max: the blocks of the grid share the partitions, one slot per thread.
 template <class K>
-__global__ void part_pad_kernel(const uint64_t* __restrict__ start, const uint64_t* __restrict__ count, uint32_t fan,
-                                uint32_t align, K* __restrict__ keys, uint32_t* __restrict__ payload) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t p = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; p < fan; p += stride) {
-    const uint64_t end = start[p] + count[p];
-    const uint64_t stop = start[p] + (count[p] + align - 1) / align * align;
-    for (uint64_t i = end; i < stop; ++i) {
-      keys[i] = key_max<K>();
-      if (payload) payload[i] = 0xFFFFFFFFu;
+__device__ __forceinline__ void pad_partitions(const uint64_t* __restrict__ start, const uint64_t* __restrict__ count,
+                                               uint32_t fan, uint32_t align, K* __restrict__ keys,
+                                               uint32_t* __restrict__ payload) {
+  const uint32_t mine = (fan + gridDim.x - 1) / gridDim.x;  // partitions per block
+  for (uint32_t t = threadIdx.x; t < mine * align; t += blockDim.x) {
+    const uint32_t p = blockIdx.x + (t / align) * gridDim.x;
+    if (p >= fan) continue;
+    const uint64_t n = count[p], at = n + t % align;
+    if (at < (n + align - 1) / align * align) {
+      keys[start[p] + at] = key_max<K>();
+      if (payload) payload[start[p] + at] = 0xFFFFFFFFu;
     }
   }
 }
 
-inline unsigned pad_grid(uint64_t fan) { return static_cast<unsigned>(std::max<uint64_t>(1, ceil_div(fan, 256))); }
+// Scatter.  in_payload == nullptr: payload = payload_base + input position.  A block walks
+// its chunk in tiles of B x I items.  Per tile:
+//   rank    Stable: each wave ranks its items among the equal digits of the wave (ballots
+//           give the lanes with the same digit, a 16-bit row of counts per wave carries
+//           the running rank from one 64-item slice to the next); otherwise an LDS atomic
+//           add per item ranks it among the tile's equal digits in any order
+//   scan    per partition: the waves' counts become exclusive prefixes, a block scan gives
+//           the partition's offset in the tile, and the block's cursor moves on
+//   place   keys and payloads into the tile buffer, in partition order
+//   store   the tile buffer in order: neighbouring lanes store to neighbouring slots of
+//           the same partition's run
+// inv (optional): where every item went, in input order.
+//
+// What bounds it: HBM streaming (a key read, a key and a payload written) and, at large
+// fan-outs, the short runs (B I / 2^bits items per partition and tile) in which the
+// output is written; the next tile's items load while this one is placed and stored.  A
+// scatter straight from registers (one store per lane to a random partition) and one that
+// kept an open 128-byte segment per partition in LDS ran before: 10^7 u64 keys at fan-out
+// 2^10, stable, 300 us a launch; this one XX.
+__host__ __device__ constexpr size_t tile_lds_bytes(uint32_t fan, int key_bytes, bool payload, bool stable, int block,
+                                                    int items) {
+  const size_t tile = static_cast<size_t>(block) * items;
+  return tile * key_bytes + (payload ? tile * 4 : 0)                            // tile keys, payloads
+         + static_cast<size_t>(fan) * 8                                         // base, cur
+         + static_cast<size_t>(fan) * (stable ? 2 * (block / kWave) + 2 : 4);   // rows and offsets, or counts
+}
 
-// Stable scatter.  in_payload == nullptr: payload = payload_base + input position.
-// A block walks its chunk in tiles of kPartTile items held in registers (wave w
-// owns items [w * 1024, (w + 1) * 1024) of the tile, lane-minor).  Per tile:
-//   count   each wave counts its items per partition (LDS atomic adds into the
-//           wave's row)
-//   cursor  per partition: wave cursors = block cursor + counts of earlier waves
-//   scatter each wave writes its items at its cursors (rank among equal digits
-//           from ballots) and advances them; no ordering between waves is needed
-// so a tile costs two block barriers, and the output order is the input order
-// inside every partition.
-template <class K>
-__global__ __launch_bounds__(kPartBlock) void part_scatter_kernel(
+template <class K, bool Stable, bool InPayload, int B, int I>
+__global__ __launch_bounds__(B, 4) void part_scatter_kernel(
     const K* __restrict__ keys, const uint32_t* __restrict__ in_payload, uint32_t payload_base, uint64_t m,
     uint64_t chunk, uint32_t shift, uint32_t bits, const uint32_t* __restrict__ block_off,
-    const uint64_t* __restrict__ start, K* __restrict__ out_keys, uint32_t* __restrict__ out_payload,
-    uint32_t* __restrict__ inv, uint64_t cap, unsigned long long* __restrict__ dropped, Seg sg) {
-  extern __shared__ uint32_t sm[];
+    const uint64_t* __restrict__ start, const uint64_t* __restrict__ count, uint32_t align, K* __restrict__ out_keys,
+    uint32_t* __restrict__ out_payload, uint32_t* __restrict__ inv, uint64_t cap,
+    unsigned long long* __restrict__ dropped, Seg sg) {
+  constexpr int T = B * I;
+  constexpr int W = B / kWave;
+  static_assert(T <= 65535, "tile offsets and ranks are 16-bit");
+  constexpr int kRankItems = I / 2;  // slices ranked together (registers)
+  extern __shared__ uint64_t tsm_[];
+  __shared__ uint32_t wsum[W];
   const uint32_t fan = 1u << bits;
-  uint32_t* cnt = sm;                        // [kPartWaves][fan]: counts, then cursors
-  uint32_t* brun = sm + kPartWaves * fan;    // [fan]: block cursor (absolute position)
+  if (align > 1) pad_partitions<K>(start, count, (sg.segs ? sg.segs : 1u) * fan, align, out_keys, out_payload);
+  K* sk = reinterpret_cast<K*>(tsm_);                                // [T] tile keys, partition order
+  uint32_t* sp = reinterpret_cast<uint32_t*>(sk + T);                // [T] tile payloads (with out_payload)
+  uint32_t* base = sp + (out_payload ? T : 0);                       // [fan] output position of tile slot 0
+  uint32_t* cur = base + fan;                                        // [fan] next output position
+  uint32_t* cnt = cur + fan;                                         // [fan] counts, then tile offsets (unordered)
+  uint16_t* rows = reinterpret_cast<uint16_t*>(cur + fan);           // [W][fan] (stable)
+  uint16_t* off = rows + static_cast<size_t>(W) * fan;               // [fan] tile offsets (stable)
   // neighbouring chunks run on one XCD, so the partial lines that neighbouring
   // chunks write into a partition's run meet in the same L2
-  const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block();
-  uint64_t lo, hi, pbase;
-  if (!seg_range(sg, c, chunk, m, fan, lo, hi, pbase)) return;  // block-uniform, before any barrier
-  for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x) {
-    brun[p] = static_cast<uint32_t>(start[pbase + p]) + block_off[c * fan + p];
-#pragma unroll
-    for (int w = 0; w < kPartWaves; ++w) cnt[w * fan + p] = 0;
-  }
-  __syncthreads();
-  const int w = threadIdx.x / kWave;
-  const int ln = lane();
-  const uint64_t lt = (ln == 0) ? 0ull : (~0ull >> (64 - ln));  // lanes below this one
-  uint32_t* mine = cnt + w * fan;
-  for (uint64_t tile = lo; tile < hi; tile += kPartTile) {
-    const uint64_t wbase = tile + static_cast<uint64_t>(w) * (kPartItems * kWave);
-    K k[kPartItems];
-    uint32_t pay[kPartItems];
-#pragma unroll
-    for (int j = 0; j < kPartItems; ++j) {
-      const uint64_t i = wbase + static_cast<uint64_t>(j * kWave + ln);
-      const bool valid = i < hi;
-      k[j] = valid ? load_stream(keys + i) : K(0);
-      pay[j] = valid ? (in_payload ? load_stream(in_payload + i) : payload_base + static_cast<uint32_t>(i)) : 0u;
-    }
-    // lanes of this wave whose item j has the same digit (invalid items match nothing)
-    auto peers_of = [&](int j, uint32_t d) {
-      const uint64_t i = wbase + static_cast<uint64_t>(j * kWave + ln);
-      uint64_t peers = ballot(i < hi);
-      for (uint32_t b = 0; b < bits; ++b) {
-        const uint64_t set = ballot((d >> b) & 1u);
-        peers &= ((d >> b) & 1u) ? set : ~set;
-      }
-      return (i < hi) ? peers : 0ull;
-    };
-    // counts need no ranks: one LDS atomic add per item
-#pragma unroll
-    for (int j = 0; j < kPartItems; ++j) {
-      const uint64_t i = wbase + static_cast<uint64_t>(j * kWave + ln);
-      if (i < hi) atomicAdd(&mine[digit_of(k[j], shift, fan - 1)], 1u);
-    }
-    __syncthreads();
-    // a cursor is written only where the wave has items of the partition: those
-    // entries are the ones the wave zeroes after its scatter, so every entry is a
-    // zero count again when the next tile starts
-    for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x) {
-      uint32_t r = brun[p];
-#pragma unroll
-      for (int v = 0; v < kPartWaves; ++v) {
-        const uint32_t c = cnt[v * fan + p];
-        if (c != 0) cnt[v * fan + p] = r;
-        r += c;
-      }
-      brun[p] = r;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kPartItems; ++j) {
-      const uint32_t d = digit_of(k[j], shift, fan - 1);
-      const uint64_t peers = peers_of(j, d);
-      if (peers) {
-        const uint32_t at = mine[d];  // every lane of the group reads the cursor before the leader moves it
-        const uint32_t pos = at + static_cast<uint32_t>(__popcll(peers & lt));
-        if (pos < cap) {  // always true for a consistent histogram
-          out_keys[pos] = k[j];
-          if (out_payload) out_payload[pos] = pay[j];
-        } else {
-          drop(dropped);
-        }
-        if (inv) inv[wbase + static_cast<uint64_t>(j * kWave + ln)] = pos;
-        if ((peers & lt) == 0) mine[d] = at + static_cast<uint32_t>(__popcll(peers));
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-    // cursors back to zero counts for the next tile (this wave's row only)
-#pragma unroll
-    for (int j = 0; j < kPartItems; ++j) {
-      const uint32_t d = digit_of(k[j], shift, fan - 1);
-      const uint64_t i = wbase + static_cast<uint64_t>(j * kWave + ln);
-      if (i < hi) mine[d] = 0;
-    }
-    __syncthreads();  // the next tile's cursor step reads every wave's row
-  }
-}
-
-// Unordered scatter for callers that carry each tuple's position in its payload
-// (the partitioned lookup driver): an item's slot is an LDS atomic add on the
-// block's cursor of its partition, so a tile needs no counts, ranks or barriers.
-// The block's items of partition p still fill exactly the run the histogram gave
-// the block, [start[p] + block_off[c][p], + hist[c][p]); only their order inside
-// it is arbitrary.
-template <class K>
-__global__ __launch_bounds__(kPartBlock) void part_scatter_any_kernel(
-    const K* __restrict__ keys, const uint32_t* __restrict__ in_payload, uint32_t payload_base, uint64_t m,
-    uint64_t chunk, uint32_t shift, uint32_t bits, const uint32_t* __restrict__ block_off,
-    const uint64_t* __restrict__ start, K* __restrict__ out_keys, uint32_t* __restrict__ out_payload, uint64_t cap,
-    unsigned long long* __restrict__ dropped) {
-  extern __shared__ uint32_t brun[];  // [fan]: block cursor (absolute position)
-  const uint32_t fan = 1u << bits;
-  const uint64_t c = xcd_logical_block();
-  for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x)
-    brun[p] = static_cast<uint32_t>(start[p]) + block_off[c * fan + p];
-  __syncthreads();
-  const uint64_t lo = c * chunk;
-  const uint64_t hi = std::min<uint64_t>(m, lo + chunk);
-  for (uint64_t tile = lo; tile < hi; tile += kPartTile) {
-    K k[kPartItems];
-    uint32_t pay[kPartItems];
-#pragma unroll
-    for (int j = 0; j < kPartItems; ++j) {
-      const uint64_t i = tile + static_cast<uint64_t>(j * kPartBlock + threadIdx.x);
-      const bool valid = i < hi;
-      k[j] = valid ? load_stream(keys + i) : K(0);
-      pay[j] = valid ? (in_payload ? load_stream(in_payload + i) : payload_base + static_cast<uint32_t>(i)) : 0u;
-    }
-#pragma unroll
-    for (int j = 0; j < kPartItems; ++j) {
-      const uint64_t i = tile + static_cast<uint64_t>(j * kPartBlock + threadIdx.x);
-      if (i < hi) {
-        const uint32_t pos = atomicAdd(&brun[digit_of(k[j], shift, fan - 1)], 1u);
-        if (pos < cap) {  // always true for a consistent histogram
-          out_keys[pos] = k[j];
-          out_payload[pos] = pay[j];
-        } else {
-          drop(dropped);
-        }
-      }
-    }
-  }
-}
-
-// Write-combining scatter.  A random scatter into 2^bits runs leaves most output
-// lines partly written when L2 evicts them; each eviction then writes a partial
-// line, and a line is written back several times.  Here a block stages its items
-// in LDS and stores only whole aligned segments of L = 2^seg_bits slots (64 or
-// 128 bytes of keys), written by L consecutive lanes.
-//
-// LDS per block: a carry buffer of L slots per partition holding the items of the
-// partition's open segment, and the current tile of kWcTile items in partition
-// order.  Per tile:
-//   count   per partition (unordered: LDS atomic add, whose result is the item's
-//           rank in the tile; stable: per-wave rows as in part_scatter_kernel)
-//   scan    one block scan of (items, complete segments) per partition gives the
-//           tile offset of each partition and the list of segments to store
-//   place   items into the tile buffer at tile offset + rank
-//   store   each complete segment by L lanes: slots below the partition cursor
-//           come from the carry buffer, the others from the tile buffer
-//   carry   items past the last complete segment move into the carry buffer
-// At the end of the chunk the open segments are stored as they are.  The first
-// segment of a block's run is shared with the previous block: slots below the
-// run's first position (run0) are never stored by this block.
-constexpr int kWcTile = 2048;
-// Block size: at the larger fan-outs the carry buffer fills most of the LDS and
-// one block runs per CU, so the unordered scatter uses 1024 threads (4 waves per
-// SIMD) to keep loads in flight; the stable one uses 256 (its per-wave count rows
-// grow with the waves) and runs only where two blocks fit per CU.
-constexpr int wc_block(bool stable) { return stable ? 256 : 1024; }
-// Pair: the unordered kernel's LDS leaves room for two blocks per CU, and the kernel is
-// held to 64 VGPRs (8 waves per SIMD) so that both run.  Measured on 2^24-item windows:
-// fan-out 2^8 153 -> 129 us per launch with two blocks against one at 73 VGPRs, although
-// the cap spills 32 bytes; where the LDS admits one block only (fan-out 2^10) the cap
-// only adds the spills (+13 %), so it is not applied there.
-constexpr int wc_min_waves(bool stable, bool pair) { return (!stable && pair) ? 8 : 1; }
-
-__host__ __device__ constexpr uint32_t wc_max_segments(uint32_t fan, uint32_t seg_bits) {
-  // a tile completes at most one segment per partition beyond kWcTile / L
-  return (static_cast<uint32_t>(kWcTile) >> seg_bits) + (fan < static_cast<uint32_t>(kWcTile) ? fan : kWcTile);
-}
-
-__host__ __device__ constexpr size_t wc_lds_bytes(uint32_t fan, uint32_t seg_bits, int key_bytes, bool stable) {
-  const size_t item = static_cast<size_t>(key_bytes) + 4;
-  return static_cast<size_t>(fan) * (1u << seg_bits) * item      // carry keys + payloads
-         + static_cast<size_t>(kWcTile) * item                   // tile keys + payloads
-         + static_cast<size_t>(fan) * 4 * 4                      // cur, run0, off, endp
-         + static_cast<size_t>(fan) * 4 * (stable ? wc_block(true) / kWave : 1)  // counts
-         + (static_cast<size_t>(wc_max_segments(fan, seg_bits)) * 2 + 3) / 4 * 4;  // segment list
-}
-
-template <class K, bool Stable, bool Pair>
-__global__ __launch_bounds__(wc_block(Stable), wc_min_waves(Stable, Pair)) void part_scatter_wc_kernel(
-    const K* __restrict__ keys, const uint32_t* __restrict__ in_payload, uint32_t payload_base, uint64_t m,
-    uint64_t chunk, uint32_t shift, uint32_t bits, uint32_t seg_bits, const uint32_t* __restrict__ block_off,
-    const uint64_t* __restrict__ start, K* __restrict__ out_keys, uint32_t* __restrict__ out_payload,
-    uint32_t* __restrict__ inv, uint64_t cap, unsigned long long* __restrict__ dropped, Seg sg) {
-  constexpr int kBlock = wc_block(Stable);
-  constexpr int kWaves = kBlock / kWave;
-  constexpr int kItems = kWcTile / kBlock;  // items per lane per tile
-  constexpr int kRows = Stable ? kWaves : 1;
-  extern __shared__ uint64_t wsm_[];
-  __shared__ uint32_t wsum[kWaves];
-  const uint32_t fan = 1u << bits;
-  const uint32_t L = 1u << seg_bits;
-  const uint32_t lmask = L - 1;
-  K* ck = reinterpret_cast<K*>(wsm_);              // [fan][L] carry keys
-  K* sk = ck + static_cast<size_t>(fan) * L;        // [kWcTile] tile keys, partition order
-  uint32_t* cp = reinterpret_cast<uint32_t*>(sk + kWcTile);  // [fan][L] carry payloads
-  uint32_t* sp = cp + static_cast<size_t>(fan) * L;  // [kWcTile] tile payloads
-  uint32_t* cur = sp + kWcTile;                      // [fan] next output position of the block's run
-  uint32_t* run0 = cur + fan;                        // [fan] first position of the block's run
-  uint32_t* off = run0 + fan;                        // [fan] tile offset | first segment << 16
-  uint32_t* endp = off + fan;                        // [fan] cursor after the tile
-  uint32_t* cnt = endp + fan;                        // [kRows][fan]
-  uint16_t* segp = reinterpret_cast<uint16_t*>(cnt + kRows * fan);  // segment -> partition
-
   const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block();  // as part_hist_kernel
   uint64_t lo, hi, pbase;
   if (!seg_range(sg, c, chunk, m, fan, lo, hi, pbase)) return;  // block-uniform, before any barrier
-  for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x) {
-    const uint32_t r = static_cast<uint32_t>(start[pbase + p]) + block_off[c * fan + p];
-    cur[p] = r;
-    run0[p] = r;
-#pragma unroll
-    for (int v = 0; v < kRows; ++v) cnt[v * fan + p] = 0;
-  }
-  __syncthreads();
-  const int w = threadIdx.x / kWave;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   const int ln = lane();
-  const uint64_t lt = (ln == 0) ? 0ull : (~0ull >> (64 - ln));
-  // partitions owned by this thread in the scan: [p0, p0 + per)
-  const uint32_t per = fan > static_cast<uint32_t>(kBlock) ? fan / kBlock : 1u;
-  const uint32_t p0 = threadIdx.x * per;
-  const uint32_t groups = static_cast<uint32_t>(kBlock) >> seg_bits;  // L lanes per segment store
-  const uint32_t g = threadIdx.x >> seg_bits;
-  const uint32_t q = threadIdx.x & lmask;
-
-  // The next tile's items are loaded while this tile is counted, placed and stored (the
-  // barriers wait for LDS operations only, so the loads stay in flight across them).
-  K kn[kItems];
-  uint32_t pn[kItems];
-  auto load_tile = [&](uint64_t t) {
-    const uint64_t b = t + static_cast<uint64_t>(w) * (kItems * kWave);
-#pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const uint64_t i = b + static_cast<uint64_t>(j * kWave + ln);
-      const bool valid = i < hi;
-      kn[j] = valid ? load_stream(keys + i) : K(0);
-      pn[j] = valid ? (in_payload ? load_stream(in_payload + i) : payload_base + static_cast<uint32_t>(i)) : 0u;
+  const uint64_t lt = (ln == 0) ? 0ull : (~0ull >> (64 - ln));  // lanes below this one
+  uint16_t* mine = rows + static_cast<size_t>(w) * fan;
+  for (uint32_t p = threadIdx.x; p < fan; p += B) {
+    cur[p] = static_cast<uint32_t>(start[pbase + p]) + block_off[c * fan + p];
+    if constexpr (!Stable) cnt[p] = 0;
+  }
+  auto clear_row = [&] {
+    if (fan >= 8) {
+      for (uint32_t p = ln * 8; p < fan; p += kWave * 8) *reinterpret_cast<u32x4*>(mine + p) = u32x4{0, 0, 0, 0};
+    } else if (static_cast<uint32_t>(ln) < fan) {
+      mine[ln] = 0;
     }
   };
-  load_tile(lo);
-  for (uint64_t tile = lo; tile < hi; tile += kWcTile) {
-    const uint64_t wbase = tile + static_cast<uint64_t>(w) * (kItems * kWave);
-    K k[kItems];
-    uint32_t pay[kItems];
-    uint32_t rk[kItems];
+  if constexpr (Stable) clear_row();
+  __syncthreads();
+
+  // Counts -> tile offsets; the cursors move on.  Each thread owns PER consecutive
+  // partitions, whose 16-bit counts it adds two to a word.
+  auto scan = [&]<int PER>() {
+    const uint32_t p0 = threadIdx.x * PER;
+    const bool own = p0 < fan;
+    uint32_t n[PER], local = 0;
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      k[j] = kn[j];
-      pay[j] = pn[j];
-    }
-    if (tile + kWcTile < hi) load_tile(tile + kWcTile);  // block-uniform
-    // count
+    for (int u = 0; u < PER; ++u) n[u] = 0;
+    if (own) {
+      if constexpr (!Stable) {
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const uint64_t i = wbase + static_cast<uint64_t>(j * kWave + ln);
-      rk[j] = 0;
-      if (i < hi) {
-        const uint32_t d = digit_of(k[j], shift, fan - 1);
-        if constexpr (Stable)
-          atomicAdd(&cnt[w * fan + d], 1u);
-        else
-          rk[j] = atomicAdd(&cnt[d], 1u);
+        for (int u = 0; u < PER; ++u) n[u] = cnt[p0 + u];
+      } else if constexpr (PER == 1) {
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+          const uint32_t t = rows[v * fan + p0];
+          rows[v * fan + p0] = static_cast<uint16_t>(n[0]);
+          n[0] += t;
+        }
+      } else {
+        struct alignas(2 * PER) Words {
+          uint32_t w[PER / 2];
+        };
+        Words r{};
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+          Words* at = reinterpret_cast<Words*>(rows + v * fan + p0);
+          const Words t = *at;
+          *at = r;
+#pragma unroll
+          for (int q = 0; q < PER / 2; ++q) r.w[q] += t.w[q];  // a tile's counts sum below 2^16
+        }
+#pragma unroll
+        for (int u = 0; u < PER; ++u) n[u] = (r.w[u / 2] >> (16 * (u & 1))) & 0xFFFFu;
       }
-    }
-    __syncthreads();
-    // scan: per partition v = items | complete segments << 16 (both sums stay below 2^16)
-    uint32_t local = 0;
-    for (uint32_t u = 0; u < per; ++u) {
-      const uint32_t p = p0 + u;
-      if (p < fan) {
-        uint32_t n = 0;
 #pragma unroll
-        for (int v = 0; v < kRows; ++v) n += cnt[v * fan + p];
-        const uint32_t a = cur[p] & ~lmask;
-        const uint32_t e = cur[p] + n;
-        endp[p] = e;
-        local += n | (((e & ~lmask) - a) >> seg_bits) << 16;
-      }
+      for (int u = 0; u < PER; ++u) local += n[u];
     }
     uint32_t x = local;
 #pragma unroll
@@ -615,123 +461,140 @@ __global__ __launch_bounds__(wc_block(Stable), wc_min_waves(Stable, Pair)) void 
     if (ln == kWave - 1) wsum[w] = x;
     __syncthreads();
     uint32_t run = x - local;
-    uint32_t total = 0;
 #pragma unroll
-    for (int v = 0; v < kWaves; ++v) {
-      if (v < w) run += wsum[v];
-      total += wsum[v];
-    }
-    const uint32_t nseg_total = total >> 16;
-    for (uint32_t u = 0; u < per; ++u) {
-      const uint32_t p = p0 + u;
-      if (p < fan) {
-        off[p] = run;
-        uint32_t n = 0;
-        if constexpr (Stable) {
-          // wave rows become tile cursors: tile offset + items of earlier waves
-          uint32_t r = run & 0xFFFFu;
+    for (int v = 0; v < W; ++v) run += v < w ? wsum[v] : 0u;
+    if (own) {
 #pragma unroll
-          for (int v = 0; v < kWaves; ++v) {
-            const uint32_t t = cnt[v * fan + p];
-            cnt[v * fan + p] = r;
-            r += t;
-          }
-          n = r - (run & 0xFFFFu);
-        } else {
-          n = cnt[p];
-        }
-        const uint32_t ns = ((endp[p] & ~lmask) - (cur[p] & ~lmask)) >> seg_bits;
-        for (uint32_t t = 0; t < ns; ++t) segp[(run >> 16) + t] = static_cast<uint16_t>(p);
-        run += n | (ns << 16);
+      for (int u = 0; u < PER; ++u) {
+        const uint32_t q = cur[p0 + u];
+        if constexpr (Stable) off[p0 + u] = static_cast<uint16_t>(run);
+        else cnt[p0 + u] = run;
+        base[p0 + u] = q - run;
+        cur[p0 + u] = q + n[u];
+        run += n[u];
       }
     }
+  };
+
+  // The next tile's keys load while this tile is ranked, placed and stored (the barriers
+  // wait for LDS operations only, so the loads stay in flight across them).
+  K kn[I];
+  // items of this wave in the tile that starts at t (may be none)
+  auto wave_items = [&](uint64_t t) -> uint32_t {
+    const uint64_t b = t + static_cast<uint64_t>(w) * (I * kWave);
+    return b < hi ? static_cast<uint32_t>(std::min<uint64_t>(hi - b, I * kWave)) : 0u;
+  };
+  auto load_tile = [&](uint64_t t) {
+    const uint32_t nn = wave_items(t);
+    const K* src = keys + (t + static_cast<uint64_t>(w) * (I * kWave));
+#pragma unroll
+    for (int j = 0; j < I; ++j) {
+      const uint32_t i = static_cast<uint32_t>(j * kWave + ln);
+      kn[j] = i < nn ? load_stream(src + i) : K(0);
+    }
+  };
+  load_tile(lo);
+  for (uint64_t tile = lo; tile < hi; tile += T) {
+    const uint64_t wbase = tile + static_cast<uint64_t>(w) * (I * kWave);
+    const uint32_t wn = wave_items(tile);
+    K k[I];
+    uint32_t pay[InPayload ? I : 1], rk[I];
+#pragma unroll
+    for (int j = 0; j < I; ++j) {
+      k[j] = kn[j];
+      if constexpr (InPayload) {
+        const uint32_t i = static_cast<uint32_t>(j * kWave + ln);
+        pay[j] = i < wn ? load_stream(in_payload + wbase + i) : 0u;
+      }
+    }
+    if (tile + T < hi) load_tile(tile + T);  // block-uniform
+    if constexpr (Stable) {
+#pragma unroll
+      for (int j0 = 0; j0 < I; j0 += kRankItems) {
+        uint32_t plo[kRankItems], phi[kRankItems];  // lanes of the slice with this lane's digit
+#pragma unroll
+        for (int j = 0; j < kRankItems; ++j) {
+          const uint64_t valid = ballot(static_cast<uint32_t>((j0 + j) * kWave + ln) < wn);
+          plo[j] = static_cast<uint32_t>(valid);
+          phi[j] = static_cast<uint32_t>(valid >> 32);
+        }
+        for (uint32_t b = 0; b < bits; ++b) {
+#pragma unroll
+          for (int j = 0; j < kRankItems; ++j) {
+            const uint32_t one = 0u - digit_of(k[j0 + j], shift + b, 1u);  // all ones where the digit's bit b is set
+            const uint64_t set = ballot(one != 0);
+            plo[j] &= ~(static_cast<uint32_t>(set) ^ one);
+            phi[j] &= ~(static_cast<uint32_t>(set >> 32) ^ one);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < kRankItems; ++j) {
+          const uint32_t d = digit_of(k[j0 + j], shift, fan - 1);
+          const uint32_t before = static_cast<uint32_t>(__popc(plo[j] & static_cast<uint32_t>(lt)) +
+                                                        __popc(phi[j] & static_cast<uint32_t>(lt >> 32)));
+          const bool valid = static_cast<uint32_t>((j0 + j) * kWave + ln) < wn;
+          const uint32_t at = mine[d];  // every lane of the group reads the count before its first lane moves it
+          rk[j0 + j] = at + before;
+          if (valid && before == 0) mine[d] = static_cast<uint16_t>(at + __popc(plo[j]) + __popc(phi[j]));
+          __builtin_amdgcn_wave_barrier();
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < I; ++j) {
+        rk[j] = 0;
+        if (static_cast<uint32_t>(j * kWave + ln) < wn) rk[j] = atomicAdd(&cnt[digit_of(k[j], shift, fan - 1)], 1u);
+      }
+    }
+    __syncthreads();
+    if (fan <= static_cast<uint32_t>(B)) scan.template operator()<1>();
+    else if (fan == 2u * B) scan.template operator()<2>();
+    else if (fan == 4u * B) scan.template operator()<4>();
+    else scan.template operator()<8>();
     __syncthreads();
     // place
-    uint32_t pos[kItems];
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const uint64_t i = wbase + static_cast<uint64_t>(j * kWave + ln);
-      const bool valid = i < hi;
-      const uint32_t d = digit_of(k[j], shift, fan - 1);
-      uint32_t slot = 0;
-      if constexpr (Stable) {
-        uint64_t peers = ballot(valid);
-        for (uint32_t b = 0; b < bits; ++b) {
-          const uint64_t set = ballot((d >> b) & 1u);
-          peers &= ((d >> b) & 1u) ? set : ~set;
-        }
-        if (valid) {
-          const uint32_t at = cnt[w * fan + d];  // read by every lane of the group before the leader moves it
-          slot = at + static_cast<uint32_t>(__popcll(peers & lt));
-          if ((peers & lt) == 0) cnt[w * fan + d] = at + static_cast<uint32_t>(__popcll(peers));
-        }
-        __builtin_amdgcn_wave_barrier();
-      } else {
-        slot = (off[d] & 0xFFFFu) + rk[j];
-      }
-      pos[j] = 0xFFFFFFFFu;
-      if (valid && slot < static_cast<uint32_t>(kWcTile)) {  // slot < kWcTile for a consistent count
-        sk[slot] = k[j];
-        sp[slot] = pay[j];
-        pos[j] = cur[d] + slot - (off[d] & 0xFFFFu);
-      } else if (valid) {
-        drop(dropped);
-      }
-      if (inv && valid) inv[i] = pos[j];
-    }
-    __syncthreads();
-    // store the complete segments, L lanes each
-    for (uint32_t sg = g; sg < nseg_total; sg += groups) {
-      const uint32_t p = segp[sg];
-      const uint32_t o = off[p];
-      const uint32_t cp0 = cur[p];
-      const uint32_t at = (cp0 & ~lmask) + ((sg - (o >> 16)) << seg_bits) + q;
-      if (at >= run0[p] && at >= cap) drop(dropped);
-      if (at >= run0[p] && at < cap) {
-        K kk;
-        uint32_t pp;
-        if (at < cp0) {
-          kk = ck[p * L + (at & lmask)];
-          pp = cp[p * L + (at & lmask)];
-        } else {
-          const uint32_t t = (o & 0xFFFFu) + (at - cp0);
-          kk = sk[t];
-          pp = sp[t];
-        }
-        out_keys[at] = kk;
-        if (out_payload) out_payload[at] = pp;
-      }
-    }
-    __syncthreads();
-    // carry the items of each open segment; cursors move to the tile's end
-#pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      if (pos[j] != 0xFFFFFFFFu) {
+    for (int j = 0; j < I; ++j) {
+      if (static_cast<uint32_t>(j * kWave + ln) < wn) {
         const uint32_t d = digit_of(k[j], shift, fan - 1);
-        if (pos[j] >= (endp[d] & ~lmask)) {
-          ck[d * L + (pos[j] & lmask)] = k[j];
-          cp[d * L + (pos[j] & lmask)] = pay[j];
+        uint32_t slot;
+        if constexpr (Stable) slot = off[d] + mine[d] + rk[j];
+        else slot = cnt[d] + rk[j];
+        if (slot < static_cast<uint32_t>(T)) {  // always true for a consistent count
+          sk[slot] = k[j];
+          if (out_payload) {
+            if constexpr (InPayload) sp[slot] = pay[j];
+            else sp[slot] = payload_base + static_cast<uint32_t>(wbase) + static_cast<uint32_t>(j * kWave + ln);
+          }
+        }
+        if (inv) (inv + wbase)[j * kWave + ln] = base[d] + slot;
+      }
+    }
+    if constexpr (Stable) {
+      __builtin_amdgcn_wave_barrier();
+      clear_row();
+    }
+    __syncthreads();
+    if constexpr (!Stable) {  // read by the place phase, counted again from the next tile's start on
+      for (uint32_t p = threadIdx.x; p < fan; p += B) cnt[p] = 0;
+    }
+    // store
+    const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(hi - tile, T));
+#pragma unroll
+    for (int j = 0; j < I; ++j) {
+      const uint32_t t = static_cast<uint32_t>(j * B) + threadIdx.x;
+      if (t < n) {
+        const K kk = sk[t];
+        const uint32_t pos = base[digit_of(kk, shift, fan - 1)] + t;
+        if (pos < cap) {  // always true for a consistent histogram
+          out_keys[pos] = kk;
+          if (out_payload) out_payload[pos] = sp[t];
+        } else {
+          drop(dropped);
         }
       }
     }
-    for (uint32_t u = 0; u < per; ++u) {
-      const uint32_t p = p0 + u;
-      if (p < fan) {
-        cur[p] = endp[p];
-#pragma unroll
-        for (int v = 0; v < kRows; ++v) cnt[v * fan + p] = 0;
-      }
-    }
-    __syncthreads();
-  }
-  // open segments: the slots of the block's run in [segment start, cursor)
-  for (uint32_t p = g; p < fan; p += groups) {
-    const uint32_t at = (cur[p] & ~lmask) + q;
-    if (at >= run0[p] && at < cur[p] && at >= cap) drop(dropped);
-    if (at >= run0[p] && at < cur[p] && at < cap) {
-      out_keys[at] = ck[p * L + q];
-      if (out_payload) out_payload[at] = cp[p * L + q];
-    }
+    if constexpr (!Stable) __syncthreads();  // the counts are zero before the next tile adds to them
   }
 }
 
@@ -853,19 +716,53 @@ uint64_t hist_bytes(uint64_t m, uint32_t bits, int cu) {
   return kScanSumsBytes + ceil_div(static_cast<uint64_t>(p.blocks) * p.fan * 4 + 256, 256) * 256;
 }
 
-// Segment size (log2 of slots) of the write-combining scatter: the largest with
-// segments of at most 128 bytes of keys whose LDS fits the block; 0 selects the
-// register-tile scatter.  The unordered scatter runs 1024 threads in one block
-// per CU and fits up to fan-out 1024.  The stable one runs 256 threads and pays
-// off only with two blocks per CU (fan-out up to 128 for u64 keys); with one it
-// is slower than the register-tile scatter.
-uint32_t wc_seg_bits(uint32_t bits, int key_bytes, bool stable) {
-  const uint32_t fan = 1u << bits;
-  const uint32_t sb = key_bytes == 4 ? 5u : 4u;
-  if (stable) return wc_lds_bytes(fan, sb, key_bytes, true) <= kMaxLds / 2 ? sb : 0u;
-  for (uint32_t b = sb; b >= 2; --b)
-    if (wc_lds_bytes(fan, b, key_bytes, false) <= kMaxLds) return b;
-  return 0;
+// Workgroups of the scatter: 512 threads of 8 items, 4096 items a tile (two workgroups per
+// CU at fan-out 2^10).  10^7 u64 keys, whole call: at 2^10 partitions 147 us against 206
+// with 2048-item tiles (shorter runs) and 149 with 8192-item ones (one workgroup per CU);
+// at 2^4 87 against 88 and 113.
+constexpr int kTileBlock = 512;
+constexpr int kTileItems = 8;
+static_assert(kTileBlock * kTileItems == kPartTile, "chunks are whole tiles");
+
+// What a scatter launch reads and writes (see part_scatter_kernel).
+template <class K>
+struct Scatter {
+  const K* keys;
+  const uint32_t* in_payload;
+  uint32_t payload_base;
+  uint64_t m, chunk;
+  uint32_t shift, bits;
+  const uint32_t* hist;
+  const uint64_t* start;
+  const uint64_t* count;
+  uint32_t align;
+  K* out_keys;
+  uint32_t* out_payload;
+  uint32_t* inv;
+  uint64_t cap;
+  unsigned long long* dropped;
+  Seg sg;
+};
+
+template <class K>
+void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, hipStream_t s) {
+  const size_t lds = tile_lds_bytes(1u << a.bits, sizeof(K), a.out_payload != nullptr, stable, kTileBlock, kTileItems);
+  GJ_REQUIRE(lds <= kMaxLds - 1024 && (1u << a.bits) <= 8u * kTileBlock, GJ_ERR_INTERNAL,
+             "partition fan-out does not fit the LDS");
+  auto go = [&]<bool Stable, bool InPayload>() {
+    auto kernel = &part_scatter_kernel<K, Stable, InPayload, kTileBlock, kTileItems>;
+    if (lds > 65536)
+      GJ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kTileBlock), lds, s, a.keys, a.in_payload, a.payload_base, a.m, a.chunk,
+                       a.shift, a.bits, a.hist, a.start, a.count, a.align, a.out_keys, a.out_payload, a.inv, a.cap,
+                       a.dropped, a.sg);
+    GJ_HIP_CHECK(hipGetLastError());
+  };
+  if (stable && a.in_payload) go.template operator()<true, true>();
+  else if (stable) go.template operator()<true, false>();
+  else if (a.in_payload) go.template operator()<false, true>();
+  else go.template operator()<false, false>();
 }
 
 // Above 2^12 partitions: a first pass on the high seg_high_bits() bits, then the
@@ -904,60 +801,20 @@ uint64_t scratch_for(uint64_t m, int key_bytes, uint32_t bits, uint32_t passes, 
 template <class K>
 void partition_pass(const K* keys, const uint32_t* in_payload, uint32_t payload_base, uint64_t m, uint32_t shift,
                     uint32_t bits, uint32_t align, bool stable, K* out_keys, uint32_t* out_payload, uint64_t* start,
-                    uint64_t* count, uint32_t* hist, uint64_t* sums, unsigned long long* dropped, int cu,
-                    hipStream_t s) {
-  const uint32_t sb = wc_seg_bits(bits, sizeof(K), stable);
-  size_t slds = 0;
-  uint32_t per_cu = bits > 10 ? 2 : 4;  // the register-tile scatter holds 5 x 4 B per partition
-  if (sb) {
-    slds = wc_lds_bytes(1u << bits, sb, sizeof(K), stable);
-    per_cu = static_cast<uint32_t>(std::min<size_t>(kMaxBlocksPerCu, std::max<size_t>(1, kMaxLds / slds)));
-  }
-  const PartPlan p = plan(m, bits, cu, per_cu);
-  const size_t lds = p.fan * sizeof(uint32_t);
-  // with one or two chunks per CU a chunk gets 1024 threads
-  hipLaunchKernelGGL(part_hist_kernel<K>, dim3(p.blocks), dim3(per_cu <= 2 ? 1024 : kPartBlock), lds, s, keys, m,
-                     p.chunk, shift, bits, hist, Seg{});
+                    uint64_t* start2, uint64_t* count, uint32_t* hist, uint64_t* sums, unsigned long long* dropped,
+                    int cu, hipStream_t s) {
+  const PartPlan p = plan(m, bits, cu, 2);
+  hipLaunchKernelGGL(part_hist_kernel<K>, dim3(p.blocks), dim3(1024), p.fan * sizeof(uint32_t), s,
+                     keys, m, p.chunk, shift, bits, hist, Seg{});
   GJ_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(part_colscan_kernel, dim3((p.fan + 3) / 4), dim3(256), 0, s, hist, p.blocks, p.fan, count);
+  hipLaunchKernelGGL(part_colscan_kernel, dim3((p.fan + kWave - 1) / kWave), dim3(kColThreads), 0, s, hist, p.blocks,
+                     p.fan, count);
   GJ_HIP_CHECK(hipGetLastError());
-  launch_scan_starts(count, p.fan, align, start, sums, s);
-  if (align > 1) {
-    hipLaunchKernelGGL(part_pad_kernel<K>, dim3(pad_grid(p.fan)), dim3(256), 0, s, start, count, p.fan, align,
-                       out_keys, out_payload);
-    GJ_HIP_CHECK(hipGetLastError());
-  }
+  launch_scan_starts(count, p.fan, align, start, start2, sums, s);
   const uint64_t cap = m + (align > 1 ? static_cast<uint64_t>(p.fan) * align : 0ull);
-  if (sb) {
-    auto launch = [&](auto kernel) {
-      if (slds > 65536)
-        GJ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(slds)));
-      hipLaunchKernelGGL(kernel, dim3(p.blocks), dim3(wc_block(stable)), slds, s, keys, in_payload, payload_base, m,
-                         p.chunk, shift, bits, sb, hist, start, out_keys, out_payload, nullptr, cap, dropped, Seg{});
-      GJ_HIP_CHECK(hipGetLastError());
-    };
-    if (stable)
-      launch(&part_scatter_wc_kernel<K, true, false>);
-    else if (per_cu >= 2)
-      launch(&part_scatter_wc_kernel<K, false, true>);
-    else
-      launch(&part_scatter_wc_kernel<K, false, false>);
-    return;
-  }
-  if (!stable) {
-    hipLaunchKernelGGL(part_scatter_any_kernel<K>, dim3(p.blocks), dim3(kPartBlock), lds, s, keys, in_payload,
-                       payload_base, m, p.chunk, shift, bits, hist, start, out_keys, out_payload, cap, dropped);
-    GJ_HIP_CHECK(hipGetLastError());
-    return;
-  }
-  const size_t rlds = static_cast<size_t>(kPartWaves + 1) * p.fan * sizeof(uint32_t);  // <= 80 KiB of the 160
-  if (rlds > 65536)
-    GJ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&part_scatter_kernel<K>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(rlds)));
-  hipLaunchKernelGGL(part_scatter_kernel<K>, dim3(p.blocks), dim3(kPartBlock), rlds, s, keys, in_payload, payload_base,
-                     m, p.chunk, shift, bits, hist, start, out_keys, out_payload, nullptr, cap, dropped, Seg{});
-  GJ_HIP_CHECK(hipGetLastError());
+  launch_scatter<K>({keys, in_payload, payload_base, m, p.chunk, shift, bits, hist, start, count, align, out_keys,
+                     out_payload, nullptr, cap, dropped, Seg{}},
+                    stable, p.blocks, s);
 }
 
 uint64_t partition_capacity(uint64_t m, int key_bytes, uint32_t bits) {
@@ -972,12 +829,11 @@ uint64_t partition_scratch(uint64_t m, int key_bytes, uint32_t bits, uint32_t pa
 // on the high bits) at [start1[h], start1[h] + count1[h]) of keys / payload; each segment
 // is partitioned on the low `bits` bits (digit (k >> shift) & (2^bits - 1)) into output
 // partitions h * 2^bits + p, with 128-byte aligned starts.  Chunks never straddle
-// segments, so every histogram row and cursor belongs to one segment.  Stable: tiles of
-// kPartTile items through the register-tile scatter.  Unordered: chunks of kSegWcChunk
-// items through the write-combining scatter where its buffers fit (the register tiles
-// write each wave's few items per partition as partial lines: 52 B of writes per 12 B
-// tuple at 2^8 partitions per 2^16-item segment).
-constexpr uint64_t kSegWcChunk = 8 * kWcTile;
+// segments, so every histogram row and cursor belongs to one segment.
+constexpr uint64_t kSegChunk = 16384;
+// Segments of this many chunks on average scan their histogram columns with a workgroup
+// per 64 partitions; shorter ones take one thread per partition.
+constexpr uint64_t kSegWideChunks = 32;
 
 template <class K>
 void partition_segmented(const K* keys, const uint32_t* payload, uint64_t m, uint32_t shift, uint32_t bits,
@@ -987,49 +843,26 @@ void partition_segmented(const K* keys, const uint32_t* payload, uint64_t m, uin
                          unsigned long long* dropped, hipStream_t s) {
   const uint32_t fan = 1u << bits;
   const uint64_t total_fan = static_cast<uint64_t>(segs) * fan;
-  const uint32_t sb = stable ? 0u : wc_seg_bits(bits, sizeof(K), false);
-  const uint64_t chunk = sb ? kSegWcChunk : static_cast<uint64_t>(kPartTile);
-  const uint64_t blocks = ceil_div(m, chunk) + segs;  // an upper bound on the chunks
+  const uint64_t blocks = ceil_div(m, kSegChunk) + segs;  // an upper bound on the chunks
   GJ_REQUIRE(blocks < (1ull << 31), GJ_ERR_INVALID, "too many partition chunks");
-  hipLaunchKernelGGL(seg_chunks_kernel, dim3(1), dim3(1024), 0, s, count1, segs, chunk, chunk0);
+  hipLaunchKernelGGL(seg_chunks_kernel, dim3(1), dim3(1024), 0, s, count1, segs, kSegChunk, chunk0);
   GJ_HIP_CHECK(hipGetLastError());
   const Seg sg{chunk0, start1, count1, segs};
-  hipLaunchKernelGGL(part_hist_kernel<K>, dim3(static_cast<unsigned>(blocks)), dim3(sb ? 1024 : kPartBlock),
-                     fan * sizeof(uint32_t), s, keys, m, chunk, shift, bits, hist, sg);
+  hipLaunchKernelGGL(part_hist_kernel<K>, dim3(static_cast<unsigned>(blocks)), dim3(kTileBlock),
+                     fan * sizeof(uint32_t), s, keys, m, kSegChunk, shift, bits, hist, sg);
   GJ_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(seg_colscan_kernel, dim3(static_cast<unsigned>(ceil_div(total_fan, 256))), dim3(256), 0, s, hist,
-                     chunk0, segs, fan, count);
+  if (ceil_div(m, kSegChunk) >= kSegWideChunks * segs)
+    hipLaunchKernelGGL(seg_colscan_wide_kernel, dim3(segs * ((fan + kWave - 1) / kWave)), dim3(kColThreads), 0, s, hist,
+                       chunk0, fan, count);
+  else
+    hipLaunchKernelGGL(seg_colscan_kernel, dim3(static_cast<unsigned>(ceil_div(total_fan, 256))), dim3(256), 0, s, hist,
+                       chunk0, segs, fan, count);
   GJ_HIP_CHECK(hipGetLastError());
-  launch_scan_starts(count, total_fan, align, start, sums, s);
-  if (align > 1) {
-    hipLaunchKernelGGL(part_pad_kernel<K>, dim3(pad_grid(total_fan)), dim3(256), 0, s, start, count,
-                       static_cast<uint32_t>(total_fan), align, out_keys, out_payload);
-    GJ_HIP_CHECK(hipGetLastError());
-  }
+  launch_scan_starts(count, total_fan, align, start, nullptr, sums, s);
   const uint64_t cap = m + (align > 1 ? total_fan * align : 0ull);
-  if (sb) {
-    const size_t slds = wc_lds_bytes(fan, sb, sizeof(K), false);
-    auto launch = [&](auto kernel) {
-      if (slds > 65536)
-        GJ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(slds)));
-      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(wc_block(false)), slds, s, keys, payload,
-                         0u, m, chunk, shift, bits, sb, hist, start, out_keys, out_payload, inv, cap, dropped, sg);
-      GJ_HIP_CHECK(hipGetLastError());
-    };
-    if (kMaxLds / slds >= 2)
-      launch(&part_scatter_wc_kernel<K, false, true>);
-    else
-      launch(&part_scatter_wc_kernel<K, false, false>);
-    return;
-  }
-  const size_t rlds = static_cast<size_t>(kPartWaves + 1) * fan * sizeof(uint32_t);  // <= 80 KiB of the 160
-  if (rlds > 65536)
-    GJ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&part_scatter_kernel<K>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(rlds)));
-  hipLaunchKernelGGL(part_scatter_kernel<K>, dim3(static_cast<unsigned>(blocks)), dim3(kPartBlock), rlds, s, keys,
-                     payload, 0u, m, chunk, shift, bits, hist, start, out_keys, out_payload, inv, cap, dropped, sg);
-  GJ_HIP_CHECK(hipGetLastError());
+  launch_scatter<K>({keys, payload, 0u, m, kSegChunk, shift, bits, hist, start, count, align, out_keys, out_payload, inv,
+                     cap, dropped, sg},
+                    stable, static_cast<unsigned>(blocks), s);
 }
 
 namespace {
@@ -1134,7 +967,7 @@ template void partition_windows<uint64_t>(const uint64_t*, uint64_t, uint64_t, u
 template <class K>
 void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t bits, uint32_t ignore, uint32_t passes,
                     bool stable, K* out_keys, uint32_t* out_payload, uint64_t* start, uint64_t* count, uint8_t* scratch,
-                    unsigned long long* dropped, int cu, hipStream_t s) {
+                    unsigned long long* dropped, int cu, hipStream_t s, uint64_t* start2) {
   auto* sums = reinterpret_cast<uint64_t*>(scratch);
   uint32_t* hist = reinterpret_cast<uint32_t*>(scratch + kScanSumsBytes);
   const uint32_t align = part_align(sizeof(K));
@@ -1148,15 +981,16 @@ void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t b
     auto* start1 = reinterpret_cast<uint64_t*>(small);
     auto* count1 = start1 + segs + 2;
     auto* chunk0 = count1 + segs + 2;
-    partition_pass<K>(keys, nullptr, payload_base, m, ignore + lb, hb, 1, stable, tk, tp, start1, count1, hist,
+    partition_pass<K>(keys, nullptr, payload_base, m, ignore + lb, hb, 1, stable, tk, tp, start1, nullptr, count1, hist,
                       sums, dropped, cu, s);
     partition_segmented<K>(tk, tp, m, ignore, lb, segs, start1, count1, chunk0, align, stable, out_keys, out_payload,
                            nullptr, start, count, hist, sums, dropped, s);
+    if (start2) GJ_HIP_CHECK(hipMemcpyAsync(start2, start, (1ull << bits) * 8, hipMemcpyDeviceToDevice, s));
     return;
   }
   if (passes == 1 || bits < 2) {
-    partition_pass<K>(keys, nullptr, payload_base, m, ignore, bits, align, stable, out_keys, out_payload, start, count,
-                      hist, sums, dropped, cu, s);
+    partition_pass<K>(keys, nullptr, payload_base, m, ignore, bits, align, stable, out_keys, out_payload, start, start2,
+                      count, hist, sums, dropped, cu, s);
     return;
   }
   // pass 1: the high half of the digit, unpadded, into scratch; pass 2: the full digit.
@@ -1164,17 +998,17 @@ void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t b
   uint8_t* tmp = scratch + hist_bytes(m, bits, cu);
   K* tk = reinterpret_cast<K*>(tmp);
   uint32_t* tp = reinterpret_cast<uint32_t*>(tmp + ceil_div((m + 32) * sizeof(K), 256) * 256);
-  partition_pass<K>(keys, nullptr, payload_base, m, ignore + (bits - b_hi), b_hi, 1, stable, tk, tp, start, count,
-                    hist, sums, dropped, cu, s);
-  partition_pass<K>(tk, tp, 0, m, ignore, bits, align, stable, out_keys, out_payload, start, count, hist, sums,
+  partition_pass<K>(keys, nullptr, payload_base, m, ignore + (bits - b_hi), b_hi, 1, stable, tk, tp, start, nullptr,
+                    count, hist, sums, dropped, cu, s);
+  partition_pass<K>(tk, tp, 0, m, ignore, bits, align, stable, out_keys, out_payload, start, start2, count, hist, sums,
                     dropped, cu, s);
 }
 template void partition_keys<uint32_t>(const uint32_t*, uint64_t, uint32_t, uint32_t, uint32_t, uint32_t, bool,
                                        uint32_t*, uint32_t*, uint64_t*, uint64_t*, uint8_t*, unsigned long long*, int,
-                                       hipStream_t);
+                                       hipStream_t, uint64_t*);
 template void partition_keys<uint64_t>(const uint64_t*, uint64_t, uint32_t, uint32_t, uint32_t, uint32_t, bool,
                                        uint64_t*, uint32_t*, uint64_t*, uint64_t*, uint8_t*, unsigned long long*, int,
-                                       hipStream_t);
+                                       hipStream_t, uint64_t*);
 
 }  // namespace gj
 
@@ -1226,9 +1060,8 @@ int gj_partition(const void* d_keys, uint64_t m, int key_bytes, const gj_partiti
     dispatch_key(key_bytes, [&]<class K>() {
       partition_keys<K>(static_cast<const K*>(d_keys), m, 0, bits, params->ignore_bits, params->passes, true,
                         static_cast<K*>(out->d_keys), out->d_payloads, start, out->d_counts, sc,
-                        reinterpret_cast<unsigned long long*>(out->d_dropped), cu, s);
+                        reinterpret_cast<unsigned long long*>(out->d_dropped), cu, s, out->d_offsets);
     });
-    GJ_HIP_CHECK(hipMemcpyAsync(out->d_offsets, start, (1ull << bits) * 8, hipMemcpyDeviceToDevice, s));
   });
 }
 
