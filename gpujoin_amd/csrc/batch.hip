@@ -1174,9 +1174,9 @@ struct gj_batch_plan {
   const uint8_t* flag = nullptr;
   gj_agg_result* results = nullptr;
   // device copies (persistent)
-  dbuf d_batches, d_tile_start, d_counter;
-  dbuf d_tile_batch;  // batch of each persistent work item
-  dbuf d_partial;  // workgroup partial sums of the per-batch join-aggregate launches
+  dbuf d_batches{dbuf::unpooled_t{}}, d_tile_start{dbuf::unpooled_t{}}, d_counter{dbuf::unpooled_t{}};
+  dbuf d_tile_batch{dbuf::unpooled_t{}};  // batch of each persistent work item
+  dbuf d_partial{dbuf::unpooled_t{}};  // workgroup partial sums of the per-batch join-aggregate launches
   // side streams of the launch mode
   gj::GraphLanes lanes;
   // graph

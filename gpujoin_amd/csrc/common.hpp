@@ -58,26 +58,33 @@ int guarded(F&& f) {
   }
 }
 
+// Device blocks that released buffers leave for later ones (runtime.hip).  take: a block of
+// at least `bytes` on the current device, its true size in `cap`; its contents are
+// arbitrary.  give: waits for the device, like hipFree, and keeps or frees the block.
+void* device_take(size_t bytes, size_t& cap, int& dev);
+void device_give(void* p, size_t cap, int dev) noexcept;
+
 // Owning buffer (the role of device_array_wrapper, src/device_array.hpp:132-236): HBM,
 // or page-locked host memory mapped into the GPU's address space after to_host().
 struct dbuf {
   void* p = nullptr;
   size_t bytes = 0;
   bool host = false;
+  bool pooled = true;  // release() gives the block to the pool; false: hipMalloc and hipFree alone
+  size_t cap = 0;
+  int dev = 0;
+
+  struct unpooled_t {};
   dbuf() = default;
+  explicit dbuf(unpooled_t) : pooled(false) {}
   explicit dbuf(size_t b) { alloc(b); }
   dbuf(const dbuf&) = delete;
   dbuf& operator=(const dbuf&) = delete;
-  dbuf(dbuf&& o) noexcept : p(o.p), bytes(o.bytes), host(o.host) { o.p = nullptr; o.bytes = 0; o.host = false; }
+  dbuf(dbuf&& o) noexcept { take_over(o); }
   dbuf& operator=(dbuf&& o) noexcept {
     if (this != &o) {
       release();
-      p = o.p;
-      bytes = o.bytes;
-      host = o.host;
-      o.p = nullptr;
-      o.bytes = 0;
-      o.host = false;
+      take_over(o);
     }
     return *this;
   }
@@ -92,15 +99,20 @@ struct dbuf {
       (void)hipHostFree(h);
       GJ_HIP_CHECK(e);
     }
-    (void)hipFree(p);
+    const size_t b = bytes;
+    release();
     p = h;
+    bytes = b;
     host = true;
   }
   ~dbuf() { release(); }
   void alloc(size_t b) {
     release();
     if (b == 0) return;
-    GJ_HIP_CHECK(hipMalloc(&p, b));
+    if (pooled)
+      p = device_take(b, cap, dev);
+    else
+      GJ_HIP_CHECK(hipMalloc(&p, b));
     bytes = b;
   }
   // grow-only reallocation for reusable scratch
@@ -108,12 +120,32 @@ struct dbuf {
     if (b > bytes) alloc(b);
   }
   void release() {
-    if (p) (void)(host ? hipHostFree(p) : hipFree(p));
+    if (p) {
+      if (host)
+        (void)hipHostFree(p);
+      else if (pooled)
+        device_give(p, cap, dev);
+      else
+        (void)hipFree(p);
+    }
     p = nullptr;
     bytes = 0;
     host = false;
   }
   template <class T> T* as() const { return static_cast<T*>(p); }
+
+ private:
+  void take_over(dbuf& o) noexcept {
+    p = o.p;
+    bytes = o.bytes;
+    host = o.host;
+    pooled = o.pooled;
+    cap = o.cap;
+    dev = o.dev;
+    o.p = nullptr;
+    o.bytes = 0;
+    o.host = false;
+  }
 };
 
 inline hipStream_t S(gj_stream_t s) { return reinterpret_cast<hipStream_t>(s); }

@@ -83,7 +83,7 @@ struct gj_index {
   // join-aggregate's partial sums): one set per stream, grown on demand and kept
   // until the index is destroyed, so calls on different streams never share it.
   struct StreamScratch {
-    gj::dbuf a, b;
+    gj::dbuf a{gj::dbuf::unpooled_t{}}, b{gj::dbuf::unpooled_t{}};
   };
   mutable std::mutex scratch_mu;
   mutable std::map<hipStream_t, std::unique_ptr<StreamScratch>> scratch_by_stream;
