@@ -418,7 +418,6 @@ void build_extended(gj_index& ix, hipStream_t s) {
     case GJ_RADIX_SPLINE: build_rs<K>(ix, s); break;
     case GJ_LEARNED_PLR:
     case GJ_LEARNED_MLP:
-      build_btree<K>(ix, s);
       build_learned<K>(ix, s);
       break;
     case GJ_HASH: {

@@ -48,6 +48,48 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
+template <class T>
+__device__ __forceinline__ T wave_min(T v) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const T o = __shfl_xor(v, off, 64);
+    v = o < v ? o : v;
+  }
+  return v;
+}
+template <class T>
+__device__ __forceinline__ T wave_max(T v) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const T o = __shfl_xor(v, off, 64);
+    v = o > v ? o : v;
+  }
+  return v;
+}
+
+// out[at .. at + count) = value, each lane its own run (called by whole waves).  Long runs
+// (a gap between clusters can span a large part of the table) are written by the whole
+// wave, one run after the other.
+__device__ __forceinline__ void fill_runs(uint32_t* __restrict__ out, uint32_t at, uint32_t count, uint32_t value) {
+  constexpr uint32_t kOwn = 32;
+  uint64_t todo = ballot(count > kOwn);
+  if (count <= kOwn)
+    for (uint32_t k = 0; k < count; ++k) out[at + k] = value;
+  while (todo) {  // wave-uniform
+    const int src = __ffsll(static_cast<unsigned long long>(todo)) - 1;
+    const uint32_t a = shfl32(at, src), c = shfl32(count, src), v = shfl32(value, src);
+    for (uint32_t k = static_cast<uint32_t>(lane()); k < c; k += kWave) out[a + k] = v;
+    todo &= todo - 1;
+  }
+}
+
+__global__ void fill_words_kernel(uint32_t* __restrict__ out, uint64_t count, uint32_t value) {
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += stride) out[i] = value;
+}
+void fill_words(uint32_t* d, uint64_t count, uint32_t value, hipStream_t s) {
+  hipLaunchKernelGGL(fill_words_kernel, dim3(grid_for(count, 1024)), dim3(256), 0, s, d, count, value);
+  GJ_HIP_CHECK(hipGetLastError());
+}
+
 struct RootFitSums {
   double sx, sxx, st, sxt;
 };
@@ -233,21 +275,33 @@ struct Router {
   }
 };
 
-// start[l] = first position routed to a leaf >= l (start[] pre-filled with n); counts
-// routing inversions (which must not occur: the root is monotone).
-template <class K>
-__global__ void leaf_bounds_kernel(const K* __restrict__ col, uint64_t n, Router<K> route, uint32_t* __restrict__ start,
-                                   unsigned long long* inversions) {
+// start[l] = first position whose bin is >= l, for bins that ascend with the position
+// (start[] pre-filled with n); counts the positions whose bin is below their predecessor's
+// or at or past `bins` (neither occurs under a monotone model) in *bad.  The predecessor's
+// bin comes from the neighbouring lane.
+template <class K, class BinOf>
+__device__ __forceinline__ void bin_starts(const K* __restrict__ col, uint64_t n, uint64_t bins, BinOf&& bin_of,
+                                           uint32_t* __restrict__ start, unsigned long long* bad) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const uint32_t li = route(col[i]);
-    const int64_t lp = (i == 0) ? -1 : static_cast<int64_t>(route(col[i - 1]));
-    if (static_cast<int64_t>(li) < lp) {
-      atomicAdd(inversions, 1ull);
-      continue;
-    }
-    for (int64_t l = lp + 1; l <= static_cast<int64_t>(li); ++l) start[l] = static_cast<uint32_t>(i);
+  const uint64_t first = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (uint64_t base = first - lane(); base < n; base += stride) {
+    const uint64_t i = base + lane();
+    const bool active = i < n;
+    const uint64_t b = active ? bin_of(col[i]) : 0;
+    uint64_t before = shfl64(b, lane() == 0 ? 0 : lane() - 1) + 1;  // the first bin that starts here
+    if (lane() == 0) before = i == 0 ? 0 : bin_of(col[i - 1]) + 1;
+    const bool wrong = active && (b >= bins || b + 1 < before);
+    if (wrong) atomicAdd(bad, 1ull);
+    const bool run = active && !wrong && b + 1 > before;
+    fill_runs(start, static_cast<uint32_t>(before), run ? static_cast<uint32_t>(b + 1 - before) : 0u,
+              static_cast<uint32_t>(i));
   }
+}
+
+template <class K>
+__global__ __launch_bounds__(256) void leaf_bounds_kernel(const K* __restrict__ col, uint64_t n, Router<K> route,
+                                                          uint32_t* __restrict__ start, unsigned long long* inversions) {
+  bin_starts(col, n, route.leaves, [&](K key) { return static_cast<uint64_t>(route(key)); }, start, inversions);
 }
 
 // Build-time facts of one leaf (not read by lookups).
@@ -256,21 +310,42 @@ struct LeafFit {
   int32_t err_lo, err_hi;  // extremes of position - pred over the leaf's keys
 };
 
-// One block per leaf: least squares of local position on FP32 key offsets.
-// Leaf l covers positions [lo[l], hi[l]).
-template <class K>
-__global__ __launch_bounds__(256) void leaf_fit_kernel(const K* __restrict__ col, uint64_t n,
-                                                       const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
-                                                       uint32_t leaves, LeafModel* __restrict__ out,
-                                                       LeafFit* __restrict__ fit) {
-  const uint32_t l = blockIdx.x;
-  if (l >= leaves) return;
-  const uint64_t s = lo[l];
-  const uint64_t e = hi[l];
-  const uint64_t cnt = e > s ? e - s : 0;
+// Leaves are fitted and calibrated a wave each: the sums, the model and the error of every
+// key of the leaf under the exact lookup arithmetic in one kernel, without atomics (a
+// block per leaf and a pass of two atomics per key took 146 and 92 us over 2^20 keys in 2^16
+// leaves; this takes 14 us).  What bounds it: the wave's latency over its few keys, so a
+// leaf of more than kBigLeaf keys, which would be a long serial chain, is put on a list
+// that blocks of 1024 threads work off.
+constexpr uint32_t kBigLeaf = 4096;
+constexpr uint32_t kSmallLeaf = 64;  // keys per leaf, on average, up to which 16 lanes take one
+constexpr int kBigBlock = 1024;
+
+// v reduced by `pick` over the T threads (a part of a wave, a wave, or a block) that work
+// on a leaf; red: T / 64 entries of LDS, unused up to a wave.
+template <int T, class V, class Pick>
+__device__ __forceinline__ V leaf_reduce(V v, V* red, Pick&& pick) {
+  for (int off = (T < kWave ? T : kWave) / 2; off > 0; off >>= 1) v = pick(v, __shfl_xor(v, off, kWave));
+  if constexpr (T > kWave) {
+    __syncthreads();
+    if (lane() == 0) red[threadIdx.x / kWave] = v;
+    __syncthreads();
+    v = red[0];
+    for (int w = 1; w < T / kWave; ++w) v = pick(v, red[w]);
+  }
+  return v;
+}
+template <int T>
+__device__ __forceinline__ double leaf_sum(double v, double* red) {
+  return leaf_reduce<T>(v, red, [](double a, double b) { return a + b; });
+}
+
+// Least squares of local position on FP32 key offsets over the keys at [s, s + cnt).
+template <int T, class K>
+__device__ __forceinline__ LeafModel leaf_fit(const K* __restrict__ col, uint64_t n, uint64_t s, uint64_t cnt,
+                                              uint32_t t, double* red) {
   const uint64_t base = cnt ? static_cast<uint64_t>(col[s]) : 0;
   double sd = 0, sdd = 0, sj = 0, sdj = 0;
-  for (uint64_t j = threadIdx.x; j < cnt; j += blockDim.x) {
+  for (uint64_t j = t; j < cnt; j += T) {
     const double d = leaf_dkey(col[s + j], base);
     const double jj = static_cast<double>(j);
     sd += d;
@@ -278,80 +353,218 @@ __global__ __launch_bounds__(256) void leaf_fit_kernel(const K* __restrict__ col
     sj += jj;
     sdj += d * jj;
   }
-  sd = wave_sum(sd);
-  sdd = wave_sum(sdd);
-  sj = wave_sum(sj);
-  sdj = wave_sum(sdj);
-  __shared__ double red[4][4];
-  const int w = threadIdx.x / 64;
-  if (lane() == 0) {
-    red[w][0] = sd;
-    red[w][1] = sdd;
-    red[w][2] = sj;
-    red[w][3] = sdj;
+  sd = leaf_sum<T>(sd, red);
+  sdd = leaf_sum<T>(sdd, red);
+  sj = leaf_sum<T>(sj, red);
+  sdj = leaf_sum<T>(sdj, red);
+  double slope = 0, icpt = 0;
+  if (cnt > 1) {
+    const double c = static_cast<double>(cnt);
+    const double var = sdd - sd * sd / c;
+    if (var > 0) slope = (sdj - sd * sj / c) / var;
+    icpt = (sj - slope * sd) / c;
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < static_cast<int>(blockDim.x / 64); ++i) {
-      sd += red[i][0];
-      sdd += red[i][1];
-      sj += red[i][2];
-      sdj += red[i][3];
-    }
-    double slope = 0, icpt = 0;
-    if (cnt > 1) {
-      const double c = static_cast<double>(cnt);
-      const double var = sdd - sd * sd / c;
-      if (var > 0) slope = (sdj - sd * sj / c) / var;
-      icpt = (sj - slope * sd) / c;
-    }
-    double st = static_cast<double>(s) + std::floor(icpt + 0.5);
-    st = st < 0 ? 0 : (st > static_cast<double>(n) ? static_cast<double>(n) : st);
-    LeafModel m;
-    m.base_key = base;
-    m.start = static_cast<uint32_t>(st);
-    m.slope = static_cast<float>(slope);
-    out[l] = m;
-    fit[l] = LeafFit{static_cast<uint32_t>(s), static_cast<uint32_t>(cnt), INT_MAX, INT_MIN};
-  }
+  double st = static_cast<double>(s) + std::floor(icpt + 0.5);
+  st = st < 0 ? 0 : (st > static_cast<double>(n) ? static_cast<double>(n) : st);
+  LeafModel m;
+  m.base_key = base;
+  m.start = static_cast<uint32_t>(st);
+  m.slope = static_cast<float>(slope);
+  return m;
 }
 
-// err_lo/err_hi of the leaf each key is routed to, under the exact lookup arithmetic.
-template <class K>
-__global__ void leaf_error_kernel(const K* __restrict__ col, uint64_t n, Router<K> route,
-                                  const LeafModel* __restrict__ lm, LeafFit* __restrict__ fit) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const K key = col[i];
-    const uint32_t l = route(key);
-    const LeafModel m = lm[l];
-    const int64_t pred = leaf_pred(m, leaf_dkey(key, m.base_key));
-    int64_t e = static_cast<int64_t>(i) - pred;
+// Extremes of position - pred(key) over the leaf's keys, as the leaf's calibration.  An
+// empty leaf has none; one wider than max_width gets an emptied range (err_hi < err_lo).
+template <int T, class K, class Pred>
+__device__ __forceinline__ LeafFit leaf_calibrate(const K* __restrict__ col, uint64_t s, uint64_t cnt, uint32_t t,
+                                                  int64_t max_width, int* red, Pred&& pred) {
+  int lo = INT_MAX, hi = INT_MIN;
+  for (uint64_t j = t; j < cnt; j += T) {
+    int64_t e = static_cast<int64_t>(s + j) - pred(col[s + j]);
     e = e < INT_MIN / 2 ? INT_MIN / 2 : (e > INT_MAX / 2 ? INT_MAX / 2 : e);
-    atomicMin(&fit[l].err_lo, static_cast<int>(e));
-    atomicMax(&fit[l].err_hi, static_cast<int>(e));
+    lo = static_cast<int>(e) < lo ? static_cast<int>(e) : lo;
+    hi = static_cast<int>(e) > hi ? static_cast<int>(e) : hi;
   }
-}
-
-// Empty leaves predict their start (no key is routed to them); leaves wider than
-// max_width go to the B-tree (slope = NaN, error range emptied: err_hi < err_lo).
-__global__ void leaf_finalize_kernel(LeafModel* __restrict__ lm, LeafFit* __restrict__ fit, uint32_t leaves,
-                                     int64_t max_width) {
-  const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= leaves) return;
-  LeafFit f = fit[l];
-  if (f.count == 0) {
-    f.err_lo = 0;
-    f.err_hi = 0;
-    lm[l].slope = 0.0f;
-  } else if (static_cast<int64_t>(f.err_hi) - f.err_lo + 1 > max_width) {
+  lo = leaf_reduce<T>(lo, red, [](int a, int b) { return a < b ? a : b; });
+  hi = leaf_reduce<T>(hi, red, [](int a, int b) { return a > b ? a : b; });
+  LeafFit f{static_cast<uint32_t>(s), static_cast<uint32_t>(cnt), lo, hi};
+  if (cnt == 0) {
+    f.err_lo = f.err_hi = 0;
+  } else if (static_cast<int64_t>(hi) - lo + 1 > max_width) {
     f.err_lo = 1;
     f.err_hi = 0;
-    lm[l].slope = __builtin_nanf("");
-    lm[l].start = kNoSplit;
   }
-  fit[l] = f;
+  return f;
 }
+
+// What a leaf kernel does with leaf l, covering positions [s, s + cnt), with T threads.
+// Fits the 16-byte model; a leaf wider than max_width goes to the B-tree (slope = NaN).
+template <class K>
+struct FitLeaf {
+  LeafModel* out;
+  template <int T>
+  __device__ __forceinline__ LeafFit run(const K* col, uint64_t n, uint32_t l, uint64_t s, uint64_t cnt, uint32_t t,
+                                         int64_t max_width, void* red) const {
+    LeafModel m = leaf_fit<T>(col, n, s, cnt, t, static_cast<double*>(red));
+    const LeafFit f = leaf_calibrate<T>(col, s, cnt, t, max_width, static_cast<int*>(red),
+                                        [&](K key) { return leaf_pred(m, leaf_dkey(key, m.base_key)); });
+    if (f.err_hi < f.err_lo) {
+      m.slope = __builtin_nanf("");
+      m.start = kNoSplit;
+    }
+    if (t == 0) out[l] = m;
+    return f;
+  }
+};
+
+// 16-byte leaf -> compact leaf over its group: start + slope * (key - base) equals
+// group.start + slope * (key - group.base) + icpt for icpt = start - group.start
+// + slope * (group.base - base).
+template <class K>
+struct CompactLeaf {
+  const LeafModel* lm;
+  const LeafGroup* groups;
+  uint32_t gshift;
+  LeafCompact* out;
+  template <int T>
+  __device__ __forceinline__ LeafFit run(const K* col, uint64_t, uint32_t l, uint64_t s, uint64_t cnt, uint32_t t,
+                                         int64_t max_width, void* red) const {
+    const LeafModel m = lm[l];
+    const LeafGroup g = groups[l >> gshift];
+    double icpt = static_cast<double>(static_cast<int64_t>(m.start) - static_cast<int64_t>(g.start));
+    if (m.slope != 0.0f)
+      icpt += static_cast<double>(m.slope) * static_cast<double>(static_cast<int64_t>(g.base_key - m.base_key));
+    const LeafCompact c{m.slope, static_cast<float>(icpt)};
+    if (t == 0) out[l] = c;
+    return leaf_calibrate<T>(col, s, cnt, t, max_width, static_cast<int*>(red),
+                             [&](K key) { return compact_pred(c, g, leaf_dkey(key, g.base_key)); });
+  }
+};
+
+// Leaf l covers positions [lo[l], hi[l]); big leaves are appended to `big` (null: none is left out).
+template <int T, class K, class Op>
+__global__ __launch_bounds__(256) void leaf_wave_kernel(const K* __restrict__ col, uint64_t n,
+                                                        const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
+                                                        uint32_t leaves, int64_t max_width, Op op,
+                                                        LeafFit* __restrict__ fit, uint32_t* __restrict__ big_count,
+                                                        uint32_t* __restrict__ big) {
+  const uint32_t l = blockIdx.x * (256 / T) + threadIdx.x / T;
+  if (l >= leaves) return;
+  const uint64_t s = lo[l], e = hi[l];
+  const uint64_t cnt = e > s ? e - s : 0;
+  const uint32_t t = threadIdx.x % T;
+  if (cnt > kBigLeaf) {
+    if (t == 0) big[atomicAdd(big_count, 1u)] = l;
+    return;
+  }
+  const LeafFit f = op.template run<T>(col, n, l, s, cnt, t, max_width, nullptr);
+  if (t == 0) fit[l] = f;
+}
+
+template <class K, class Op>
+__global__ __launch_bounds__(kBigBlock) void leaf_big_kernel(const K* __restrict__ col, uint64_t n,
+                                                             const uint32_t* __restrict__ lo,
+                                                             const uint32_t* __restrict__ hi, int64_t max_width, Op op,
+                                                             LeafFit* __restrict__ fit,
+                                                             const uint32_t* __restrict__ big_count,
+                                                             const uint32_t* __restrict__ big) {
+  __shared__ double red[kBigBlock / kWave];
+  const uint32_t count = *big_count;
+  for (uint32_t q = blockIdx.x; q < count; q += gridDim.x) {
+    const uint32_t l = big[q];
+    const uint64_t s = lo[l];
+    const LeafFit f = op.template run<kBigBlock>(col, n, l, s, hi[l] - s, threadIdx.x, max_width, red);
+    if (threadIdx.x == 0) fit[l] = f;
+    __syncthreads();  // the next leaf's reductions reuse red
+  }
+}
+
+// Totals over the leaves, those with an emptied range (routed to the B-tree) apart.
+struct LeafStats {
+  unsigned long long fb_leaves, fb_keys, wsum, wkeys;  // wsum: window widths weighted by keys
+  uint32_t wmax;
+  int32_t err_lo, err_hi;
+  uint32_t big;  // entries of the big-leaf list
+};
+__global__ __launch_bounds__(kBigBlock) void leaf_stats_kernel(const LeafFit* __restrict__ fit, uint32_t leaves,
+                                                         LeafStats* __restrict__ st) {
+  uint64_t fbl = 0, fbk = 0, ws = 0, wk = 0;
+  uint32_t wm = 0;
+  int lo = 0, hi = 0;
+  for (uint32_t l = blockIdx.x * blockDim.x + threadIdx.x; l < leaves; l += gridDim.x * blockDim.x) {
+    const LeafFit f = fit[l];
+    if (f.count == 0) continue;
+    if (f.err_hi < f.err_lo) {
+      ++fbl;
+      fbk += f.count;
+    } else {
+      const uint32_t w = static_cast<uint32_t>(f.err_hi - f.err_lo + 1);
+      wm = w > wm ? w : wm;
+      ws += static_cast<uint64_t>(w) * f.count;
+      wk += f.count;
+      lo = f.err_lo < lo ? f.err_lo : lo;
+      hi = f.err_hi > hi ? f.err_hi : hi;
+    }
+  }
+  // block totals first: atomics on one address cost 10 ns each
+  __shared__ LeafStats part[kBigBlock / kWave];
+  LeafStats t{wave_sum(fbl), wave_sum(fbk), wave_sum(ws), wave_sum(wk), wave_max(wm), wave_min(lo), wave_max(hi), 0};
+  if (lane() == 0) part[threadIdx.x / kWave] = t;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < kBigBlock / kWave; ++w) {
+    t.fb_leaves += part[w].fb_leaves;
+    t.fb_keys += part[w].fb_keys;
+    t.wsum += part[w].wsum;
+    t.wkeys += part[w].wkeys;
+    t.wmax = part[w].wmax > t.wmax ? part[w].wmax : t.wmax;
+    t.err_lo = part[w].err_lo < t.err_lo ? part[w].err_lo : t.err_lo;
+    t.err_hi = part[w].err_hi > t.err_hi ? part[w].err_hi : t.err_hi;
+  }
+  if (t.fb_leaves) {
+    atomicAdd(&st->fb_leaves, t.fb_leaves);
+    atomicAdd(&st->fb_keys, t.fb_keys);
+  }
+  if (t.wkeys) {
+    atomicAdd(&st->wsum, t.wsum);
+    atomicAdd(&st->wkeys, t.wkeys);
+    atomicMax(&st->wmax, t.wmax);
+    if (t.err_lo < 0) atomicMin(&st->err_lo, t.err_lo);
+    if (t.err_hi > 0) atomicMax(&st->err_hi, t.err_hi);
+  }
+}
+
+// Runs Op over the leaves and reads their totals back.
+struct LeafPass {
+  dbuf work;  // LeafStats | big-leaf list
+  template <class K, class Op>
+  LeafStats run(const K* col, uint64_t n, const uint32_t* lo, const uint32_t* hi, uint32_t leaves, int64_t max_width,
+                const Op& op, LeafFit* fit, hipStream_t s) {
+    const uint64_t bigs = std::min<uint64_t>(leaves, n / kBigLeaf + 1);
+    work.reserve(sizeof(LeafStats) + bigs * sizeof(uint32_t));
+    LeafStats* st = work.as<LeafStats>();
+    uint32_t* big = reinterpret_cast<uint32_t*>(st + 1);
+    fill_bytes(st, 0, sizeof(LeafStats), s);
+    auto fit_with = [&]<int T>() {
+      hipLaunchKernelGGL((leaf_wave_kernel<T, K, Op>), dim3(grid_for(leaves, 256 / T, 0x7FFFFFFFu)), dim3(256), 0, s, col,
+                         n, lo, hi, leaves, max_width, op, fit, &st->big, big);
+    };
+    if (n / leaves <= kSmallLeaf)
+      fit_with.template operator()<16>();
+    else
+      fit_with.template operator()<kWave>();
+    GJ_HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL((leaf_big_kernel<K, Op>), dim3(static_cast<unsigned>(std::min<uint64_t>(bigs, 256))),
+                       dim3(kBigBlock), 0, s, col, n, lo, hi, max_width, op, fit, &st->big, big);
+    GJ_HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(leaf_stats_kernel, dim3(grid_for(leaves, kBigBlock, 32)), dim3(kBigBlock), 0, s, fit, leaves, st);
+    GJ_HIP_CHECK(hipGetLastError());
+    LeafStats h{};
+    GJ_HIP_CHECK(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
+    GJ_HIP_CHECK(hipStreamSynchronize(s));
+    return h;
+  }
+};
 
 // Separator line of split j: sub-leaf t covers [sub_lo, sub_hi); its separator is the
 // key at sub_hi - 1 (at the leaf's first position for an empty leading sub-leaf), the
@@ -372,28 +585,6 @@ __global__ void split_sep_kernel(const K* __restrict__ col, const uint32_t* __re
   const uint32_t h = sub_hi[g];
   const uint32_t at = h > leaf_lo[j] ? h - 1 : leaf_lo[j];
   sep[g] = static_cast<uint64_t>(col[at]);
-}
-
-// err_lo/err_hi of the sub-leaves: one block per split leaf, over the leaf's keys,
-// with the separator count and arithmetic of the lookup.
-template <class K>
-__global__ void split_error_kernel(const K* __restrict__ col, const uint32_t* __restrict__ leaf_lo,
-                                   const uint32_t* __restrict__ leaf_hi, const uint64_t* __restrict__ sep,
-                                   const LeafModel* __restrict__ subs, LeafFit* __restrict__ fit) {
-  const uint32_t j = blockIdx.x;
-  const uint64_t* sp = sep + static_cast<uint64_t>(j) * kSplitWays;
-  for (uint64_t i = leaf_lo[j] + threadIdx.x; i < leaf_hi[j]; i += blockDim.x) {
-    const K key = col[i];
-    uint32_t t = 0;
-    for (uint32_t u = 0; u < kSplitWays; ++u) t += sp[u] < static_cast<uint64_t>(key) ? 1u : 0u;
-    t = t < kSplitWays ? t : kSplitWays - 1;
-    const uint64_t g = static_cast<uint64_t>(j) * kSplitWays + t;
-    const LeafModel m = subs[g];
-    int64_t e = static_cast<int64_t>(i) - leaf_pred(m, leaf_dkey(key, m.base_key));
-    e = e < INT_MIN / 2 ? INT_MIN / 2 : (e > INT_MAX / 2 ? INT_MAX / 2 : e);
-    atomicMin(&fit[g].err_lo, static_cast<int>(e));
-    atomicMax(&fit[g].err_hi, static_cast<int>(e));
-  }
 }
 
 // The split leaves' own models: slope = NaN, start = split index.
@@ -422,74 +613,235 @@ __global__ void compact_groups_kernel(const K* __restrict__ col, uint64_t n, con
   out[g] = r;
 }
 
-// 16-byte leaf -> compact leaf over its group: start + slope * (key - base) equals
-// group.start + slope * (key - group.base) + icpt for icpt = start - group.start
-// + slope * (group.base - base).  Resets the leaf's error range for re-measuring.
-__global__ void compact_convert_kernel(const LeafModel* __restrict__ lm, const LeafGroup* __restrict__ groups,
-                                       uint32_t leaves, uint32_t gshift, LeafCompact* __restrict__ out,
-                                       LeafFit* __restrict__ fit) {
-  const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= leaves) return;
-  const LeafModel m = lm[l];
-  const LeafGroup g = groups[l >> gshift];
-  double icpt = static_cast<double>(static_cast<int64_t>(m.start) - static_cast<int64_t>(g.start));
-  if (m.slope != 0.0f)
-    icpt += static_cast<double>(m.slope) * static_cast<double>(static_cast<int64_t>(g.base_key - m.base_key));
-  out[l] = LeafCompact{m.slope, static_cast<float>(icpt)};
-  fit[l].err_lo = INT_MAX;
-  fit[l].err_hi = INT_MIN;
-}
-
-// err_lo/err_hi of every compact leaf under the exact lookup arithmetic.
-template <class K>
-__global__ void compact_error_kernel(const K* __restrict__ col, uint64_t n, Router<K> route,
-                                     const LeafCompact* __restrict__ lc, const LeafGroup* __restrict__ groups,
-                                     uint32_t gshift, LeafFit* __restrict__ fit) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const K key = col[i];
-    const uint32_t l = route(key);
-    const LeafGroup g = groups[l >> gshift];
-    const int64_t pred = compact_pred(lc[l], g, leaf_dkey(key, g.base_key));
-    int64_t e = static_cast<int64_t>(i) - pred;
-    e = e < INT_MIN / 2 ? INT_MIN / 2 : (e > INT_MAX / 2 ? INT_MAX / 2 : e);
-    atomicMin(&fit[l].err_lo, static_cast<int>(e));
-    atomicMax(&fit[l].err_hi, static_cast<int>(e));
-  }
-}
-
 // ---- lines layout ------------------------------------------------------------
 
+// What the placement reports to the host.
+struct LineStats {
+  unsigned long long bad;    // keys whose target is not monotone or not below the line count
+  unsigned long long carry;  // sum over lines l of the keys with a target below l that are placed at l or later
+  uint32_t base_end;         // first key past the target lines
+  uint32_t max_spill;        // farthest line from its first key's target
+};
+
 // first[l] = first position whose target line is >= l (first[] pre-filled with n).
-// Counts keys whose target falls below their predecessor's or at or past
-// `targets` (neither may occur: the target is monotone and bounded).
 template <class K>
-__global__ void line_first_kernel(const K* __restrict__ col, uint64_t n, LinesDev<K> d, const uint8_t* rp,
-                                  uint64_t targets, uint32_t* __restrict__ first, unsigned long long* bad) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const uint64_t t = d.target(col[i], rp);
-    const int64_t tp = (i == 0) ? -1 : static_cast<int64_t>(d.target(col[i - 1], rp));
-    if (t >= targets || static_cast<int64_t>(t) < tp) {
-      atomicAdd(bad, 1ull);
-      continue;
+__global__ __launch_bounds__(256) void line_first_kernel(const K* __restrict__ col, uint64_t n, LinesDev<K> d,
+                                                         const uint8_t* rp, uint64_t targets,
+                                                         uint32_t* __restrict__ first, LineStats* st) {
+  bin_starts(col, n, targets, [&](K key) { return d.target(key, rp); }, first, &st->bad);
+}
+
+// Placement.  In key order, line l takes the keys carried over from line l - 1, then its own
+// (targets of l), up to CAP; the rest moves on.  With base[l] = keys placed before line l:
+//   base[l + 1] = min(first[l + 1], base[l] + CAP), hence
+//   base[l] = CAP * l + min over j <= l of (first[j] - CAP * j),
+// a running minimum: one pass for the minima of the blocks' spans, one that scans each span
+// from the minimum before it.  Past the last target line every line takes CAP keys, so
+// base[targets + k] = min(n, base[targets] + CAP * k) needs no entry.
+// What bounds it: streaming.  On the host the same recurrence cost 3.0 of the 4.4 ms of a
+// build over 12.3 M u64 keys (1.23 M lines), and its arrays another 0.8 ms of copies;
+// the two passes take 17 us.
+constexpr int kPlaceBlock = 256;
+constexpr int kPlaceItems = 8;                              // consecutive lines per thread
+constexpr uint64_t kPlaceTile = kPlaceBlock * kPlaceItems;  // lines per step of a block
+constexpr uint64_t kPlaceBlocks = 2048;                     // each block reads the minima of all earlier ones
+
+__device__ __forceinline__ int64_t block_min(int64_t v, int64_t* red) {
+  v = wave_min(v);
+  __syncthreads();
+  if (lane() == 0) red[threadIdx.x / kWave] = v;
+  __syncthreads();
+  int64_t r = red[0];
+  for (int w = 1; w < kPlaceBlock / kWave; ++w) r = red[w] < r ? red[w] : r;
+  return r;
+}
+
+template <uint32_t CAP>
+__global__ __launch_bounds__(kPlaceBlock) void line_span_min_kernel(const uint32_t* __restrict__ first, uint64_t entries,
+                                                                    uint64_t span, int64_t* __restrict__ mins) {
+  __shared__ int64_t red[kPlaceBlock / kWave];
+  const uint64_t lo = blockIdx.x * span, hi = lo + span < entries ? lo + span : entries;
+  int64_t m = INT64_MAX;
+  for (uint64_t j = lo + threadIdx.x; j < hi; j += kPlaceBlock) {
+    const int64_t f = static_cast<int64_t>(first[j]) - static_cast<int64_t>(j * CAP);
+    m = f < m ? f : m;
+  }
+  m = block_min(m, red);
+  if (threadIdx.x == 0) mins[blockIdx.x] = m;
+}
+
+// base[] continued past the target lines
+struct LineBases {
+  const uint32_t* base;  // targets + 1 entries
+  uint64_t targets;
+  uint32_t end;  // base[targets]
+  uint32_t n, cap;
+  __device__ __forceinline__ uint32_t operator()(uint64_t l) const {
+    if (l <= targets) return base[l];
+    const uint64_t b = end + (l - targets) * cap;
+    return b < n ? static_cast<uint32_t>(b) : n;
+  }
+};
+
+// The leaves whose lines [line0[j], line0[j + 1]) are marked as the source of a run.
+struct LeafMarks {
+  const uint32_t* line0;  // leaves + 1 entries; null: no marks
+  uint32_t leaves;
+  uint8_t* mark;
+  __device__ __forceinline__ void set(uint64_t line) const {
+    if (!line0) return;
+    uint32_t lo = 0, len = leaves + 1;  // lo: entries of line0 that are <= line
+    while (len > 0) {
+      const uint32_t half = len >> 1;
+      if (line0[lo + half] <= line) {
+        lo += half + 1;
+        len -= half + 1;
+      } else {
+        len = half;
+      }
     }
-    for (int64_t l = tp + 1; l <= static_cast<int64_t>(t); ++l) first[l] = static_cast<uint32_t>(i);
+    if (lo >= 1 && lo - 1 < leaves) mark[lo - 1] = 1;
+  }
+};
+
+// How far line l (first key at position b) lies from its first key's target, the smallest
+// target in the line; marks the leaf of a target that a key spills two or more lines from.
+template <class K>
+__device__ __forceinline__ uint32_t line_spill(const K* __restrict__ col, const LinesDev<K>& d, const uint8_t* rp,
+                                               uint64_t l, uint32_t b, const LeafMarks& marks) {
+  const uint64_t t = d.target(col[b], rp);
+  const uint32_t spill = t < l ? static_cast<uint32_t>(l - t) : 0u;
+  if (spill >= 2) marks.set(t);
+  return spill;
+}
+
+// One span's contribution to the placement's totals.  Blocks store theirs and one block
+// adds them up: thousands of atomics on one address cost 10 ns each (215 us of the 430 us
+// that the placement's kernels took with them).
+struct SpanTotals {
+  unsigned long long carry;
+  uint32_t max_spill, pad;
+};
+
+template <class K>
+__global__ __launch_bounds__(kPlaceBlock) void line_base_kernel(const K* __restrict__ col, uint32_t n, LinesDev<K> d,
+                                                                const uint8_t* rp, const uint32_t* __restrict__ first,
+                                                                uint64_t entries, uint64_t span,
+                                                                const int64_t* __restrict__ mins, LeafMarks marks,
+                                                                uint32_t* __restrict__ base,
+                                                                SpanTotals* __restrict__ totals) {
+  constexpr uint32_t CAP = LinesDev<K>::CAP;
+  __shared__ int64_t red[kPlaceBlock / kWave];
+  const uint64_t lo = blockIdx.x * span, hi = lo + span < entries ? lo + span : entries;
+  int64_t run = INT64_MAX;  // the minimum over every earlier line
+  for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kPlaceBlock) run = mins[b] < run ? mins[b] : run;
+  run = block_min(run, red);
+  uint64_t carry = 0;
+  uint32_t worst = 0;
+  for (uint64_t tile = lo; tile < hi; tile += kPlaceTile) {
+    const uint64_t at = tile + static_cast<uint64_t>(threadIdx.x) * kPlaceItems;
+    uint32_t v[kPlaceItems + 1];
+    int64_t m[kPlaceItems];  // running minimum inside the thread
+    int64_t mine = INT64_MAX;
+#pragma unroll
+    for (int k = 0; k <= kPlaceItems; ++k) v[k] = at + k < entries ? first[at + k] : n;
+#pragma unroll
+    for (int k = 0; k < kPlaceItems; ++k) {
+      const int64_t f = static_cast<int64_t>(v[k]) - static_cast<int64_t>((at + k) * CAP);
+      mine = at + k < hi && f < mine ? f : mine;
+      m[k] = mine;
+    }
+    // minimum over the lanes before this one, then over the waves before this one
+    int64_t incl = mine;
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int64_t o = __shfl_up(incl, off, kWave);
+      if (lane() >= off && o < incl) incl = o;
+    }
+    int64_t before = __shfl_up(incl, 1, kWave);
+    if (lane() == 0) before = INT64_MAX;
+    __syncthreads();  // the last step's readers of red[]
+    if (lane() == kWave - 1) red[threadIdx.x / kWave] = incl;
+    __syncthreads();
+    int64_t all = run;
+#pragma unroll
+    for (int w = 0; w < kPlaceBlock / kWave; ++w) {
+      if (w < static_cast<int>(threadIdx.x / kWave)) before = red[w] < before ? red[w] : before;
+      all = red[w] < all ? red[w] : all;
+    }
+    before = run < before ? run : before;
+    run = all;
+#pragma unroll
+    for (int k = 0; k < kPlaceItems; ++k) {
+      if (at + k < hi) {
+        const int64_t mk = m[k] < before ? m[k] : before;
+        const uint32_t b = static_cast<uint32_t>(mk + static_cast<int64_t>((at + k) * CAP));
+        base[at + k] = b;
+        carry += v[k] - b;
+        // only a line behind a full one holds keys of earlier targets; an empty one none
+        if (b < v[k] && at + k + 1 < entries && b < v[k + 1]) {
+          const uint32_t s = line_spill(col, d, rp, at + k, b, marks);
+          worst = s > worst ? s : worst;
+        }
+      }
+    }
+  }
+  carry = wave_sum(carry);
+  worst = wave_max(worst);
+  __shared__ SpanTotals part[kPlaceBlock / kWave];
+  if (lane() == 0) part[threadIdx.x / kWave] = SpanTotals{carry, worst, 0};
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    SpanTotals t = part[0];
+    for (int w = 1; w < kPlaceBlock / kWave; ++w) {
+      t.carry += part[w].carry;
+      t.max_spill = part[w].max_spill > t.max_spill ? part[w].max_spill : t.max_spill;
+    }
+    totals[blockIdx.x] = t;
   }
 }
 
-// Line l holds the keys at positions [base[l], base[l + 1]), after its header.
+// Adds the spans up (block 0) and looks at the lines past the targets, if there are any.
 template <class K>
-__global__ void line_fill_kernel(const K* __restrict__ col, const uint32_t* __restrict__ base, uint64_t lines,
-                                 K* __restrict__ out) {
+__global__ __launch_bounds__(kPlaceBlock) void line_total_kernel(const K* __restrict__ col, uint32_t n, LinesDev<K> d,
+                                                                 const uint8_t* rp, const uint32_t* __restrict__ base,
+                                                                 uint64_t targets, LeafMarks marks,
+                                                                 const SpanTotals* __restrict__ totals, uint32_t spans,
+                                                                 LineStats* st) {
+  constexpr uint32_t CAP = LinesDev<K>::CAP;
+  const LineBases at{base, targets, base[targets], n, CAP};
+  const uint64_t tail = (static_cast<uint64_t>(n - at.end) + CAP - 1) / CAP;
+  uint64_t carry = 0;
+  uint32_t worst = 0;
+  if (blockIdx.x == 0) {
+    for (uint32_t b = threadIdx.x; b < spans; b += kPlaceBlock) {
+      carry += totals[b].carry;
+      worst = totals[b].max_spill > worst ? totals[b].max_spill : worst;
+    }
+    if (threadIdx.x == 0) st->base_end = at.end;
+  }
+  for (uint64_t k = static_cast<uint64_t>(blockIdx.x) * kPlaceBlock + threadIdx.x; k < tail;
+       k += static_cast<uint64_t>(gridDim.x) * kPlaceBlock) {
+    const uint32_t s = line_spill(col, d, rp, targets + k, at(targets + k), marks);
+    worst = s > worst ? s : worst;
+  }
+  carry = wave_sum(carry);
+  worst = wave_max(worst);
+  if (lane() != 0) return;
+  if (carry) atomicAdd(&st->carry, static_cast<unsigned long long>(carry));
+  if (worst) atomicMax(&st->max_spill, worst);
+}
+
+// Line l holds the keys at positions [base(l), base(l + 1)), after its header.
+template <class K>
+__global__ void line_fill_kernel(const K* __restrict__ col, LineBases base, uint64_t lines, K* __restrict__ out) {
   using D = LinesDev<K>;
   const uint64_t slots = lines * D::SLOTS;
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g < slots; g += stride) {
     const uint64_t l = g / D::SLOTS;
     const uint32_t sl = static_cast<uint32_t>(g % D::SLOTS);
-    const uint32_t b = base[l];
-    const uint32_t cnt = base[l + 1] - b;
+    const uint32_t b = base(l);
+    const uint32_t cnt = base(l + 1) - b;
     K v;
     if (sl < D::HDR) {
       const uint64_t hdr = (static_cast<uint64_t>(cnt) << 32) | b;
@@ -536,81 +888,81 @@ struct LinesBuild {
   bool ok = false;
 };
 
-// Places the keys under target model d (d.leaves / d.mult already set; d.lines unused)
-// over `targets` target lines plus whatever tail lines the last full lines push keys into.
-// src_line (optional) receives, per line, the smallest target line among its keys.
-template <class K>
-void place_lines(const gj_index& ix, LinesDev<K> d, const uint8_t* rp, uint64_t targets, LinesBuild& out,
-                 hipStream_t s, std::vector<uint32_t>* src_line = nullptr) {
-  using D = LinesDev<K>;
-  const K* col = static_cast<const K*>(ix.d_col);
-  const uint64_t n = ix.n;
-  dbuf first((targets + 1) * sizeof(uint32_t));
-  {
-    std::vector<uint32_t> init(targets + 1, static_cast<uint32_t>(n));
-    GJ_HIP_CHECK(hipMemcpyAsync(first.p, init.data(), init.size() * 4, hipMemcpyHostToDevice, s));
-    dbuf bad(sizeof(unsigned long long));
-    fill_bytes(bad.p, 0, bad.bytes, s);
-    hipLaunchKernelGGL(line_first_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, col, n, d, rp, targets,
-                       first.as<uint32_t>(), bad.as<unsigned long long>());
+// Working memory of a placement: first | base | span minima | span totals | stats | marks.
+struct Placement {
+  dbuf buf;
+  uint64_t targets = 0;
+  uint32_t *first = nullptr, *base = nullptr;
+  LineStats* stats = nullptr;
+  uint8_t* mark = nullptr;
+  LineStats h{};
+
+  // Places the keys under target model d (d.leaves / d.mult already set; d.lines unused)
+  // over `targets` target lines plus whatever tail lines the last full lines push keys
+  // into, and reads the outcome back.  line0 (optional, `leaves` + 1 entries): mark[j]
+  // is set for the leaves that keys spill two or more lines from.
+  template <class K>
+  void measure(const gj_index& ix, LinesDev<K> d, const uint8_t* rp, uint64_t lines, hipStream_t s,
+               const uint32_t* line0 = nullptr, uint32_t leaves = 0) {
+    constexpr uint32_t CAP = LinesDev<K>::CAP;
+    const K* col = static_cast<const K*>(ix.d_col);
+    const uint64_t n = ix.n, entries = lines + 1;
+    targets = lines;
+    auto up = [](uint64_t b) { return (b + 255) / 256 * 256; };
+    const uint64_t o_base = up(entries * 4), o_min = o_base + up(entries * 4), o_tot = o_min + up(kPlaceBlocks * 8),
+                   o_st = o_tot + up(kPlaceBlocks * sizeof(SpanTotals)), o_mark = o_st + up(sizeof(LineStats));
+    buf.reserve(o_mark + up(line0 ? leaves : 0));
+    uint8_t* p = buf.as<uint8_t>();
+    first = reinterpret_cast<uint32_t*>(p);
+    base = reinterpret_cast<uint32_t*>(p + o_base);
+    stats = reinterpret_cast<LineStats*>(p + o_st);
+    mark = line0 ? p + o_mark : nullptr;
+    int64_t* mins = reinterpret_cast<int64_t*>(p + o_min);
+    SpanTotals* totals = reinterpret_cast<SpanTotals*>(p + o_tot);
+    const LeafMarks marks{line0, leaves, mark};
+    fill_words(first, entries, static_cast<uint32_t>(n), s);
+    fill_bytes(stats, 0, o_mark - o_st + (line0 ? leaves : 0), s);  // and the marks behind them
+    hipLaunchKernelGGL(line_first_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, col, n, d, rp, targets, first,
+                       stats);
     GJ_HIP_CHECK(hipGetLastError());
-    unsigned long long hbad = 0;
-    GJ_HIP_CHECK(hipMemcpyAsync(&hbad, bad.p, sizeof(hbad), hipMemcpyDeviceToHost, s));
-    GJ_HIP_CHECK(hipMemcpyAsync(init.data(), first.p, init.size() * 4, hipMemcpyDeviceToHost, s));
-    GJ_HIP_CHECK(hipStreamSynchronize(s));
-    GJ_REQUIRE(hbad == 0, GJ_ERR_INTERNAL, "learned lines: target model is not monotone");
-    // Greedy placement in key order: line l takes its carried-over keys and its own,
-    // up to CAP; the rest moves on.  base[l] = row id of line l's first key.
-    std::vector<uint32_t> base;
-    base.reserve(targets + 16);
-    uint64_t carry = 0, pos = 0;
-    double sum_line = 0.0, sum_target = 0.0;
-    for (uint64_t l = 0; l < targets; ++l) {
-      const uint64_t c = static_cast<uint64_t>(init[l + 1]) - init[l];
-      const uint64_t avail = carry + c;
-      const uint64_t placed = avail < D::CAP ? avail : D::CAP;
-      carry = avail - placed;
-      base.push_back(static_cast<uint32_t>(pos));
-      pos += placed;
-      sum_line += static_cast<double>(l) * static_cast<double>(placed);
-      sum_target += static_cast<double>(l) * static_cast<double>(c);
-    }
-    for (uint64_t l = targets; carry > 0; ++l) {  // tail lines for what the last full lines push on
-      const uint64_t placed = carry < D::CAP ? carry : D::CAP;
-      base.push_back(static_cast<uint32_t>(pos));
-      pos += placed;
-      carry -= placed;
-      sum_line += static_cast<double>(l) * static_cast<double>(placed);
-    }
-    GJ_REQUIRE(pos == n, GJ_ERR_INTERNAL, "learned lines: placement lost keys");
-    const uint64_t total = base.size();
-    base.push_back(static_cast<uint32_t>(n));
-    // largest spill: the first key of a line has the smallest target in it
-    uint64_t t = 0, max_spill = 0;
-    if (src_line) src_line->assign(total, 0);
-    for (uint64_t l = 0; l < total; ++l) {
-      if (base[l + 1] == base[l]) {
-        if (src_line) (*src_line)[l] = static_cast<uint32_t>(l);
-        continue;
-      }
-      while (t + 1 < targets && init[t + 1] <= base[l]) ++t;
-      max_spill = std::max<uint64_t>(max_spill, l - t);
-      if (src_line) (*src_line)[l] = static_cast<uint32_t>(t);
-    }
-    out.num_lines = total;
-    out.avg_lines = 1.0 + (sum_line - sum_target) / static_cast<double>(n);
-    out.max_lines = static_cast<uint32_t>(std::min<uint64_t>(max_spill + 1, 0xFFFFFFFFull));
-    first.release();
-    dbuf d_base(base.size() * sizeof(uint32_t));
-    GJ_HIP_CHECK(hipMemcpyAsync(d_base.p, base.data(), base.size() * 4, hipMemcpyHostToDevice, s));
-    out.lines.alloc(total * 128);
-    hipLaunchKernelGGL(line_fill_kernel<K>, dim3(grid_for(total * D::SLOTS, 256)), dim3(256), 0, s, col,
-                       d_base.as<const uint32_t>(), total, out.lines.as<K>());
+    const uint64_t span = ceil_div(std::max<uint64_t>(kPlaceTile, ceil_div(entries, kPlaceBlocks)), kPlaceTile) * kPlaceTile;
+    const unsigned blocks = static_cast<unsigned>(ceil_div(entries, span));
+    hipLaunchKernelGGL((line_span_min_kernel<CAP>), dim3(blocks), dim3(kPlaceBlock), 0, s, first, entries, span, mins);
     GJ_HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(line_base_kernel<K>, dim3(blocks), dim3(kPlaceBlock), 0, s, col, static_cast<uint32_t>(n), d, rp,
+                       first, entries, span, mins, marks, base, totals);
+    GJ_HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(line_total_kernel<K>, dim3(64), dim3(kPlaceBlock), 0, s, col, static_cast<uint32_t>(n), d, rp,
+                       base, targets, marks, totals, blocks, stats);
+    GJ_HIP_CHECK(hipGetLastError());
+    GJ_HIP_CHECK(hipMemcpyAsync(&h, stats, sizeof(h), hipMemcpyDeviceToHost, s));
     GJ_HIP_CHECK(hipStreamSynchronize(s));
+    GJ_REQUIRE(h.bad == 0, GJ_ERR_INTERNAL, "learned lines: target model is not monotone");
   }
-  out.ok = true;
-}
+
+  // Writes the lines of the measured placement.
+  template <class K>
+  void emit(const gj_index& ix, LinesBuild& out, hipStream_t s) const {
+    constexpr uint32_t CAP = LinesDev<K>::CAP;
+    const uint64_t n = ix.n;
+    // tail lines: what the last full lines push on, CAP keys at a time
+    const uint64_t rest = n - h.base_end, tail = ceil_div(rest, CAP);
+    double carry = static_cast<double>(h.carry);
+    if (tail > 1)
+      carry += static_cast<double>(tail - 1) * static_cast<double>(rest) -
+               static_cast<double>(CAP) * 0.5 * static_cast<double>(tail - 1) * static_cast<double>(tail);
+    out.num_lines = targets + tail;
+    out.avg_lines = 1.0 + carry / static_cast<double>(n);
+    out.max_lines = h.max_spill + 1;
+    out.lines.alloc(out.num_lines * 128);
+    const LineBases at{base, targets, h.base_end, static_cast<uint32_t>(n), CAP};
+    hipLaunchKernelGGL(line_fill_kernel<K>, dim3(grid_for(out.num_lines * LinesDev<K>::SLOTS, 256)), dim3(256), 0, s,
+                       static_cast<const K*>(ix.d_col), at, out.num_lines, out.lines.as<K>());
+    GJ_HIP_CHECK(hipGetLastError());
+    GJ_HIP_CHECK(hipStreamSynchronize(s));  // the placement's working memory may go
+    out.ok = true;
+  }
+};
 
 // Root-only lines: the key range spread linearly over ceil(n / line_keys) lines.
 template <class K>
@@ -627,7 +979,9 @@ void lines_root_only(const gj_index& ix, uint32_t line_keys, LinesBuild& out, hi
   d.mult = out.mult;
   out.num_leaves = 0;
   out.root = RootModel{};
-  place_lines<K>(ix, d, nullptr, targets, out, s);
+  Placement pl;
+  pl.measure<K>(ix, d, nullptr, targets, s);
+  pl.emit<K>(ix, out, s);
 }
 
 // Two-stage lines: `root` routes keys to 2^bits leaves; each leaf gets lines for its
@@ -641,9 +995,9 @@ void lines_two_stage(const gj_index& ix, const RootModel& root, uint32_t bits, u
   const K kmin = static_cast<K>(ix.min_key);
   Router<K> route{kmin, root, L};
   dbuf start((static_cast<uint64_t>(L) + 1) * sizeof(uint32_t));
-  std::vector<uint32_t> hs(L + 1, static_cast<uint32_t>(n));
+  std::vector<uint32_t> hs(L + 1);
   {
-    GJ_HIP_CHECK(hipMemcpyAsync(start.p, hs.data(), hs.size() * 4, hipMemcpyHostToDevice, s));
+    fill_words(start.as<uint32_t>(), hs.size(), static_cast<uint32_t>(n), s);
     dbuf inv(sizeof(unsigned long long));
     fill_bytes(inv.p, 0, inv.bytes, s);
     hipLaunchKernelGGL(leaf_bounds_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, col, n, route,
@@ -662,7 +1016,9 @@ void lines_two_stage(const gj_index& ix, const RootModel& root, uint32_t bits, u
   // kInflateRounds times.
   constexpr int kInflateRounds = 4;
   constexpr uint32_t kMaxInflate = 16;
-  std::vector<uint32_t> inflate(L, 1), line0(L + 1, 0), src;
+  std::vector<uint32_t> inflate(L, 1), line0(L + 1, 0);
+  std::vector<uint8_t> mark(L);
+  Placement pl;
   dbuf d_line0((static_cast<uint64_t>(L) + 1) * sizeof(uint32_t));
   out.leaves.alloc(sizeof(LineLeaf) * L);
   out.num_leaves = L;
@@ -688,16 +1044,10 @@ void lines_two_stage(const gj_index& ix, const RootModel& root, uint32_t bits, u
     d.num_leaves = L;
     // FP32 rounding can carry a leaf's last keys to floor(p) = its line count, the first
     // line of the next leaf (still monotone); for the last leaf that is target line `lines`
-    place_lines<K>(ix, d, reinterpret_cast<const uint8_t*>(root.params()), lines + 1, out, s, &src);
-    if (out.max_lines <= 2 || round + 1 >= kInflateRounds) break;
-    std::vector<uint8_t> mark(L, 0);
-    for (uint64_t l = 0; l < src.size(); ++l) {
-      if (l - src[l] < 2) continue;
-      // the leaf whose lines hold the source line
-      const uint32_t j = static_cast<uint32_t>(
-          std::upper_bound(line0.begin(), line0.end(), src[l]) - line0.begin() - 1);
-      if (j < L) mark[j] = 1;
-    }
+    pl.measure<K>(ix, d, reinterpret_cast<const uint8_t*>(root.params()), lines + 1, s, d_line0.as<const uint32_t>(), L);
+    if (pl.h.max_spill <= 1 || round + 1 >= kInflateRounds) break;
+    GJ_HIP_CHECK(hipMemcpyAsync(mark.data(), pl.mark, L, hipMemcpyDeviceToHost, s));
+    GJ_HIP_CHECK(hipStreamSynchronize(s));
     bool grew = false;
     for (uint32_t j = 0; j < L; ++j) {
       if (mark[j] && inflate[j] < kMaxInflate) {
@@ -707,10 +1057,10 @@ void lines_two_stage(const gj_index& ix, const RootModel& root, uint32_t bits, u
     }
     if (!grew) break;
   }
+  pl.emit<K>(ix, out, s);
 }
 
-// Adopts a lines build into the index: the column layout's leaves and the B-tree
-// fallback are not needed.
+// Adopts a lines build into the index: the column layout's leaves are not needed.
 void adopt_lines(gj_index& ix, LinesBuild& b) {
   ix.lm_layout = GJ_LAYOUT_LINES;
   ix.lm_lines = std::move(b.lines);
@@ -726,8 +1076,6 @@ void adopt_lines(gj_index& ix, LinesBuild& b) {
   ix.lm_compact = false;
   ix.lm_splits = 0;
   ix.lm_fallback_any = 0;
-  ix.btree_nodes.release();
-  ix.bt = BTreeLayout{};
   ix.stats.layout = GJ_LAYOUT_LINES;
   ix.stats.lines = b.num_lines;
   ix.stats.avg_lines = b.avg_lines;
@@ -762,7 +1110,11 @@ void build_learned(gj_index& ix, hipStream_t s) {
   std::vector<float> mlp_init;  // the MLP root's parameters before training
   ix.stats.root_trained = (ix.kind == GJ_LEARNED_MLP && !(ix.params.learned_flags & GJ_LEARNED_UNTRAINED)) ? 1u : 0u;
 
-  if (ix.kind == GJ_LEARNED_PLR) {
+  // learned_plr's linear root, fitted when the first candidate that routes by it is built
+  bool root_fitted = false;
+  auto fit_root = [&] {
+    if (ix.kind != GJ_LEARNED_PLR || root.segments || root_fitted) return;
+    root_fitted = true;
     const unsigned blocks = grid_for(n, 256, 2048);
     dbuf partial(sizeof(RootFitSums) * blocks);
     hipLaunchKernelGGL(root_sums_kernel<K>, dim3(blocks), dim3(256), 0, s, col, n, kmin, root.inv_range,
@@ -784,8 +1136,8 @@ void build_learned(gj_index& ix, hipStream_t s) {
     if (a < 0) a = 0;
     root.a = static_cast<float>(a);
     root.b = static_cast<float>((t.st - a * t.sx) / c);
-    root.hidden = 0;
-  } else {
+  };
+  if (ix.kind == GJ_LEARNED_MLP) {
     const uint32_t h = ix.params.mlp_hidden;
     GJ_REQUIRE(h == 8 || h == 16 || h == 32 || h == 64, GJ_ERR_INVALID, "mlp_hidden must be 8, 16, 32 or 64");
     const uint32_t np = 3 * h + 1;
@@ -936,8 +1288,10 @@ void build_learned(gj_index& ix, hipStream_t s) {
     const bool linear_root = root.hidden == 0 && root.segments == 0;
     if (linear_root && ix.params.learned_leaf_bits == 0)
       consider([&](LinesBuild& c) { lines_root_only<K>(ix, lk, c, s); });
-    if (!best.ok || best.avg_lines > kGoodLines)
+    if (!best.ok || best.avg_lines > kGoodLines) {
+      fit_root();
       consider([&](LinesBuild& c) { lines_two_stage<K>(ix, root, lbits, lk, c, s); });
+    }
     if (ix.kind == GJ_LEARNED_PLR && linear_root && ix.params.learned_root_segments == 0 &&
         (!best.ok || best.avg_lines > kGoodLines) && n >= 4)
       consider([&](LinesBuild& c) { lines_two_stage<K>(ix, spline_root(2048), lbits, lk, c, s); });
@@ -980,6 +1334,8 @@ void build_learned(gj_index& ix, hipStream_t s) {
   }
   ix.lm_layout = GJ_LAYOUT_COLUMN;
   ix.stats.layout = GJ_LAYOUT_COLUMN;
+  fit_root();
+  build_btree<K>(ix, s);  // the fallback of leaves that no window covers; the lines need none
 
   dbuf last_start, last_fit;  // leaf starts and fits of the last build_leaves
   // routing, leaf fits and calibration under a root; returns the build keys routed to the B-tree
@@ -989,9 +1345,7 @@ void build_learned(gj_index& ix, hipStream_t s) {
     Router<K> route{kmin, root, L};
     dbuf start((static_cast<uint64_t>(L) + 1 + 3) * sizeof(uint32_t));
     {
-      // fill start[] with n
-      std::vector<uint32_t> init(L + 1, static_cast<uint32_t>(n));
-      GJ_HIP_CHECK(hipMemcpyAsync(start.p, init.data(), init.size() * 4, hipMemcpyHostToDevice, s));
+      fill_words(start.as<uint32_t>(), static_cast<uint64_t>(L) + 1, static_cast<uint32_t>(n), s);
       dbuf inv(sizeof(unsigned long long));
       fill_bytes(inv.p, 0, inv.bytes, s);
       hipLaunchKernelGGL(leaf_bounds_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, col, n, route,
@@ -1004,29 +1358,27 @@ void build_learned(gj_index& ix, hipStream_t s) {
     }
     ix.lm_leaves.alloc(sizeof(LeafModel) * L);
     dbuf fit(sizeof(LeafFit) * L);
-    hipLaunchKernelGGL(leaf_fit_kernel<K>, dim3(L), dim3(256), 0, s, col, n, start.as<const uint32_t>(),
-                       start.as<const uint32_t>() + 1, L, ix.lm_leaves.as<LeafModel>(), fit.as<LeafFit>());
-    GJ_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(leaf_error_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, col, n, route,
-                       ix.lm_leaves.as<const LeafModel>(), fit.as<LeafFit>());
-    GJ_HIP_CHECK(hipGetLastError());
     const int64_t max_width = 2 * static_cast<int64_t>(ix.params.learned_max_error) + 2;
-    hipLaunchKernelGGL(leaf_finalize_kernel, dim3(grid_for(L, 256)), dim3(256), 0, s, ix.lm_leaves.as<LeafModel>(),
-                       fit.as<LeafFit>(), L, max_width);
-    GJ_HIP_CHECK(hipGetLastError());
-
-    std::vector<LeafFit> hf(L);
-    GJ_HIP_CHECK(hipMemcpyAsync(hf.data(), fit.p, fit.bytes, hipMemcpyDeviceToHost, s));
-    GJ_HIP_CHECK(hipStreamSynchronize(s));
+    LeafPass pass;
+    LeafStats st = pass.run(col, n, start.as<const uint32_t>(), start.as<const uint32_t>() + 1, L, max_width,
+                            FitLeaf<K>{ix.lm_leaves.as<LeafModel>()}, fit.as<LeafFit>(), s);
+    std::vector<LeafFit> hf;  // read back only if a leaf is too wide
+    if (st.fb_leaves) {
+      hf.resize(L);
+      GJ_HIP_CHECK(hipMemcpyAsync(hf.data(), fit.p, fit.bytes, hipMemcpyDeviceToHost, s));
+      GJ_HIP_CHECK(hipStreamSynchronize(s));
+    }
 
     // split a leaf that is too wide into kSplitWays equal-count sub-leaves, unless its
     // sub-leaves would still hold over 4 average leaves each (then no line fits them
     // either, and the extra separator read would only delay the B-tree)
     const uint64_t split_max = static_cast<uint64_t>(kSplitWays) * 4 * std::max<uint64_t>(1, ceil_div(n, L));
     std::vector<uint32_t> split_id, split_lo, split_hi, sub_lo, sub_hi;
-    for (uint32_t l = 0; l < L; ++l) {
+    for (uint32_t l = 0; l < hf.size(); ++l) {
       const LeafFit& f = hf[l];
       if (f.count == 0 || f.err_hi >= f.err_lo || f.count > split_max) continue;
+      st.fb_leaves -= 1;  // split leaves count through their sub-leaves
+      st.fb_keys -= f.count;
       split_id.push_back(l);
       split_lo.push_back(f.start);
       split_hi.push_back(f.start + f.count);
@@ -1036,7 +1388,6 @@ void build_learned(gj_index& ix, hipStream_t s) {
       }
     }
     const uint32_t J = static_cast<uint32_t>(split_id.size());
-    std::vector<LeafFit> hs;
     ix.lm_splits = J;
     ix.lm_seps.release();
     ix.lm_subs.release();
@@ -1053,67 +1404,40 @@ void build_learned(gj_index& ix, hipStream_t s) {
       hipLaunchKernelGGL(split_sep_kernel<K>, dim3(grid_for(S, 256)), dim3(256), 0, s, col, d_slo.as<const uint32_t>(),
                          d_shi.as<const uint32_t>(), d_lo.as<const uint32_t>(), J, ix.lm_seps.as<uint64_t>());
       GJ_HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(leaf_fit_kernel<K>, dim3(static_cast<unsigned>(S)), dim3(256), 0, s, col, n,
-                         d_slo.as<const uint32_t>(), d_shi.as<const uint32_t>(), static_cast<uint32_t>(S),
-                         ix.lm_subs.as<LeafModel>(), sfit.as<LeafFit>());
-      GJ_HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(split_error_kernel<K>, dim3(J), dim3(256), 0, s, col, d_lo.as<const uint32_t>(),
-                         d_hi.as<const uint32_t>(), ix.lm_seps.as<const uint64_t>(), ix.lm_subs.as<const LeafModel>(),
-                         sfit.as<LeafFit>());
-      GJ_HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(leaf_finalize_kernel, dim3(grid_for(S, 256)), dim3(256), 0, s, ix.lm_subs.as<LeafModel>(),
-                         sfit.as<LeafFit>(), static_cast<uint32_t>(S), max_width);
-      GJ_HIP_CHECK(hipGetLastError());
+      const LeafStats sub = pass.run(col, n, d_slo.as<const uint32_t>(), d_shi.as<const uint32_t>(),
+                                     static_cast<uint32_t>(S), max_width, FitLeaf<K>{ix.lm_subs.as<LeafModel>()},
+                                     sfit.as<LeafFit>(), s);
+      st.fb_leaves += sub.fb_leaves;
+      st.fb_keys += sub.fb_keys;
+      st.wsum += sub.wsum;
+      st.wkeys += sub.wkeys;
+      st.wmax = std::max(st.wmax, sub.wmax);
+      st.err_lo = std::min(st.err_lo, sub.err_lo);
+      st.err_hi = std::max(st.err_hi, sub.err_hi);
       hipLaunchKernelGGL(split_mark_kernel, dim3(grid_for(J, 256)), dim3(256), 0, s, ix.lm_leaves.as<LeafModel>(),
                          d_id.as<const uint32_t>(), J);
       GJ_HIP_CHECK(hipGetLastError());
-      hs.resize(S);
-      GJ_HIP_CHECK(hipMemcpyAsync(hs.data(), sfit.p, sfit.bytes, hipMemcpyDeviceToHost, s));
-      GJ_HIP_CHECK(hipStreamSynchronize(s));
+      GJ_HIP_CHECK(hipStreamSynchronize(s));  // the work lists may go
     }
 
-    // window bounds over the (sub-)leaves that are not routed to the B-tree, and statistics
-    uint64_t fb_leaves = 0, fb_keys = 0, wsum = 0, wkeys = 0;
-    uint32_t wmax = 0;
-    int32_t elo = 0, ehi = 0;
-    std::vector<uint8_t> is_split(L, 0);
-    for (const uint32_t l : split_id) is_split[l] = 1;
-    std::vector<const LeafFit*> live_fits;
-    for (uint32_t l = 0; l < L; ++l)
-      if (!is_split[l]) live_fits.push_back(&hf[l]);  // split leaves count through their sub-leaves
-    for (const auto& f : hs) live_fits.push_back(&f);
-    for (const LeafFit* fp : live_fits) {
-      const LeafFit& f = *fp;
-      if (f.count == 0) continue;
-      if (f.err_hi < f.err_lo) {
-        ++fb_leaves;
-        fb_keys += f.count;
-      } else {
-        const uint32_t w = static_cast<uint32_t>(f.err_hi - f.err_lo + 1);
-        wmax = std::max(wmax, w);
-        wsum += static_cast<uint64_t>(w) * f.count;
-        wkeys += f.count;
-        elo = std::min(elo, f.err_lo);
-        ehi = std::max(ehi, f.err_hi);
-      }
-    }
-    ix.lm_err_lo = elo;
-    ix.lm_err_hi = ehi;
+    // window bounds over the (sub-)leaves that are not routed to the B-tree
+    ix.lm_err_lo = st.err_lo;
+    ix.lm_err_hi = st.err_hi;
     ix.lm_root = root;
     ix.stats.root_segments = root.segments;
     ix.lm_num_leaves = L;
-    ix.lm_fallback_any = fb_leaves ? 1u : 0u;
+    ix.lm_fallback_any = st.fb_leaves ? 1u : 0u;
     ix.stats.leaves = L;
-    ix.stats.fallback_leaves = fb_leaves;
-    ix.stats.fallback_keys = fb_keys;
+    ix.stats.fallback_leaves = st.fb_leaves;
+    ix.stats.fallback_keys = st.fb_keys;
     ix.stats.split_leaves = J;
-    ix.stats.max_window = wmax;
-    ix.stats.avg_window = wkeys ? static_cast<double>(wsum) / static_cast<double>(wkeys) : 0.0;
+    ix.stats.max_window = st.wmax;
+    ix.stats.avg_window = st.wkeys ? static_cast<double>(st.wsum) / static_cast<double>(st.wkeys) : 0.0;
     ix.stats.depth = 2;
     ix.stats.lds_levels = ix.bt.lds_levels;
     last_start = std::move(start);
     last_fit = std::move(fit);
-    return fb_keys;
+    return st.fb_keys;
   };
 
   // compact leaves from the last build's 16-byte leaves; false (index unchanged) when a
@@ -1126,39 +1450,21 @@ void build_learned(gj_index& ix, hipStream_t s) {
     hipLaunchKernelGGL(compact_groups_kernel<K>, dim3(grid_for(G, 256)), dim3(256), 0, s, col, n,
                        last_start.as<const uint32_t>(), G, gshift, groups.as<LeafGroup>());
     GJ_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(compact_convert_kernel, dim3(grid_for(L, 256)), dim3(256), 0, s,
-                       ix.lm_leaves.as<const LeafModel>(), groups.as<const LeafGroup>(), L, gshift,
-                       cl.as<LeafCompact>(), last_fit.as<LeafFit>());
-    GJ_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(compact_error_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, col, n,
-                       Router<K>{kmin, root, L}, cl.as<const LeafCompact>(), groups.as<const LeafGroup>(), gshift,
-                       last_fit.as<LeafFit>());
-    GJ_HIP_CHECK(hipGetLastError());
-    std::vector<LeafFit> hf(L);
-    GJ_HIP_CHECK(hipMemcpyAsync(hf.data(), last_fit.p, last_fit.bytes, hipMemcpyDeviceToHost, s));
-    GJ_HIP_CHECK(hipStreamSynchronize(s));
-    const int64_t max_width = 2 * static_cast<int64_t>(ix.params.learned_max_error) + 2;
-    uint64_t wsum = 0, wkeys = 0;
-    uint32_t wmax = 0;
-    int32_t elo = 0, ehi = 0;
-    for (const LeafFit& f : hf) {
-      if (f.count == 0) continue;
-      const int64_t w = static_cast<int64_t>(f.err_hi) - f.err_lo + 1;
-      if (w > max_width) return false;
-      wmax = std::max(wmax, static_cast<uint32_t>(w));
-      wsum += static_cast<uint64_t>(w) * f.count;
-      wkeys += f.count;
-      elo = std::min(elo, f.err_lo);
-      ehi = std::max(ehi, f.err_hi);
-    }
+    LeafPass pass;
+    const LeafStats st = pass.run(col, n, last_start.as<const uint32_t>(), last_start.as<const uint32_t>() + 1, L,
+                                  2 * static_cast<int64_t>(ix.params.learned_max_error) + 2,
+                                  CompactLeaf<K>{ix.lm_leaves.as<const LeafModel>(), groups.as<const LeafGroup>(),
+                                                 gshift, cl.as<LeafCompact>()},
+                                  last_fit.as<LeafFit>(), s);
+    if (st.fb_leaves) return false;
     ix.lm_leaves = std::move(cl);
     ix.lm_groups = std::move(groups);
     ix.lm_gshift = gshift;
     ix.lm_compact = true;
-    ix.lm_err_lo = elo;
-    ix.lm_err_hi = ehi;
-    ix.stats.max_window = wmax;
-    ix.stats.avg_window = wkeys ? static_cast<double>(wsum) / static_cast<double>(wkeys) : 0.0;
+    ix.lm_err_lo = st.err_lo;
+    ix.lm_err_hi = st.err_hi;
+    ix.stats.max_window = st.wmax;
+    ix.stats.avg_window = st.wkeys ? static_cast<double>(st.wsum) / static_cast<double>(st.wkeys) : 0.0;
     return true;
   };
 
