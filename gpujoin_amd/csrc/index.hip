@@ -87,7 +87,6 @@ BTreeLayout btree_layout(uint64_t n, int key_bytes, uint32_t lds_budget_bytes, u
     if (bytes + L.level_cnt[lvl] * node_bytes > lds_budget_bytes) break;
     bytes += L.level_cnt[lvl] * node_bytes;
     L.lds_levels = lvl + 1;
-    L.lds_nodes = L.level_off[lvl] + L.level_cnt[lvl];
   }
   return L;
 }

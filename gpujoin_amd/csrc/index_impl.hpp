@@ -16,7 +16,6 @@ struct BTreeLayout {
   uint32_t node_bytes = 128;  // bytes per node and per leaf chunk (64, 128 or 256)
   uint32_t levels = 0;      // inner levels
   uint32_t lds_levels = 0;  // top levels staged in LDS
-  uint64_t lds_nodes = 0;
   uint64_t total_nodes = 0;
   uint64_t level_off[kMaxLevels] = {};
   uint64_t level_cnt[kMaxLevels + 1] = {};
@@ -213,7 +212,6 @@ struct gj_index {
     d.nodes = btree_nodes.as<const K>();
     d.levels = bt.levels;
     d.lds_levels = bt.lds_levels;
-    d.lds_nodes = bt.lds_nodes;
     for (int i = 0; i < gj::kMaxLevels; ++i) d.level_off[i] = bt.level_off[i];
     for (int i = 0; i <= gj::kMaxLevels; ++i) d.level_cnt[i] = bt.level_cnt[i];
     return d;

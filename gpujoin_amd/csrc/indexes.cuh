@@ -192,7 +192,11 @@ __device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, ui
 //   * slot s of node i holds the max key of child i*NK + s (key_max past the end),
 //     so the child index is the count of separators below the probe and no
 //     child pointers are stored (the reference stores pointers, src/btree.cuh:58-63);
-//   * levels are stored top first; the top lds_levels levels are staged in LDS.
+//   * levels are stored top first; the lowest level that fits the LDS budget with all
+//     above it is staged in LDS and searched there by each lane for itself: about 6
+//     instructions per halving, where a node's line by quads takes 75.  2^24 probes, the
+//     levels above by quads -> searched: 2^20 u32 keys 229 -> 205 us, 2^20 u64 322 -> 287,
+//     2^22 u64 402 -> 384.
 // ---------------------------------------------------------------------------
 template <class K, int NB = 128>
 struct BTreeDev {
@@ -203,12 +207,27 @@ struct BTreeDev {
   const K* nodes;  // all inner levels, top level first, NK keys per node
   uint32_t levels;
   uint32_t lds_levels;
-  uint64_t lds_nodes;
   uint64_t level_off[kMaxLevels];      // first node of level l (top = 0)
   uint64_t level_cnt[kMaxLevels + 1];  // nodes of level l; level_cnt[levels] = column chunks
 
-  __host__ __device__ size_t lds_bytes() const { return lds_nodes * NB; }
-  __device__ void stage(uint8_t* lds) const { stage_to_lds(lds, nodes, lds_nodes * NB); }
+  // The lowest of the levels that fit the LDS budget is the only one staged: its slots are
+  // the separators of all the nodes below it in key order, so a binary search over them
+  // finds the node that the levels above would lead to.
+  __host__ __device__ size_t lds_bytes() const { return lds_levels ? level_cnt[lds_levels - 1] * NB : 0; }
+  __device__ void stage(uint8_t* lds) const {
+    if (lds_levels) stage_to_lds(lds, nodes + level_off[lds_levels - 1] * NK, lds_bytes());
+  }
+
+  // Separators of the staged level below x, which is x's node in the next level.
+  __device__ __forceinline__ uint32_t top_search(K x, const K* seps) const {
+    uint32_t at = 0;
+    for (uint32_t len = static_cast<uint32_t>(level_cnt[lds_levels - 1]) * NK; len > 1;) {  // kernel-uniform
+      const uint32_t half = len >> 1;
+      at = seps[at + half - 1] < x ? at + half : at;
+      len -= half;
+    }
+    return at + (seps[at] < x ? 1u : 0u);
+  }
 
   __device__ __forceinline__ void descend(uint32_t& node, bool& live, uint32_t c, uint32_t lvl) const {
     const uint64_t child = static_cast<uint64_t>(node) * NK + c;
@@ -221,10 +240,12 @@ struct BTreeDev {
     const QuadProbes<K> q(x);
     bool live = active;
     uint32_t node = 0;  // fewer than 2^32 / NK chunks, hence nodes of any level
-    uint32_t lvl = 0;
-    const K* lds_nodes_p = reinterpret_cast<const K*>(lds);
-    for (; lvl < lds_levels; ++lvl)
-      descend(node, live, quad_count_less<K, NB>(lds_nodes_p + level_off[lvl] * NK, node, q, ql), lvl);
+    if (lds_levels) {
+      node = top_search(x, reinterpret_cast<const K*>(lds));
+      live = live && node < level_cnt[lds_levels];
+      node = live ? node : 0u;
+    }
+    uint32_t lvl = lds_levels;
     for (; lvl < levels; ++lvl)
       descend(node, live, quad_count_less<K, NB>(nodes + level_off[lvl] * NK, node, q, ql), lvl);
     return quad_find_equal<K, NB>(col, n, node, live, x, q, ql);
