@@ -12,8 +12,14 @@ namespace gj {
 // (the reference rounds its loop bound to a warp multiple for the same
 // reason, :235) with 64-bit indices (the reference uses int, which limits it
 // to 2^31 probes).
+//
+// kMinWaves: waves per SIMD that the registers are cut to.  Binary search by lines over u32
+// keys fits 64 registers without a spill (65 by itself: 7 waves; sorted probes over 2^22 keys
+// 201 -> 183 us); over u64 keys the cut spills (505 -> 669 us).
+template <class Dev> constexpr int kMinWaves = 1;
+template <> inline constexpr int kMinWaves<BSearchDev<uint32_t, true>> = 8;
 template <class Dev, class K>
-__global__ __launch_bounds__(256) void lookup_plain_kernel(Dev d, const K* __restrict__ probes, uint64_t m,
+__global__ __launch_bounds__(256, kMinWaves<Dev>) void lookup_plain_kernel(Dev d, const K* __restrict__ probes, uint64_t m,
                                                            uint32_t* __restrict__ out) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   d.stage(lds);

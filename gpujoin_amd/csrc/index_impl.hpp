@@ -97,9 +97,9 @@ struct gj_index {
 
   gj_index_stats stats{};
 
-  template <class K>
-  gj::BSearchDev<K> bsearch_dev() const {
-    gj::BSearchDev<K> d{};
+  template <class K, bool Lines>
+  gj::BSearchDev<K, Lines> bsearch_dev() const {
+    gj::BSearchDev<K, Lines> d{};
     d.col = static_cast<const K*>(d_col);
     d.n = n;
     d.samples = samples.as<const K>();

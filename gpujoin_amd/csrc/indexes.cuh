@@ -20,46 +20,6 @@ namespace gj {
 constexpr int kMaxLevels = 16;
 
 // ---------------------------------------------------------------------------
-// Binary search (binary_search_index, src/indexes.cuh:336-375 with
-// lower_bound, src/search.cuh:26-41).  One probe per lane.  The column is
-// cut into 2^sample_bits equal buckets; the max key of every bucket sits in
-// LDS, so the first sample_bits steps of the search never leave the CU.  The
-// rest is a branch-free lower_bound inside the bucket, then an equality check.
-// ---------------------------------------------------------------------------
-template <class K>
-struct BSearchDev {
-  const K* col;
-  uint64_t n;
-  const K* samples;  // 2^sample_bits bucket maxima (key_max for empty buckets)
-  uint64_t step;     // keys per bucket
-  uint32_t sample_bits;
-
-  __host__ __device__ size_t lds_bytes() const { return sizeof(K) << sample_bits; }
-  __device__ void stage(uint8_t* lds) const { stage_to_lds(lds, samples, lds_bytes()); }
-
-  __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
-    const K* s = reinterpret_cast<const K*>(lds);
-    const uint32_t nb = 1u << sample_bits;
-    uint32_t b = 0;
-    for (uint32_t h = nb >> 1; h > 0; h >>= 1) b = (s[b + h - 1] < x) ? b + h : b;
-    b += (s[b] < x) ? 1u : 0u;
-    if (!active || b >= nb) return kNotFound;
-    const uint64_t lo = static_cast<uint64_t>(b) * step;
-    if (lo >= n) return kNotFound;
-    const uint64_t hi = (lo + step < n) ? lo + step : n;
-    const K* base = col + lo;
-    uint64_t len = hi - lo;
-    while (len > 1) {
-      const uint64_t half = len >> 1;
-      base = (base[half] < x) ? base + half : base;
-      len -= half;
-    }
-    const uint64_t p = static_cast<uint64_t>(base - col) + ((base[0] < x) ? 1u : 0u);
-    return (p < hi && col[p] == x) ? static_cast<uint32_t>(p) : kNotFound;
-  }
-};
-
-// ---------------------------------------------------------------------------
 // Cooperative search of NB-byte sorted lines (tree nodes, column lines, key lines)
 // by quads.  Each lane owns one probe; a quad serves its four probes in four rounds:
 // in round r its lanes fetch the line of lane r's probe, a quarter each, and each lane
@@ -181,6 +141,148 @@ __device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, ui
   if (tail && live) below = tail_below(col, n, at, x, eq);
   return (live && eq) ? static_cast<uint32_t>(at + below) : kNotFound;
 }
+
+// ---------------------------------------------------------------------------
+// Binary search (binary_search_index, src/indexes.cuh:336-375 with
+// lower_bound, src/search.cuh:26-41).  One probe per lane.  The column is
+// cut into 2^sample_bits equal buckets; the max key of every bucket sits in
+// LDS, so the first sample_bits steps of the search never leave the CU.  Inside the
+// bucket, quads read whole 128-byte lines: the first two are interpolated between the
+// nearest keys known on either side (the bucket's bounds, then the first line's own edge),
+// the third is the second's neighbour, and what is still open then (keys that crowd in
+// their bucket) halves the rest of its range key by key.  The column may hold equal keys;
+// the answer is the first of them, so a line that begins with the probe's key is a
+// candidate and the search goes on to the left.
+//
+// What bounds it: fabric lines (about 52 G/s).  Halving alone touches log2(bucket bytes /
+// 128) + 1 lines per probe, one dependent load each; in a bucket of evenly spread keys the
+// first guess is off by sqrt(bucket) / 3 keys on average and the second finds the line.
+// It stays for buckets of at most kHalve keys (Lines = false: two or three loads of a line
+// that is in reach anyway: 2^24 probes of 2^12 u32 keys 118 us, by quads 170), and for waves whose
+// probes all lie in about one bucket, whose lanes share their loads (sorted probes over
+// 2^22 u64 keys 216 us, by quads 402).
+// 2^24 uniform probes, halving alone -> by lines, us: 2^16 u64 keys 522 -> 220, 2^20 1032 ->
+// 307, 2^22 2357 -> 505, 2^24 3560 -> 667; u32 2^22 1897 -> 329; behind the blockwise sort,
+// 2^22 u64 1261 -> 829.
+// ---------------------------------------------------------------------------
+template <class K, bool Lines = true>
+struct BSearchDev {
+  using L = QuadLine<K, 128>;
+  static constexpr uint32_t LK = L::kKeys;
+  static constexpr int kGuesses = 2;  // interpolated lines, then one neighbour
+  static constexpr uint32_t kHalve = 8;
+  const K* col;
+  uint64_t n;
+  const K* samples;  // 2^sample_bits bucket maxima (key_max for empty buckets)
+  uint64_t step;     // keys per bucket
+  uint32_t sample_bits;
+
+  __host__ __device__ size_t lds_bytes() const { return sizeof(K) << sample_bits; }
+  __device__ void stage(uint8_t* lds) const { stage_to_lds(lds, samples, lds_bytes()); }
+
+  // Where x would sit if the keys between klo (at position plo) and khi (at phi) were
+  // evenly spread; any error only costs lines.
+  __device__ __forceinline__ static uint32_t guess(K x, K klo, K khi, uint32_t plo, uint32_t phi) {
+    const float f = static_cast<float>(x - klo) * __builtin_amdgcn_rcpf(static_cast<float>(khi - klo));
+    return plo + static_cast<uint32_t>(fminf(fmaxf(f, 0.0f), 1.0f) * static_cast<float>(phi - plo));
+  }
+
+  __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
+    const K* s = reinterpret_cast<const K*>(lds);
+    const uint32_t nb = 1u << sample_bits;
+    uint32_t b = 0;
+    for (uint32_t h = nb >> 1; h > 0; h >>= 1) b = (s[b + h - 1] < x) ? b + h : b;
+    b += (s[b] < x) ? 1u : 0u;
+    const uint64_t lo = static_cast<uint64_t>(b) * step;
+    if constexpr (!Lines) {
+      if (!active || b >= nb || lo >= n) return kNotFound;
+      const uint64_t hi = (lo + step < n) ? lo + step : n;
+      return halve(x, lo, hi - lo, hi);
+    } else {
+      bool open = active && b < nb && lo < n;
+      // x's position is in [first, last], or last + 1 where found holds it already
+      uint32_t first = open ? static_cast<uint32_t>(lo) : 0u;
+      uint32_t last = open ? static_cast<uint32_t>((lo + step < n ? lo + step : n) - 1) : 0u;
+      uint32_t found = kNotFound;
+      const uint32_t b0 = __builtin_amdgcn_readfirstlane(b);
+      if (ballot(open && (b > b0 + 1 || b + 1 < b0)) != 0)  // wave-uniform
+        narrow(x, b > 0 ? s[b - 1] : col[0], s[b < nb ? b : nb - 1], b > 0, open, first, last, found);
+      if (open) {
+        const uint32_t r = halve(x, first, static_cast<uint64_t>(last - first) + 1, static_cast<uint64_t>(last) + 1);
+        found = r != kNotFound ? r : found;
+      }
+      return found;
+    }
+  }
+
+  // Branch-free lower_bound over len keys from lo on; the row id if the key before hi is x.
+  __device__ __forceinline__ uint32_t halve(K x, uint64_t lo, uint64_t len, uint64_t hi) const {
+    const K* base = col + lo;
+    while (len > 1) {
+      const uint64_t half = len >> 1;
+      base = (base[half] < x) ? base + half : base;
+      len -= half;
+    }
+    const uint64_t p = static_cast<uint64_t>(base - col) + ((base[0] < x) ? 1u : 0u);
+    return (p < hi && col[p] == x) ? static_cast<uint32_t>(p) : kNotFound;
+  }
+
+  // Lines of the bucket [first, last] by quads.  klo, khi: the keys before the bucket (the
+  // column's first key for the first bucket) and at its end, klo < x <= khi.
+  __device__ __forceinline__ void narrow(K x, K klo, K khi, bool inner, bool& open, uint32_t& first, uint32_t& last,
+                                         uint32_t& found) const {
+    const int ql = lane() & (kQuad - 1);
+    const QuadProbes<K> q(x);
+    const K* lane_base = col + ql * L::kLaneKeys;
+    const uint32_t whole = static_cast<uint32_t>(n / LK);  // whole lines of the column
+    uint32_t plo = inner && first > 0 ? first - 1 : 0u, phi = last;
+    open = open && klo <= x;
+    uint32_t line_lo = first / LK, line_hi = last / LK;
+    uint32_t line = guess(x, klo, khi, plo, phi) / LK;
+    line = line < line_lo ? line_lo : (line > line_hi ? line_hi : line);
+    for (int t = 1; t <= kGuesses + 1 && ballot(open) != 0; ++t) {  // wave-uniform
+      const bool tail = open && line >= whole;  // the column's partial last line
+      const uint32_t rounds = quad_or(open && !tail ? 1u << ql : 0u);
+      L ln[kQuad];
+      quad_rounds([&](auto r) { ln[r].any(); });
+      quad_rounds([&](auto r) {
+        const uint32_t l = quad_bcast<r>(line);
+        if ((rounds >> r) & 1u) ln[r].load(lane_base, l);
+      });
+      uint32_t below = quad_below(ln, q, ql);
+      bool eq = quad_holds(ln, q, ql);
+      if (tail) below = tail_below(col, n, static_cast<uint64_t>(line) * LK, x, eq);
+      if (open) {
+        const uint32_t base = line * LK;
+        const bool right = !tail && below == LK;  // every key of the line is below x
+        if (right) {
+          open = line < line_hi;
+          line_lo = line + 1;
+        } else {
+          found = eq ? base + below : found;
+          open = below == 0 && line > line_lo;
+          line_hi = line - 1;
+        }
+        if (open) {
+          line = right ? line_lo : line_hi;
+          if (t < kGuesses) {  // wave-uniform
+            const uint32_t at = right ? base + LK - 1 : base;  // the edge of the line on x's side
+            const K edge = col[at];
+            klo = right ? edge : klo;
+            khi = right ? khi : edge;
+            plo = right ? at : plo;
+            phi = right ? phi : at;
+            line = guess(x, klo, khi, plo, phi) / LK;
+            line = line < line_lo ? line_lo : (line > line_hi ? line_hi : line);
+          }
+        }
+      }
+    }
+    const uint32_t a = line_lo * LK, z = line_hi * LK + LK - 1;
+    first = a > first ? a : first;
+    last = z < last ? z : last;
+  }
+};
 
 // ---------------------------------------------------------------------------
 // B+-tree, re-laid out for CDNA4.  Keeps the reference's clustered-index

@@ -111,7 +111,12 @@ template <class K> void build_extended(gj_index& ix, hipStream_t s);
 template <class K, class F>
 void with_index_dev(const gj_index& ix, F&& f) {
   switch (ix.kind) {
-    case GJ_BINARY_SEARCH: f(ix.bsearch_dev<K>()); return;
+    case GJ_BINARY_SEARCH:
+      if (ix.sample_step > BSearchDev<K>::kHalve)
+        f(ix.bsearch_dev<K, true>());
+      else
+        f(ix.bsearch_dev<K, false>());
+      return;
     case GJ_BTREE:
       if (ix.bt.node_bytes == 64)
         f(ix.btree_dev<K, 64>());
