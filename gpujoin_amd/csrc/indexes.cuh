@@ -6,6 +6,9 @@
 //   size_t   lds_bytes() const                      bytes of LDS the lookup wants resident
 //   void     stage(uint8_t* lds) const              block-cooperative fill of that LDS (no barrier)
 //   uint32_t lookup(K x, bool active, const uint8_t* lds) const
+//   uint32_t coarse(K x, const uint8_t* lds) const  roughly where x lies, from what needs no memory
+//                                                   read: a number that ascends with x
+//   uint32_t coarse_bins() const                    above every such number
 // lookup() must be called by all 64 lanes of a wave together (like the
 // reference's whole-warp cooperative_lookup, src/btree.cuh:598-605,
 // src/harmonia.cuh:740-745); inactive lanes pass active = false and get
@@ -180,6 +183,15 @@ struct BSearchDev {
   __host__ __device__ size_t lds_bytes() const { return sizeof(K) << sample_bits; }
   __device__ void stage(uint8_t* lds) const { stage_to_lds(lds, samples, lds_bytes()); }
 
+  // the bucket
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t* lds) const {
+    const K* s = reinterpret_cast<const K*>(lds);
+    uint32_t b = 0;
+    for (uint32_t h = (1u << sample_bits) >> 1; h > 0; h >>= 1) b = (s[b + h - 1] < x) ? b + h : b;
+    return b + (s[b] < x ? 1u : 0u);
+  }
+  __host__ __device__ uint32_t coarse_bins() const { return (1u << sample_bits) + 1; }
+
   // Where x would sit if the keys between klo (at position plo) and khi (at phi) were
   // evenly spread; any error only costs lines.
   __device__ __forceinline__ static uint32_t guess(K x, K klo, K khi, uint32_t plo, uint32_t phi) {
@@ -189,10 +201,7 @@ struct BSearchDev {
 
   __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
     const K* s = reinterpret_cast<const K*>(lds);
-    const uint32_t nb = 1u << sample_bits;
-    uint32_t b = 0;
-    for (uint32_t h = nb >> 1; h > 0; h >>= 1) b = (s[b + h - 1] < x) ? b + h : b;
-    b += (s[b] < x) ? 1u : 0u;
+    const uint32_t nb = 1u << sample_bits, b = coarse(x, lds);
     const uint64_t lo = static_cast<uint64_t>(b) * step;
     if constexpr (!Lines) {
       if (!active || b >= nb || lo >= n) return kNotFound;
@@ -331,6 +340,14 @@ struct BTreeDev {
     return at + (seps[at] < x ? 1u : 0u);
   }
 
+  // the node below the staged level
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t* lds) const {
+    return lds_levels ? top_search(x, reinterpret_cast<const K*>(lds)) : 0u;
+  }
+  __host__ __device__ uint32_t coarse_bins() const {
+    return lds_levels ? static_cast<uint32_t>(level_cnt[lds_levels - 1]) * NK + 1 : 1u;
+  }
+
   __device__ __forceinline__ void descend(uint32_t& node, bool& live, uint32_t c, uint32_t lvl) const {
     const uint64_t child = static_cast<uint64_t>(node) * NK + c;
     live = live && (c < static_cast<uint32_t>(NK)) && (child < level_cnt[lvl + 1]);
@@ -359,6 +376,10 @@ template <class K>
 struct NoOpDev {
   __host__ __device__ size_t lds_bytes() const { return 0; }
   __device__ void stage(uint8_t*) const {}
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t*) const {
+    return static_cast<uint32_t>(x >> (8 * sizeof(K) - 11));
+  }
+  __host__ __device__ uint32_t coarse_bins() const { return 1u << 11; }
   __device__ __forceinline__ uint32_t lookup(K, bool, const uint8_t*) const { return kNotFound; }
 };
 

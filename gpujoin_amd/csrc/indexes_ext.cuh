@@ -76,6 +76,22 @@ struct HarmoniaDev {
     if (lds_nodes) stage_to_lds(lds, keys, lds_bytes());
   }
 
+  // keys of the lowest staged level below x
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t* lds) const {
+    if (lds_levels == 0) return 0;
+    const K* s = reinterpret_cast<const K*>(lds) + first[lds_levels - 1] * MK;
+    uint32_t at = 0;
+    for (uint32_t len = coarse_bins() - 1; len > 1;) {  // kernel-uniform
+      const uint32_t half = len >> 1;
+      at = s[at + half - 1] < x ? at + half : at;
+      len -= half;
+    }
+    return at + (s[at] < x ? 1u : 0u);
+  }
+  __host__ __device__ uint32_t coarse_bins() const {
+    return lds_levels ? static_cast<uint32_t>(lds_nodes - first[lds_levels - 1]) * MK + 1 : 1u;
+  }
+
   // Count of node keys below each lane's probe (and whether the key at that
   // position equals the probe), for the G probes of the lane's group.  (Fetching each
   // round's probe and offset from its lane where used, as the B-tree's search does, takes
@@ -265,6 +281,13 @@ struct RadixSplineDev {
   __device__ void stage(uint8_t* lds) const {
     if constexpr (Lds) stage_to_lds(lds, radix, lds_bytes());
   }
+
+  // the radix prefix
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t*) const {
+    const K c = x < min_key ? min_key : (x > max_key ? max_key : x);
+    return static_cast<uint32_t>(static_cast<uint64_t>(c - min_key) >> shift_bits);
+  }
+  __host__ __device__ uint32_t coarse_bins() const { return radix_count; }
 
   // tab: the radix table (LDS during lookups, global memory at build)
   __device__ __forceinline__ double estimate(K x, const uint32_t* tab) const {
@@ -491,6 +514,10 @@ struct LearnedDev {
   __device__ __forceinline__ uint32_t route(K x, const uint8_t* lds) const {
     return route_leaf<K>(x, lds + root_offset(), root, min_key, num_leaves);
   }
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t* lds) const {  // the leaf
+    return route(x < min_key ? min_key : (x > max_key ? max_key : x), lds);
+  }
+  __host__ __device__ uint32_t coarse_bins() const { return num_leaves; }
 
   __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
     bool use_tree = false, split = false;
@@ -561,6 +588,10 @@ struct LearnedCompactDev {
     if (root.bytes()) stage_to_lds(lds, root.params(), root.bytes());
     stage_to_lds(lds + group_offset(), groups, static_cast<size_t>(num_groups) * sizeof(LeafGroup));
   }
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t* lds) const {  // the leaf
+    return route_leaf<K>(x < min_key ? min_key : (x > max_key ? max_key : x), lds, root, min_key, num_leaves);
+  }
+  __host__ __device__ uint32_t coarse_bins() const { return num_leaves; }
 
   __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
     uint64_t lo = 0, hi = 0, pred = 0;
@@ -636,6 +667,15 @@ struct LinesDev {
   __host__ __device__ size_t lds_bytes() const { return leaves ? root.bytes() : 0; }
   __device__ void stage(uint8_t* lds) const {
     if (lds_bytes()) stage_to_lds(lds, root.params(), root.bytes());
+  }
+
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t* lds) const {  // the leaf, or the line
+    const K c = x < min_key ? min_key : (x > max_key ? max_key : x);
+    if (leaves) return route_leaf<K>(c, lds, root, min_key, num_leaves);
+    return static_cast<uint32_t>(__umul64hi(static_cast<uint64_t>(c - min_key), mult));
+  }
+  __host__ __device__ uint32_t coarse_bins() const {
+    return leaves ? num_leaves : static_cast<uint32_t>(num_lines);
   }
 
   // rp: the root's parameters (LDS during lookups, global memory at build)
@@ -732,6 +772,12 @@ struct HashDev {
 
   __host__ __device__ size_t lds_bytes() const { return 0; }
   __device__ void stage(uint8_t*) const {}
+  // the home slot's part of the table, whose order is the hashes', not the keys'
+  __device__ __forceinline__ uint32_t coarse(K x, const uint8_t*) const {
+    const int bits = 64 - __clzll(static_cast<long long>(mask));
+    return static_cast<uint32_t>((key_hash<K>(static_cast<uint64_t>(x)) & mask) >> (bits > 11 ? bits - 11 : 0));
+  }
+  __host__ __device__ uint32_t coarse_bins() const { return 1u << 11; }
 
   __device__ __forceinline__ uint32_t lookup_entries(uint64_t k, bool live) const {
     if (!live) return kNotFound;

@@ -92,14 +92,17 @@ template <class Dev, class K>
 void launch_bws(const Dev& d, const K* probes, uint64_t m, uint32_t* out, const gj_lookup_params& p, hipStream_t s,
                 int cu) {
   if (m == 0) return;
-  const unsigned block = lookup_block(p);
-  const size_t lds = (d.lds_bytes() + 15) / 16 * 16 + kBwsTile * (sizeof(K) + sizeof(uint32_t));
+  (void)lookup_block(p);  // a tile is shared by kBwsBlock threads, whatever valid block size is asked for
+  const size_t lds = (d.lds_bytes() + 15) / 16 * 16 + kBwsTile * (sizeof(K) + sizeof(uint16_t)) +
+                     kBwsBins * sizeof(uint16_t) + kBwsBlock / kWave * sizeof(uint32_t);
+  uint32_t shift = 0;  // bins to at most kBwsBins
+  while (((d.coarse_bins() - 1) >> shift) >= kBwsBins) ++shift;
   const void* fn = reinterpret_cast<const void*>(&lookup_bws_kernel<Dev, K, kBwsTile>);
   const uint64_t blocks =
       p.grid_blocks ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(m, kBwsTile)))
-                    : cover_blocks(m, kBwsTile, 0, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
-  hipLaunchKernelGGL((lookup_bws_kernel<Dev, K, kBwsTile>), dim3(static_cast<unsigned>(blocks)), dim3(block), lds, s,
-                     d, probes, m, out);
+                    : cover_blocks(m, kBwsTile, 0, static_cast<uint64_t>(blocks_per_cu(fn, kBwsBlock, lds)) * cu);
+  hipLaunchKernelGGL((lookup_bws_kernel<Dev, K, kBwsTile>), dim3(static_cast<unsigned>(blocks)), dim3(kBwsBlock), lds, s,
+                     d, probes, m, shift, out);
   GJ_HIP_CHECK(hipGetLastError());
 }
 
