@@ -15,9 +15,12 @@ namespace gj {
 //
 // kMinWaves: waves per SIMD that the registers are cut to.  Binary search by lines over u32
 // keys fits 64 registers without a spill (65 by itself: 7 waves; sorted probes over 2^22 keys
-// 201 -> 183 us); over u64 keys the cut spills (505 -> 669 us).
+// 201 -> 183 us), the learned column layout over u32 keys too (2^20 keys: 2^24 uniform
+// probes 218 -> 215 us, sorted 148 -> 138); over u64 keys the cut spills (505 -> 669 and
+// 256 -> 303 us), as it does for RadixSpline and Harmonia.
 template <class Dev> constexpr int kMinWaves = 1;
 template <> inline constexpr int kMinWaves<BSearchDev<uint32_t, true>> = 8;
+template <> inline constexpr int kMinWaves<LearnedDev<uint32_t, kLeafNoFallback>> = 8;
 template <class Dev, class K>
 __global__ __launch_bounds__(256, kMinWaves<Dev>) void lookup_plain_kernel(Dev d, const K* __restrict__ probes, uint64_t m,
                                                            uint32_t* __restrict__ out) {
