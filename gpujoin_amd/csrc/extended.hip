@@ -133,11 +133,11 @@ void build_harmonia(gj_index& ix, hipStream_t s) {
 // until it does (the FP64 interpolation can round across the exact bound).
 // ---------------------------------------------------------------------------
 template <class K>
-__global__ void rs_check_kernel(RadixSplineDev<K, false> d, unsigned long long* bad) {
+__global__ void rs_check_kernel(RadixSplineDev<K, kRsRadix> d, unsigned long long* bad) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   unsigned long long cnt = 0;
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < d.n; i += stride) {
-    uint64_t lo, hi;
+    uint32_t lo, hi;
     d.window(d.estimate(d.col[i], d.radix), lo, hi);
     cnt += (i < lo || i >= hi) ? 1ull : 0ull;
   }
@@ -153,6 +153,21 @@ std::vector<uint8_t> host_column(const gj_index& ix, hipStream_t s) {
     GJ_HIP_CHECK(hipStreamSynchronize(s));
   }
   return h;
+}
+
+// Whether a sample of the knots beats the radix table: its halvings over a group of knots
+// against the table's, averaged over the keys, and the table's own read (two steps: both
+// sides measured at kRsSamples).  Keys whose segment begins under another prefix are spread over
+// prefixes with a knot or none.
+bool rs_sample_pays(const RadixSplineHost& rs) {
+  double steps = 0.0;
+  for (size_t i = 1; i < rs.knot_x.size(); ++i) {
+    const uint64_t p = (rs.knot_x[i - 1] - rs.min_key) >> rs.shift_bits, q = (rs.knot_x[i] - rs.min_key) >> rs.shift_bits;
+    const double halvings = p == q ? std::log2(1.0 + rs.radix[p + 1] - rs.radix[p]) : 0.5;
+    steps += (rs.knot_y[i] - rs.knot_y[i - 1]) * halvings;
+  }
+  steps /= std::max(1.0, rs.knot_y.back());
+  return std::log2(static_cast<double>(rs.knot_x.size()) / kRsSampleCount + 1.0) + 2.0 < steps;
 }
 
 template <class K>
@@ -172,17 +187,28 @@ void build_rs(gj_index& ix, hipStream_t s) {
   GJ_HIP_CHECK(hipMemcpyAsync(ix.rs_radix.p, rs.radix.data(), ix.rs_radix.bytes, hipMemcpyHostToDevice, s));
   // staged in LDS when the table has at most 2^rs_lds_bits + 2 entries (2^14: 64 KiB, a
   // workgroup's LDS)
-  ix.rs_lds = rs.radix.size() <= (1ull << std::min<uint32_t>(ix.params.rs_lds_bits, 14)) + 2;
-  ix.stats.lds_levels = ix.rs_lds ? 1 : 0;
+  ix.rs_mode = rs.radix.size() <= (1ull << std::min<uint32_t>(ix.params.rs_lds_bits, 14)) + 2 ? kRsRadixLds : kRsRadix;
+  ix.stats.lds_levels = ix.rs_mode == kRsRadixLds ? 1 : 0;
   std::vector<RsKnot> kn(rs.knot_x.size());
   for (size_t i = 0; i < kn.size(); ++i) kn[i] = RsKnot{static_cast<uint64_t>(rs.knot_x[i]), rs.knot_y[i]};
   ix.rs_knots.alloc(kn.size() * sizeof(RsKnot));
   GJ_HIP_CHECK(hipMemcpyAsync(ix.rs_knots.p, kn.data(), ix.rs_knots.bytes, hipMemcpyHostToDevice, s));
+  // (not where the structures go to host memory, from where every workgroup would stage them)
+  if (ix.rs_mode == kRsRadix && ix.params.placement != GJ_PLACE_HOST && rs_sample_pays(rs)) {
+    ix.rs_mode = kRsSamples;
+    ix.rs_group = static_cast<uint32_t>(ceil_div(kn.size(), kRsSampleCount));
+    std::vector<K> smp(kRsSampleCount, static_cast<K>(~static_cast<K>(0)));
+    for (size_t g = 0; g * ix.rs_group < kn.size(); ++g)
+      smp[g] = static_cast<K>(kn[std::min<size_t>((g + 1) * ix.rs_group, kn.size()) - 1].x);
+    ix.samples.alloc(smp.size() * sizeof(K));
+    GJ_HIP_CHECK(hipMemcpyAsync(ix.samples.p, smp.data(), ix.samples.bytes, hipMemcpyHostToDevice, s));
+    GJ_HIP_CHECK(hipStreamSynchronize(s));
+  }
   ix.rs_err = ix.params.rs_max_error;
   dbuf bad(sizeof(unsigned long long));
   for (int attempt = 0; attempt < 40; ++attempt) {
     fill_bytes(bad.p, 0, bad.bytes, s);
-    hipLaunchKernelGGL(rs_check_kernel<K>, dim3(grid_for(ix.n, 256, 8192)), dim3(256), 0, s, ix.rs_dev<K, false>(),
+    hipLaunchKernelGGL(rs_check_kernel<K>, dim3(grid_for(ix.n, 256, 8192)), dim3(256), 0, s, ix.rs_dev<K, kRsRadix>(),
                        bad.as<unsigned long long>());
     GJ_HIP_CHECK(hipGetLastError());
     unsigned long long h = 0;

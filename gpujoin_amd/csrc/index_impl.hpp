@@ -37,7 +37,7 @@ struct gj_index {
   int cu = 0;
   bool col_in_host = false;  // the column is page-locked host memory (read over the host link)
 
-  // binary search: bucket maxima staged in LDS
+  // bucket maxima staged in LDS (binary search), or a sample of the knots (RadixSpline)
   gj::dbuf samples;
   uint32_t sample_bits = 0;
   uint64_t sample_step = 0;
@@ -55,7 +55,8 @@ struct gj_index {
   // RadixSpline
   gj::dbuf rs_radix, rs_knots;
   uint32_t rs_shift = 0, rs_err = 0;
-  bool rs_lds = false;  // the radix table is staged in LDS
+  int rs_mode = 0;            // how lookups find the knots (kRsRadix, ...)
+  uint32_t rs_group = 0;      // knots per sample (kRsSamples; the samples are in `samples`)
   uint64_t rs_points = 0;
 
   // learned two-stage models (B-tree above is their fallback)
@@ -122,9 +123,9 @@ struct gj_index {
     return d;
   }
 
-  template <class K, bool Lds>
-  gj::RadixSplineDev<K, Lds> rs_dev() const {
-    gj::RadixSplineDev<K, Lds> d{};
+  template <class K, int Mode>
+  gj::RadixSplineDev<K, Mode> rs_dev() const {
+    gj::RadixSplineDev<K, Mode> d{};
     d.col = static_cast<const K*>(d_col);
     d.n = n;
     d.radix = rs_radix.as<const uint32_t>();
@@ -134,6 +135,9 @@ struct gj_index {
     d.max_key = static_cast<K>(max_key);
     d.shift_bits = rs_shift;
     d.err = rs_err;
+    d.samples = samples.as<const K>();
+    d.group = rs_group;
+    d.num_knots = static_cast<uint32_t>(rs_points);
     return d;
   }
 

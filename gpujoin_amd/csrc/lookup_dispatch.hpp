@@ -142,10 +142,12 @@ void with_index_dev(const gj_index& ix, F&& f) {
       }
       throw error(GJ_ERR_INVALID, "unsupported harmonia_group_lanes");
     case GJ_RADIX_SPLINE:
-      if (ix.rs_lds)
-        f(ix.rs_dev<K, true>());
+      if (ix.rs_mode == kRsRadixLds)
+        f(ix.rs_dev<K, kRsRadixLds>());
+      else if (ix.rs_mode == kRsSamples)
+        f(ix.rs_dev<K, kRsSamples>());
       else
-        f(ix.rs_dev<K, false>());
+        f(ix.rs_dev<K, kRsRadix>());
       return;
     case GJ_LEARNED_PLR:
     case GJ_LEARNED_MLP:
