@@ -36,23 +36,6 @@ __device__ __forceinline__ T shfl(T v, int src_lane) {
 
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 
-// Bits of `mask` belonging to the G-lane group that starts at lane gbase.
-template <int G>
-__device__ __forceinline__ uint32_t group_bits(uint64_t mask, int gbase) {
-  if constexpr (G == 64) {
-    return 0;  // not used with G == 64 (see group_popc / group_ffs)
-  } else {
-    return static_cast<uint32_t>((mask >> gbase) & ((1ull << G) - 1ull));
-  }
-}
-template <int G>
-__device__ __forceinline__ int group_popc(uint64_t mask, int gbase) {
-  if constexpr (G == 64) {
-    return __popcll(mask);
-  } else {
-    return __popc(group_bits<G>(mask, gbase));
-  }
-}
 // Quads: groups of four neighbouring lanes.  A quad-permute rides on an ordinary VALU
 // instruction (DPP), where a cross-lane read through the LDS crossbar (shfl) is an LDS
 // operation with its latency and a shared port.

@@ -109,9 +109,9 @@ struct gj_index {
     return d;
   }
 
-  template <class K, int G>
-  gj::HarmoniaDev<K, G> harmonia_dev() const {
-    gj::HarmoniaDev<K, G> d{};
+  template <class K>
+  gj::HarmoniaDev<K> harmonia_dev() const {
+    gj::HarmoniaDev<K> d{};
     d.col = static_cast<const K*>(d_col);
     d.n = n;
     d.keys = hm_keys.as<const K>();

@@ -7,37 +7,6 @@
 
 namespace gj {
 
-// KPL consecutive keys loaded by one lane (4, 8 or 16 bytes).
-template <class K, int KPL>
-struct LaneKeys {
-  K k[KPL];
-};
-template <class K, int KPL>
-__device__ __forceinline__ LaneKeys<K, KPL> load_lane_keys(const K* p) {
-  constexpr int B = KPL * static_cast<int>(sizeof(K));
-  LaneKeys<K, KPL> r;
-  if constexpr (B == 16) {
-    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-    if constexpr (sizeof(K) == 8) {
-      r.k[0] = (static_cast<uint64_t>(v.y) << 32) | v.x;
-      r.k[1] = (static_cast<uint64_t>(v.w) << 32) | v.z;
-    } else {
-      r.k[0] = v.x; r.k[1] = v.y; r.k[2] = v.z; r.k[3] = v.w;
-    }
-  } else if constexpr (B == 8) {
-    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
-    if constexpr (sizeof(K) == 8) {
-      r.k[0] = (static_cast<uint64_t>(v.y) << 32) | v.x;
-    } else {
-      r.k[0] = v.x; r.k[1] = v.y;
-    }
-  } else {
-    static_assert(B == 4, "4, 8 or 16 bytes per lane");
-    r.k[0] = *p;
-  }
-  return r;
-}
-
 // ---------------------------------------------------------------------------
 // Harmonia (harmonia_index, src/indexes.cuh:257-307; harmonia_tree,
 // src/harmonia.cuh:48-992).  Layout kept from the reference: 32 keys per node
@@ -49,18 +18,22 @@ __device__ __forceinline__ LaneKeys<K, KPL> load_lane_keys(const K* p) {
 // which the lookup computes instead of reading a 4-byte entry per level (at
 // 2^26 keys a 16.5 MiB array whose bottom-level reads miss L2); the top key
 // levels sit in LDS (the reference uses 42 KiB of __constant__,
-// src/harmonia.cuh:45-46); a node is searched by a group of G lanes of the
-// wave64 that fetch one 128-byte line per load and read a u64 node's second
-// line only when every key of the first line is below the probe (the
-// reference's early exit, src/harmonia.cuh:581-589).
+// src/harmonia.cuh:45-46); a node is searched by quads a 128-byte line at a time, a u64
+// node's second line only for probes above every key of the first (the reference's early
+// exit, src/harmonia.cuh:581-589).
+//
+// What bounds it: VALU issue while the nodes are in L2, then fabric lines.  Groups of 8, 16
+// or 32 lanes with a ballot and a population count per key took about three times the
+// instructions; harmonia_group_lanes is checked as before and changes nothing any more.
+// 2^24 probes, groups of 8 -> quads: 2^14 u64 keys 405 -> 213 us,
+// 2^20 u64 540 -> 355, 2^20 u32 391 -> 216, 2^22 u64 658 -> 477.
 // ---------------------------------------------------------------------------
-template <class K, int G>
+template <class K>
 struct HarmoniaDev {
+  using L = QuadLine<K, 128>;
   static constexpr int MK = 32;                                   // keys per node
-  static constexpr int LK = 128 / static_cast<int>(sizeof(K));    // keys per 128-byte line
-  static constexpr int LINES = MK / LK;                           // 2 (u64) or 1 (u32)
-  static constexpr int KPL = LK / G;                              // keys per lane per line
-  static_assert(KPL >= 1 && KPL * G == LK, "group must tile a line");
+  static constexpr uint32_t LK = L::kKeys;                        // keys per 128-byte line
+  static constexpr uint32_t LINES = MK / LK;                      // 2 (u64) or 1 (u32)
 
   const K* col;
   uint64_t n;
@@ -92,88 +65,53 @@ struct HarmoniaDev {
     return lds_levels ? static_cast<uint32_t>(lds_nodes - first[lds_levels - 1]) * MK + 1 : 1u;
   }
 
-  // Count of node keys below each lane's probe (and whether the key at that
-  // position equals the probe), for the G probes of the lane's group.  (Fetching each
-  // round's probe and offset from its lane where used, as the B-tree's search does, takes
-  // this kernel from 97 to 69 VGPRs and 4 to 7 waves per SIMD but from 18.0 to 14.8 G
-  // lookups/s at 2^26 u64 keys; shuffling only the probes, 16.9: the arrays stay.)
-  __device__ __forceinline__ uint32_t node_search(const K* base, uint64_t my_off, K my_x, int gbase, int gl,
-                                                  bool& my_eq) const {
-    uint64_t off[G];
-    K xs[G];
-    LaneKeys<K, KPL> v[G];
-#pragma unroll
-    for (int r = 0; r < G; ++r) {
-      off[r] = shfl64(my_off, gbase + r);
-      xs[r] = shfl(my_x, gbase + r);
-      v[r] = load_lane_keys<K, KPL>(base + off[r] + gl * KPL);
-    }
-    int c[G];
-    bool e[G];
-#pragma unroll
-    for (int r = 0; r < G; ++r) {
-      c[r] = 0;
-      e[r] = false;
-#pragma unroll
-      for (int j = 0; j < KPL; ++j) {
-        c[r] += group_popc<G>(ballot(v[r].k[j] < xs[r]), gbase);
-        e[r] |= group_popc<G>(ballot(v[r].k[j] == xs[r]), gbase) != 0;
-      }
-    }
+  // Keys of each lane's node below its probe; eq (leaves): the node holds the probe.
+  template <bool Leaf>
+  __device__ __forceinline__ uint32_t node_search(const K* base, uint32_t node, const QuadProbes<K>& q, int ql,
+                                                  bool& eq) const {
+    const K* lane_base = base + ql * L::kLaneKeys;
+    const uint32_t line = node * LINES;  // fewer than 2^32 keys, hence lines
+    L ln[kQuad];
+    quad_rounds([&](auto r) { ln[r].load(lane_base, quad_bcast<r>(line)); });
+    uint32_t below = quad_below(ln, q, ql);
+    if constexpr (Leaf) eq = quad_holds(ln, q, ql);
     if constexpr (LINES == 2) {
-      // every key of the first line is below the probe: read the second line; all such
-      // rounds request their second line before any is examined (one more latency, not G)
-#pragma unroll
-      for (int r = 0; r < G; ++r)
-        if (c[r] == LK) v[r] = load_lane_keys<K, KPL>(base + off[r] + LK + gl * KPL);
-#pragma unroll
-      for (int r = 0; r < G; ++r) {
-        if (c[r] != LK) continue;
-        int c2 = 0;
-        bool e2 = false;
-#pragma unroll
-        for (int j = 0; j < KPL; ++j) {
-          c2 += group_popc<G>(ballot(v[r].k[j] < xs[r]), gbase);
-          e2 |= group_popc<G>(ballot(v[r].k[j] == xs[r]), gbase) != 0;
+      const bool more = below == LK;
+      if (ballot(more) != 0) {  // wave-uniform
+        const uint32_t rounds = quad_or(more ? 1u << ql : 0u);
+        quad_rounds([&](auto r) {
+          const uint32_t l = quad_bcast<r>(line);
+          if ((rounds >> r) & 1u) ln[r].load(lane_base, l + 1);
+        });
+        const uint32_t rest = quad_below(ln, q, ql);
+        below += more ? rest : 0u;
+        if constexpr (Leaf) {
+          const bool e = quad_holds(ln, q, ql);
+          eq = more ? e : eq;
         }
-        c[r] += c2;
-        e[r] = e2;
       }
     }
-    uint32_t res = 0;
-    my_eq = false;
-#pragma unroll
-    for (int r = 0; r < G; ++r) {
-      if (gl == r) {
-        res = static_cast<uint32_t>(c[r]);
-        my_eq = e[r];
-      }
-    }
-    return res;
+    return below;
   }
 
   __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
-    const int ln = lane();
-    const int gbase = ln & ~(G - 1);
-    const int gl = ln & (G - 1);
+    const int ql = lane() & (kQuad - 1);
+    const QuadProbes<K> q(x);
     bool live = active;
     bool eq = false;
-    uint64_t pos = 0;
+    uint32_t pos = 0;  // fewer than 2^32 nodes
     uint32_t d = 0;
     const K* lds_keys = reinterpret_cast<const K*>(lds);
-    for (; d < lds_levels; ++d) {
-      const uint32_t lb = node_search(lds_keys, pos * MK, x, gbase, gl, eq);
-      const uint64_t next = first[d + 1] + 33ull * (pos - first[d]) + lb;
-      pos = live ? next : 0;
-    }
-    for (; d + 1 < depth; ++d) {
-      const uint32_t lb = node_search(keys, pos * MK, x, gbase, gl, eq);
-      const uint64_t next = first[d + 1] + 33ull * (pos - first[d]) + lb;
-      pos = live ? next : 0;
-    }
-    const uint64_t leaf = live ? pos - inner_nodes : 0;
-    const uint32_t lb = node_search(col, leaf * MK, x, gbase, gl, eq);
-    return (live && eq) ? static_cast<uint32_t>(leaf * MK + lb) : kNotFound;
+    auto step = [&](const K* from) {
+      const uint32_t lb = node_search<false>(from, pos, q, ql, eq);
+      const uint32_t f = static_cast<uint32_t>(first[d]), next = static_cast<uint32_t>(first[d + 1]);
+      pos = live ? next + 33u * (pos - f) + lb : 0u;
+    };
+    for (; d < lds_levels; ++d) step(lds_keys);
+    for (; d + 1 < depth; ++d) step(keys);
+    const uint32_t leaf = live ? pos - static_cast<uint32_t>(inner_nodes) : 0u;
+    const uint32_t lb = node_search<true>(col, leaf, q, ql, eq);
+    return (live && eq) ? leaf * MK + lb : kNotFound;
   }
 };
 

@@ -130,17 +130,8 @@ void with_index_dev(const gj_index& ix, F&& f) {
       return;
     case GJ_NO_OP: f(NoOpDev<K>{}); return;
     case GJ_HARMONIA:
-      switch (ix.params.harmonia_group_lanes) {
-        case 8: f(ix.harmonia_dev<K, 8>()); return;
-        case 16: f(ix.harmonia_dev<K, 16>()); return;
-        case 32:
-          if constexpr (sizeof(K) == 4) {
-            f(ix.harmonia_dev<K, 32>());
-            return;
-          }
-          break;
-      }
-      throw error(GJ_ERR_INVALID, "unsupported harmonia_group_lanes");
+      f(ix.harmonia_dev<K>());
+      return;
     case GJ_RADIX_SPLINE:
       if (ix.rs_mode == kRsRadixLds)
         f(ix.rs_dev<K, kRsRadixLds>());

@@ -80,7 +80,7 @@ typedef enum gj_approach {
 typedef struct gj_index_params {
   uint32_t rs_radix_bits;        /* RadixSpline radix bits, default 18 */
   uint32_t rs_max_error;         /* RadixSpline error bound, default 32 */
-  uint32_t harmonia_group_lanes; /* lanes per Harmonia node search (8, 16, or 32 for u32 keys), default 8 */
+  uint32_t harmonia_group_lanes; /* 8, 16, or 32 for u32 keys, default 8; nodes are searched by four lanes whichever it is */
   uint32_t btree_lds_bytes;      /* LDS budget for resident upper B-tree levels, default 16384 */
   uint32_t learned_leaf_bits;    /* log2 of the number of linear leaves; 0 (default) = max(16, ceil(log2 n) - 10)
                                     16-byte leaves, or twice as many 8-byte leaves from 2^22 keys when the
@@ -394,7 +394,7 @@ int gj_autotune_lookup(const gj_index* index, const void* d_probe_sample, uint64
  * parameters, times the plain lookup of the probe sample on each, and writes
  * the fastest parameter set into *best.  Candidates, starting from *base (or
  * the defaults when base is NULL):
- *   harmonia      harmonia_group_lanes 8 / 16 (/ 32 for 4-byte keys): threads per lookup
+ *   harmonia      harmonia_group_lanes 8 / 16 (/ 32 for 4-byte keys), which time alike
  *   btree         btree_lds_bytes 4096 / 16384 / 32768: the LDS-resident upper levels
  *   radix_spline  rs_radix_bits 12 / 13 (table in LDS) / 16 / 18 (global) x rs_max_error 16 / 32 / 64
  *   learned_plr   learned_leaf_bits 0 (the default: compact 8-byte leaves where the build
