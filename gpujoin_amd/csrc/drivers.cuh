@@ -89,34 +89,38 @@ __device__ __forceinline__ uint32_t xcd_logical_block() {
 // src/index_lookup_partitioning.cu:218-248): tuple t has key keys[t], and its row id
 // goes to res[t], in tuple order (full-line stores); the driver then gathers the row ids
 // back to probe order.  Padding tuples (key_max) are looked up too, their row ids never
-// read.  Each XCD takes one contiguous eighth of the tuples, and the workgroups of an
-// XCD sweep it together, one workgroup-wide step apart, so the key range in flight on
-// an XCD (hence the index nodes and column lines its L2 must hold) spans a few
-// partitions rather than one partition per workgroup.  The tuple count is read from
-// *d_total when given (it is known only on the device).
+// read.  The relation is `windows` windows one after the other, window w from tuple
+// start[w * fan] to start[(w + 1) * fan], each in key order by partition.  Each XCD takes one
+// contiguous eighth of every window, and its workgroups sweep these eighths together, a tile of
+// each window in turn, so the key range in flight on an XCD (hence the index nodes and
+// column lines its L2 must hold) spans a few partitions, the same ones in all the
+// windows.
+//
+// What bounds it: fabric lines where the tuples are sparse, else the L1 (the B-tree over 2^25
+// u64 keys: 8.6 accesses and 0.23 fabric lines a tuple).  Staging a run's separators in LDS
+// so that a tuple reads its leaf line alone took as long: the run's own chain (bounds,
+// descent, staging) costs what the inner levels do.
 template <class Dev, class K>
 __global__ __launch_bounds__(256) void lookup_tuples_kernel(Dev d, const K* __restrict__ keys,
-                                                            const uint64_t* __restrict__ d_total, uint64_t total_max,
-                                                            uint32_t* __restrict__ res) {
+                                                            const uint64_t* __restrict__ start, uint32_t windows,
+                                                            uint64_t fan, uint32_t tiles, uint32_t* __restrict__ res) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   d.stage(lds);
   __syncthreads();
-  uint64_t total = total_max;
-  if (d_total) total = *d_total < total_max ? *d_total : total_max;
   const uint32_t groups = (gridDim.x % 8 == 0) ? 8u : 1u;  // XCDs
   const uint32_t per = gridDim.x / groups;                 // workgroups per XCD
-  const uint64_t chunk = ((total + groups - 1) / groups + kWave - 1) / kWave * kWave;
-  const uint64_t lo = static_cast<uint64_t>(blockIdx.x % groups) * chunk;
-  const uint64_t hi = (lo + chunk < total) ? lo + chunk : total;
-  const uint64_t w = threadIdx.x / kWave;
-  const uint64_t step = static_cast<uint64_t>(per) * blockDim.x;
-  for (uint64_t base = lo + static_cast<uint64_t>(blockIdx.x / groups) * blockDim.x + w * kWave; base < hi;
-       base += step) {
-    const uint64_t i = base + static_cast<uint64_t>(lane());
+  const uint64_t g = blockIdx.x % groups;
+  for (uint32_t j = blockIdx.x / groups; j < tiles; j += per) {  // this XCD's tiles, windows in turn
+    const uint32_t t = windows == 1 ? j : j / windows, w = j - t * windows;
+    const uint64_t first = start[w * fan], size = start[(w + 1) * fan] - first;
+    const uint64_t chunk = ((size + groups - 1) / groups + kWave - 1) / kWave * kWave;
+    const uint64_t lo = g * chunk, hi = lo + chunk < size ? lo + chunk : size;
+    const uint64_t i = lo + static_cast<uint64_t>(t) * blockDim.x + threadIdx.x;
+    if (i - lane() >= hi) continue;  // wave-uniform
     const bool active = i < hi;
-    const K x = active ? load_stream(keys + i) : K(0);
+    const K x = active ? load_stream(keys + first + i) : K(0);
     const uint32_t r = d.lookup(x, active, lds);
-    if (active) store_stream(res + i, r);
+    if (active) store_stream(res + first + i, r);
   }
 }
 

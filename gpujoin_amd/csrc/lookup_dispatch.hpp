@@ -69,20 +69,26 @@ void launch_marked(const BTreeDev<K>& d, const K* probes, uint64_t m, uint32_t* 
   GJ_HIP_CHECK(hipGetLastError());
 }
 
-// total_max bounds the tuple count; d_total (optional) holds the exact count on the device.
+// Tuples of `windows` windows of up to window_max tuples each (padding included); start:
+// the starts of their partitions, `fan` a window, on the device.
 template <class Dev, class K>
-void launch_tuples(const Dev& d, const K* keys, const uint64_t* d_total, uint64_t total_max, uint32_t* res,
-                   const gj_lookup_params& p, hipStream_t s, int cu) {
-  if (total_max == 0) return;
+void launch_tuples(const Dev& d, const K* keys, const uint64_t* start, uint32_t windows, uint64_t fan,
+                   uint64_t window_max, uint32_t* res, const gj_lookup_params& p, hipStream_t s, int cu) {
+  if (windows == 0 || window_max == 0) return;
   const unsigned block = lookup_block(p);
   const size_t lds = d.lds_bytes();
   const void* fn = reinterpret_cast<const void*>(&lookup_tuples_kernel<Dev, K>);
+  const uint64_t total = windows * window_max;
   uint64_t blocks = p.grid_blocks
-                        ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(total_max, block)))
-                        : cover_blocks(total_max, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
-  if (blocks >= 8) blocks = blocks / 8 * 8;  // whole XCD rounds for the XCD-major chunk map
+                        ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(total, block)))
+                        : cover_blocks(total, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
+  if (blocks >= 8) blocks = ceil_div(blocks, 8) * 8;  // whole XCD rounds for the XCD-major chunk map
+  const uint64_t groups = blocks % 8 == 0 ? 8 : 1;
+  // a window's share of an XCD is rounded up to whole waves
+  const uint64_t tiles = windows * ceil_div(ceil_div(window_max, groups) + kWave, block);
+  GJ_REQUIRE(tiles + blocks < 0xFFFFFFFFull, GJ_ERR_INTERNAL, "too many tuple tiles");  // fewer than 2^32 tuples in all
   hipLaunchKernelGGL((lookup_tuples_kernel<Dev, K>), dim3(static_cast<unsigned>(blocks)), dim3(block), lds, s, d,
-                     keys, d_total, total_max, res);
+                     keys, start, windows, fan, static_cast<uint32_t>(tiles), res);
   GJ_HIP_CHECK(hipGetLastError());
 }
 
