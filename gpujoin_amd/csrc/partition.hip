@@ -62,7 +62,7 @@ __device__ __forceinline__ bool seg_range(const Seg& sg, uint64_t c, uint64_t ch
     lo = c * chunk;
     hi = std::min<uint64_t>(m, lo + chunk);
     pbase = 0;
-    return true;
+    return lo < m || c == 0;  // workgroups past the chunks have no work
   }
   if (c >= sg.chunk0[sg.segs]) return false;
   uint32_t a = 0, b = sg.segs;  // the segment h with chunk0[h] <= c < chunk0[h + 1]
@@ -744,8 +744,15 @@ struct Scatter {
   Seg sg;
 };
 
+// Workgroups past the chunks share the padding alone: with few items and many partitions a
+// thread would pad one slot after the other (5.5 k u32 items into 2^11 partitions: two
+// workgroups took 51 us, now 9.6).
 template <class K>
 void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, hipStream_t s) {
+  if (a.align > 1) {
+    const uint64_t slots = (static_cast<uint64_t>(a.sg.segs ? a.sg.segs : 1u) << a.bits) * a.align;
+    grid = std::max(grid, static_cast<unsigned>(std::min<uint64_t>(ceil_div(slots, 2 * kTileBlock), 512)));
+  }
   const size_t lds = tile_lds_bytes(1u << a.bits, sizeof(K), a.out_payload != nullptr, stable, kTileBlock, kTileItems);
   GJ_REQUIRE(lds <= kMaxLds - 1024 && (1u << a.bits) <= 8u * kTileBlock, GJ_ERR_INTERNAL,
              "partition fan-out does not fit the LDS");
@@ -831,6 +838,7 @@ uint64_t partition_scratch(uint64_t m, int key_bytes, uint32_t bits, uint32_t pa
 // partitions h * 2^bits + p, with 128-byte aligned starts.  Chunks never straddle
 // segments, so every histogram row and cursor belongs to one segment.
 constexpr uint64_t kSegChunk = 16384;
+constexpr uint64_t kSegMinChunks = 512;  // two workgroups for each of 256 CUs
 // Segments of this many chunks on average scan their histogram columns with a workgroup
 // per 64 partitions; shorter ones take one thread per partition.
 constexpr uint64_t kSegWideChunks = 32;
@@ -843,15 +851,17 @@ void partition_segmented(const K* keys, const uint32_t* payload, uint64_t m, uin
                          unsigned long long* dropped, hipStream_t s) {
   const uint32_t fan = 1u << bits;
   const uint64_t total_fan = static_cast<uint64_t>(segs) * fan;
-  const uint64_t blocks = ceil_div(m, kSegChunk) + segs;  // an upper bound on the chunks
+  // whole tiles, down to one where longer chunks would leave CUs without a workgroup
+  const uint64_t chunk = std::clamp<uint64_t>(ceil_div(ceil_div(m, kSegMinChunks), kPartTile) * kPartTile, kPartTile, kSegChunk);
+  const uint64_t blocks = ceil_div(m, chunk) + segs;  // an upper bound on the chunks
   GJ_REQUIRE(blocks < (1ull << 31), GJ_ERR_INVALID, "too many partition chunks");
-  hipLaunchKernelGGL(seg_chunks_kernel, dim3(1), dim3(1024), 0, s, count1, segs, kSegChunk, chunk0);
+  hipLaunchKernelGGL(seg_chunks_kernel, dim3(1), dim3(1024), 0, s, count1, segs, chunk, chunk0);
   GJ_HIP_CHECK(hipGetLastError());
   const Seg sg{chunk0, start1, count1, segs};
   hipLaunchKernelGGL(part_hist_kernel<K>, dim3(static_cast<unsigned>(blocks)), dim3(kTileBlock),
-                     fan * sizeof(uint32_t), s, keys, m, kSegChunk, shift, bits, hist, sg);
+                     fan * sizeof(uint32_t), s, keys, m, chunk, shift, bits, hist, sg);
   GJ_HIP_CHECK(hipGetLastError());
-  if (ceil_div(m, kSegChunk) >= kSegWideChunks * segs)
+  if (ceil_div(m, chunk) >= kSegWideChunks * segs)
     hipLaunchKernelGGL(seg_colscan_wide_kernel, dim3(segs * ((fan + kWave - 1) / kWave)), dim3(kColThreads), 0, s, hist,
                        chunk0, fan, count);
   else
@@ -860,7 +870,7 @@ void partition_segmented(const K* keys, const uint32_t* payload, uint64_t m, uin
   GJ_HIP_CHECK(hipGetLastError());
   launch_scan_starts(count, total_fan, align, start, nullptr, sums, s);
   const uint64_t cap = m + (align > 1 ? total_fan * align : 0ull);
-  launch_scatter<K>({keys, payload, 0u, m, kSegChunk, shift, bits, hist, start, count, align, out_keys, out_payload, inv,
+  launch_scatter<K>({keys, payload, 0u, m, chunk, shift, bits, hist, start, count, align, out_keys, out_payload, inv,
                      cap, dropped, sg},
                     stable, static_cast<unsigned>(blocks), s);
 }
