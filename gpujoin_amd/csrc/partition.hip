@@ -838,7 +838,9 @@ uint64_t partition_scratch(uint64_t m, int key_bytes, uint32_t bits, uint32_t pa
 // partitions h * 2^bits + p, with 128-byte aligned starts.  Chunks never straddle
 // segments, so every histogram row and cursor belongs to one segment.
 constexpr uint64_t kSegChunk = 16384;
-constexpr uint64_t kSegMinChunks = 512;  // two workgroups for each of 256 CUs
+// two workgroups for each of 256 CUs (two windows of 262144 u32 probes at fan-out 2^12, the whole
+// lookup: 107 -> 66 us)
+constexpr uint64_t kSegMinChunks = 512;
 // Segments of this many chunks on average scan their histogram columns with a workgroup
 // per 64 partitions; shorter ones take one thread per partition.
 constexpr uint64_t kSegWideChunks = 32;
