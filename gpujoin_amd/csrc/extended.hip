@@ -399,9 +399,12 @@ void build_hash_table(const gj_index& ix, dbuf& table, uint64_t& cap, dbuf& temp
   const uint32_t bits = ilog2_floor(cap) - rb;  // ranges = partitions
   const uint64_t ranges = 1ull << bits, n = ix.n;
   const uint64_t tcap = partition_capacity(n, sizeof(K), bits);
-  // temp: hashes | partitioned hashes | row ids | start (ranges + 1) | count | spills | partitioner scratch
+  // The partitioner hashes the keys itself as it reads them, twice; over the host link they
+  // are read once, into hashes in device memory (2^22 u64 keys in HBM: that pass took 16 us).
+  const bool first = ix.col_in_host;
+  // temp: hashes (first) | partitioned hashes | row ids | start (ranges + 1) | count | spills | partitioner scratch
   auto up = [](uint64_t b) { return (b + 255) / 256 * 256; };
-  const uint64_t o_pk = up(n * sizeof(K)), o_pr = o_pk + up(tcap * sizeof(K)), o_st = o_pr + up(tcap * 4),
+  const uint64_t o_pk = first ? up(n * sizeof(K)) : 0, o_pr = o_pk + up(tcap * sizeof(K)), o_st = o_pr + up(tcap * 4),
                  o_ct = o_st + up((ranges + 1) * 8), o_sp = o_ct + up(ranges * 8), o_ps = o_sp + up(ranges * 4),
                  bytes = o_ps + up(partition_scratch(n, sizeof(K), bits, 1));
   temp.reserve(bytes);
@@ -412,11 +415,13 @@ void build_hash_table(const gj_index& ix, dbuf& table, uint64_t& cap, dbuf& temp
   uint64_t* st = reinterpret_cast<uint64_t*>(base + o_st);
   uint64_t* ct = reinterpret_cast<uint64_t*>(base + o_ct);
   uint32_t* sp = reinterpret_cast<uint32_t*>(base + o_sp);
-  hipLaunchKernelGGL(ht_hash_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, static_cast<const K*>(ix.d_col), n, hk);
-  GJ_HIP_CHECK(hipGetLastError());
+  if (first) {
+    hipLaunchKernelGGL(ht_hash_kernel<K>, dim3(grid_for(n, 256)), dim3(256), 0, s, static_cast<const K*>(ix.d_col), n, hk);
+    GJ_HIP_CHECK(hipGetLastError());
+  }
   // payload = row id; the digit is the range of the home slot
-  partition_keys<K>(hk, n, 0, bits, rb, 1, false, pk, pr, st, ct, base + o_ps,
-                    ix.dropped.as<unsigned long long>(), ix.cu, s);
+  partition_keys<K>(first ? hk : static_cast<const K*>(ix.d_col), n, 0, bits, rb, 1, false, pk, pr, st, ct, base + o_ps,
+                    ix.dropped.as<unsigned long long>(), ix.cu, s, nullptr, !first);
   const size_t lds = (static_cast<size_t>(1) << rb) * (8 + 4);
   const void* fn = reinterpret_cast<const void*>(&ht_range_build_kernel<K>);
   if (lds > 65536)

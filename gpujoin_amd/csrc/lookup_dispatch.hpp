@@ -170,7 +170,8 @@ uint64_t hash_capacity(uint64_t n);
 
 // Radix partitioner (partition.hip).  stable: input order kept inside every
 // partition; otherwise the order inside a partition is arbitrary.  start2 (optional)
-// receives a second copy of the 2^bits partition starts.
+// receives a second copy of the 2^bits partition starts.  hashed: the keys' hashes
+// (key_hash) are partitioned and written in their place.
 uint64_t partition_capacity(uint64_t m, int key_bytes, uint32_t bits);
 uint64_t partition_scratch(uint64_t m, int key_bytes, uint32_t bits, uint32_t passes);
 // A batch of m probes cut into windows of `window`, each window partitioned on its own
@@ -188,7 +189,8 @@ void partition_windows(const K* keys, uint64_t m, uint64_t window, uint32_t bits
 template <class K>
 void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t bits, uint32_t ignore, uint32_t passes,
                     bool stable, K* out_keys, uint32_t* out_payload, uint64_t* start, uint64_t* count, uint8_t* scratch,
-                    unsigned long long* dropped, int cu, hipStream_t s, uint64_t* start2 = nullptr);
+                    unsigned long long* dropped, int cu, hipStream_t s, uint64_t* start2 = nullptr,
+                    bool hashed = false);
 
 // Bytes of index-private device memory held by the extended kinds.
 uint64_t extended_memory(const gj_index& ix);

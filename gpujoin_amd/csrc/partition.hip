@@ -76,8 +76,16 @@ __device__ __forceinline__ bool seg_range(const Seg& sg, uint64_t c, uint64_t ch
   return true;
 }
 
+// What is partitioned: the keys, or their hashes (the hash table's build; computing the hash
+// where a key is read costs less than a pass that writes it and two that read it back).
+template <bool Hashed, class K>
+__device__ __forceinline__ K item_of(K k) {
+  if constexpr (Hashed) return static_cast<K>(key_hash<K>(static_cast<uint64_t>(k)));
+  return k;
+}
+
 // One block per chunk (256 or 1024 threads), four loads in flight per thread.
-template <class K>
+template <class K, bool Hashed = false>
 __global__ __launch_bounds__(1024) void part_hist_kernel(const K* __restrict__ keys, uint64_t m, uint64_t chunk,
                                                          uint32_t shift, uint32_t bits, uint32_t* __restrict__ hist,
                                                          Seg sg) {
@@ -99,7 +107,7 @@ __global__ __launch_bounds__(1024) void part_hist_kernel(const K* __restrict__ k
     }
 #pragma unroll
     for (int u = 0; u < kIn; ++u)
-      if (i0 + static_cast<uint64_t>(u) * blockDim.x < hi) atomicAdd(&h[digit_of(v[u], shift, fan - 1)], 1u);
+      if (i0 + static_cast<uint64_t>(u) * blockDim.x < hi) atomicAdd(&h[digit_of(item_of<Hashed>(v[u]), shift, fan - 1)], 1u);
   }
   __syncthreads();
   for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x) hist[c * fan + p] = h[p];
@@ -166,6 +174,28 @@ __global__ __launch_bounds__(kColThreads) void seg_colscan_wide_kernel(uint32_t*
   scan_columns(hist, chunk0[h], chunk0[h + 1], (blockIdx.x % per) * kWave, fan, count + static_cast<uint64_t>(h) * fan);
 }
 
+// Sum of v over the block's earlier threads (1024 threads); total: over all of them.
+__device__ __forceinline__ uint64_t sum_before_1024(uint64_t v, uint64_t& total) {
+  __shared__ uint64_t waves[1024 / kWave];
+  uint64_t x = v;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint64_t y = __shfl_up(x, o, kWave);
+    if (lane() >= o) x += y;
+  }
+  const uint32_t w = threadIdx.x / kWave;
+  if (lane() == kWave - 1) waves[w] = x;
+  __syncthreads();
+  uint64_t before = x - v;
+  total = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < 1024 / kWave; ++q) {
+    before += q < w ? waves[q] : 0;
+    total += waves[q];
+  }
+  return before;
+}
+
 // start[p] = align_up(start[p-1] + count[p-1], align); one block of 1024 threads.
 // Each thread owns `per` consecutive partitions and reads their counts kScanBatch at a
 // time, loads first (a thread's loads do not depend on one another, so a batch is in
@@ -175,7 +205,6 @@ constexpr uint32_t kScanBatch = 8;
 __global__ __launch_bounds__(1024) void part_scan_starts_kernel(const uint64_t* __restrict__ count, uint32_t fan,
                                                                 uint32_t align, uint64_t* __restrict__ start,
                                                                 uint64_t* __restrict__ start2) {
-  __shared__ uint64_t s[1024];
   const uint32_t per = (fan + blockDim.x - 1) / blockDim.x;
   const uint32_t p0 = threadIdx.x * per;
   uint64_t local = 0;
@@ -189,15 +218,8 @@ __global__ __launch_bounds__(1024) void part_scan_starts_kernel(const uint64_t* 
 #pragma unroll
     for (uint32_t u = 0; u < kScanBatch; ++u) local += (c[u] + align - 1) / align * align;
   }
-  s[threadIdx.x] = local;
-  __syncthreads();
-  for (uint32_t off = 1; off < blockDim.x; off <<= 1) {  // Hillis-Steele inclusive scan
-    const uint64_t v = threadIdx.x >= off ? s[threadIdx.x - off] : 0;
-    __syncthreads();
-    s[threadIdx.x] += v;
-    __syncthreads();
-  }
-  uint64_t run = s[threadIdx.x] - local;
+  uint64_t total;
+  uint64_t run = sum_before_1024(local, total);
   for (uint32_t q = 0; q < per; q += kScanBatch) {
     uint64_t c[kScanBatch];
 #pragma unroll
@@ -215,7 +237,7 @@ __global__ __launch_bounds__(1024) void part_scan_starts_kernel(const uint64_t* 
       run += (c[u] + align - 1) / align * align;
     }
   }
-  if (threadIdx.x == blockDim.x - 1) start[fan] = s[threadIdx.x];  // padded total
+  if (threadIdx.x == 0) start[fan] = total;  // padded
 }
 
 // The same starts over many partitions (a batch of windows brings up to 2^18, where one
@@ -369,7 +391,7 @@ __host__ __device__ constexpr size_t tile_lds_bytes(uint32_t fan, int key_bytes,
          + static_cast<size_t>(fan) * (stable ? 2 * (block / kWave) + 2 : 4);   // rows and offsets, or counts
 }
 
-template <class K, bool Stable, bool InPayload, int B, int I>
+template <class K, bool Stable, bool InPayload, bool Hashed, int B, int I>
 __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
     const K* __restrict__ keys, const uint32_t* __restrict__ in_payload, uint32_t payload_base, uint64_t m,
     uint64_t chunk, uint32_t shift, uint32_t bits, const uint32_t* __restrict__ block_off,
@@ -501,7 +523,7 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
     uint32_t pay[InPayload ? I : 1], rk[I];
 #pragma unroll
     for (int j = 0; j < I; ++j) {
-      k[j] = kn[j];
+      k[j] = item_of<Hashed>(kn[j]);
       if constexpr (InPayload) {
         const uint32_t i = static_cast<uint32_t>(j * kWave + ln);
         pay[j] = i < wn ? load_stream(in_payload + wbase + i) : 0u;
@@ -604,7 +626,6 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
 // thousands of segments), counts read kScanBatch at a time.
 __global__ __launch_bounds__(1024) void seg_chunks_kernel(const uint64_t* __restrict__ count, uint32_t segs,
                                                           uint64_t chunk, uint64_t* __restrict__ chunk0) {
-  __shared__ uint64_t s[1024];
   const uint32_t per = (segs + blockDim.x - 1) / blockDim.x;
   const uint32_t h0 = threadIdx.x * per;
   uint64_t local = 0;
@@ -618,15 +639,8 @@ __global__ __launch_bounds__(1024) void seg_chunks_kernel(const uint64_t* __rest
 #pragma unroll
     for (uint32_t u = 0; u < kScanBatch; ++u) local += (c[u] + chunk - 1) / chunk;
   }
-  s[threadIdx.x] = local;
-  __syncthreads();
-  for (uint32_t off = 1; off < blockDim.x; off <<= 1) {  // Hillis-Steele inclusive scan
-    const uint64_t v = threadIdx.x >= off ? s[threadIdx.x - off] : 0;
-    __syncthreads();
-    s[threadIdx.x] += v;
-    __syncthreads();
-  }
-  uint64_t run = s[threadIdx.x] - local;
+  uint64_t total;
+  uint64_t run = sum_before_1024(local, total);
   for (uint32_t q = 0; q < per; q += kScanBatch) {
     uint64_t c[kScanBatch];
 #pragma unroll
@@ -641,7 +655,7 @@ __global__ __launch_bounds__(1024) void seg_chunks_kernel(const uint64_t* __rest
       run += (c[u] + chunk - 1) / chunk;
     }
   }
-  if (threadIdx.x == blockDim.x - 1) chunk0[segs] = s[threadIdx.x];
+  if (threadIdx.x == 0) chunk0[segs] = total;
 }
 
 // Segments of a batch of windows: segment h = probes [h * window, min((h + 1) * window, m)).
@@ -748,7 +762,7 @@ struct Scatter {
 // thread would pad one slot after the other (5.5 k u32 items into 2^11 partitions: two
 // workgroups took 51 us, now 9.6).
 template <class K>
-void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, hipStream_t s) {
+void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, hipStream_t s, bool hashed = false) {
   if (a.align > 1) {
     const uint64_t slots = (static_cast<uint64_t>(a.sg.segs ? a.sg.segs : 1u) << a.bits) * a.align;
     grid = std::max(grid, static_cast<unsigned>(std::min<uint64_t>(ceil_div(slots, 2 * kTileBlock), 512)));
@@ -756,8 +770,8 @@ void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, hipStream_t
   const size_t lds = tile_lds_bytes(1u << a.bits, sizeof(K), a.out_payload != nullptr, stable, kTileBlock, kTileItems);
   GJ_REQUIRE(lds <= kMaxLds - 1024 && (1u << a.bits) <= 8u * kTileBlock, GJ_ERR_INTERNAL,
              "partition fan-out does not fit the LDS");
-  auto go = [&]<bool Stable, bool InPayload>() {
-    auto kernel = &part_scatter_kernel<K, Stable, InPayload, kTileBlock, kTileItems>;
+  auto go = [&]<bool Stable, bool InPayload, bool Hashed = false>() {
+    auto kernel = &part_scatter_kernel<K, Stable, InPayload, Hashed, kTileBlock, kTileItems>;
     if (lds > 65536)
       GJ_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
@@ -766,7 +780,9 @@ void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, hipStream_t
                        a.dropped, a.sg);
     GJ_HIP_CHECK(hipGetLastError());
   };
-  if (stable && a.in_payload) go.template operator()<true, true>();
+  GJ_REQUIRE(!hashed || (!stable && !a.in_payload), GJ_ERR_INTERNAL, "hashes are partitioned unordered, by position");
+  if (hashed) go.template operator()<false, false, true>();
+  else if (stable && a.in_payload) go.template operator()<true, true>();
   else if (stable) go.template operator()<true, false>();
   else if (a.in_payload) go.template operator()<false, true>();
   else go.template operator()<false, false>();
@@ -809,10 +825,11 @@ template <class K>
 void partition_pass(const K* keys, const uint32_t* in_payload, uint32_t payload_base, uint64_t m, uint32_t shift,
                     uint32_t bits, uint32_t align, bool stable, K* out_keys, uint32_t* out_payload, uint64_t* start,
                     uint64_t* start2, uint64_t* count, uint32_t* hist, uint64_t* sums, unsigned long long* dropped,
-                    int cu, hipStream_t s) {
+                    int cu, hipStream_t s, bool hashed = false) {
   const PartPlan p = plan(m, bits, cu, 2);
-  hipLaunchKernelGGL(part_hist_kernel<K>, dim3(p.blocks), dim3(1024), p.fan * sizeof(uint32_t), s,
-                     keys, m, p.chunk, shift, bits, hist, Seg{});
+  auto histogram = hashed ? &part_hist_kernel<K, true> : &part_hist_kernel<K, false>;
+  hipLaunchKernelGGL(histogram, dim3(p.blocks), dim3(1024), p.fan * sizeof(uint32_t), s, keys, m, p.chunk, shift, bits,
+                     hist, Seg{});
   GJ_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(part_colscan_kernel, dim3((p.fan + kWave - 1) / kWave), dim3(kColThreads), 0, s, hist, p.blocks,
                      p.fan, count);
@@ -821,7 +838,7 @@ void partition_pass(const K* keys, const uint32_t* in_payload, uint32_t payload_
   const uint64_t cap = m + (align > 1 ? static_cast<uint64_t>(p.fan) * align : 0ull);
   launch_scatter<K>({keys, in_payload, payload_base, m, p.chunk, shift, bits, hist, start, count, align, out_keys,
                      out_payload, nullptr, cap, dropped, Seg{}},
-                    stable, p.blocks, s);
+                    stable, p.blocks, s, hashed);
 }
 
 uint64_t partition_capacity(uint64_t m, int key_bytes, uint32_t bits) {
@@ -979,7 +996,7 @@ template void partition_windows<uint64_t>(const uint64_t*, uint64_t, uint64_t, u
 template <class K>
 void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t bits, uint32_t ignore, uint32_t passes,
                     bool stable, K* out_keys, uint32_t* out_payload, uint64_t* start, uint64_t* count, uint8_t* scratch,
-                    unsigned long long* dropped, int cu, hipStream_t s, uint64_t* start2) {
+                    unsigned long long* dropped, int cu, hipStream_t s, uint64_t* start2, bool hashed) {
   auto* sums = reinterpret_cast<uint64_t*>(scratch);
   uint32_t* hist = reinterpret_cast<uint32_t*>(scratch + kScanSumsBytes);
   const uint32_t align = part_align(sizeof(K));
@@ -994,7 +1011,7 @@ void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t b
     auto* count1 = start1 + segs + 2;
     auto* chunk0 = count1 + segs + 2;
     partition_pass<K>(keys, nullptr, payload_base, m, ignore + lb, hb, 1, stable, tk, tp, start1, nullptr, count1, hist,
-                      sums, dropped, cu, s);
+                      sums, dropped, cu, s, hashed);
     partition_segmented<K>(tk, tp, m, ignore, lb, segs, start1, count1, chunk0, align, stable, out_keys, out_payload,
                            nullptr, start, count, hist, sums, dropped, s);
     if (start2) GJ_HIP_CHECK(hipMemcpyAsync(start2, start, (1ull << bits) * 8, hipMemcpyDeviceToDevice, s));
@@ -1002,7 +1019,7 @@ void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t b
   }
   if (passes == 1 || bits < 2) {
     partition_pass<K>(keys, nullptr, payload_base, m, ignore, bits, align, stable, out_keys, out_payload, start, start2,
-                      count, hist, sums, dropped, cu, s);
+                      count, hist, sums, dropped, cu, s, hashed);
     return;
   }
   // pass 1: the high half of the digit, unpadded, into scratch; pass 2: the full digit.
@@ -1011,16 +1028,16 @@ void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t b
   K* tk = reinterpret_cast<K*>(tmp);
   uint32_t* tp = reinterpret_cast<uint32_t*>(tmp + ceil_div((m + 32) * sizeof(K), 256) * 256);
   partition_pass<K>(keys, nullptr, payload_base, m, ignore + (bits - b_hi), b_hi, 1, stable, tk, tp, start, nullptr,
-                    count, hist, sums, dropped, cu, s);
+                    count, hist, sums, dropped, cu, s, hashed);
   partition_pass<K>(tk, tp, 0, m, ignore, bits, align, stable, out_keys, out_payload, start, start2, count, hist, sums,
                     dropped, cu, s);
 }
 template void partition_keys<uint32_t>(const uint32_t*, uint64_t, uint32_t, uint32_t, uint32_t, uint32_t, bool,
                                        uint32_t*, uint32_t*, uint64_t*, uint64_t*, uint8_t*, unsigned long long*, int,
-                                       hipStream_t, uint64_t*);
+                                       hipStream_t, uint64_t*, bool);
 template void partition_keys<uint64_t>(const uint64_t*, uint64_t, uint32_t, uint32_t, uint32_t, uint32_t, bool,
                                        uint64_t*, uint32_t*, uint64_t*, uint64_t*, uint8_t*, unsigned long long*, int,
-                                       hipStream_t, uint64_t*);
+                                       hipStream_t, uint64_t*, bool);
 
 }  // namespace gj
 
