@@ -30,10 +30,17 @@ constexpr uint32_t kMaxRadixBits = 16;
 
 __host__ __device__ __forceinline__ uint32_t part_align(int key_bytes) { return 128u / static_cast<uint32_t>(key_bytes); }
 
-template <class K>
-__device__ __forceinline__ uint32_t digit_of(K k, uint32_t shift, uint32_t mask) {
-  return static_cast<uint32_t>(static_cast<uint64_t>(k) >> shift) & mask;
-}
+// The digit (k >> shift) & (fan - 1).  ignore_bits is only held below the key's width, so a
+// digit may reach past the key's top bit, and the first pass of two may begin there: those
+// digit bits are zero, while the shift itself takes its distance modulo 64.
+struct Digit {
+  uint32_t shift, mask;
+  __device__ __forceinline__ Digit(uint32_t s, uint32_t fan) : shift(s & 63u), mask(s < 64u ? fan - 1u : 0u) {}
+  template <class K>
+  __device__ __forceinline__ uint32_t operator()(K k) const {
+    return static_cast<uint32_t>(static_cast<uint64_t>(k) >> shift) & mask;
+  }
+};
 
 // A store that would land past the output's capacity is not made; it is counted
 // instead (never for a consistent histogram), so callers can report the loss.
@@ -95,6 +102,7 @@ __global__ __launch_bounds__(1024) void part_hist_kernel(const K* __restrict__ k
   const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block();
   uint64_t lo, hi, pbase;
   if (!seg_range(sg, c, chunk, m, fan, lo, hi, pbase)) return;  // block-uniform, before any barrier
+  const Digit digit(shift, fan);
   for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x) h[p] = 0;
   __syncthreads();
   constexpr int kIn = 4;
@@ -107,7 +115,7 @@ __global__ __launch_bounds__(1024) void part_hist_kernel(const K* __restrict__ k
     }
 #pragma unroll
     for (int u = 0; u < kIn; ++u)
-      if (i0 + static_cast<uint64_t>(u) * blockDim.x < hi) atomicAdd(&h[digit_of(item_of<Hashed>(v[u]), shift, fan - 1)], 1u);
+      if (i0 + static_cast<uint64_t>(u) * blockDim.x < hi) atomicAdd(&h[digit(item_of<Hashed>(v[u]))], 1u);
   }
   __syncthreads();
   for (uint32_t p = threadIdx.x; p < fan; p += blockDim.x) hist[c * fan + p] = h[p];
@@ -418,6 +426,7 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
   const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block();  // as part_hist_kernel
   uint64_t lo, hi, pbase;
   if (!seg_range(sg, c, chunk, m, fan, lo, hi, pbase)) return;  // block-uniform, before any barrier
+  const Digit digit(shift, fan);
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   const int ln = lane();
   const uint64_t lt = (ln == 0) ? 0ull : (~0ull >> (64 - ln));  // lanes below this one
@@ -533,17 +542,19 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
     if constexpr (Stable) {
 #pragma unroll
       for (int j0 = 0; j0 < I; j0 += kRankItems) {
+        uint32_t d[kRankItems];
         uint32_t plo[kRankItems], phi[kRankItems];  // lanes of the slice with this lane's digit
 #pragma unroll
         for (int j = 0; j < kRankItems; ++j) {
           const uint64_t valid = ballot(static_cast<uint32_t>((j0 + j) * kWave + ln) < wn);
+          d[j] = digit(k[j0 + j]);
           plo[j] = static_cast<uint32_t>(valid);
           phi[j] = static_cast<uint32_t>(valid >> 32);
         }
         for (uint32_t b = 0; b < bits; ++b) {
 #pragma unroll
           for (int j = 0; j < kRankItems; ++j) {
-            const uint32_t one = 0u - digit_of(k[j0 + j], shift + b, 1u);  // all ones where the digit's bit b is set
+            const uint32_t one = 0u - ((d[j] >> b) & 1u);  // all ones where the digit's bit b is set
             const uint64_t set = ballot(one != 0);
             plo[j] &= ~(static_cast<uint32_t>(set) ^ one);
             phi[j] &= ~(static_cast<uint32_t>(set >> 32) ^ one);
@@ -551,13 +562,12 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
         }
 #pragma unroll
         for (int j = 0; j < kRankItems; ++j) {
-          const uint32_t d = digit_of(k[j0 + j], shift, fan - 1);
           const uint32_t before = static_cast<uint32_t>(__popc(plo[j] & static_cast<uint32_t>(lt)) +
                                                         __popc(phi[j] & static_cast<uint32_t>(lt >> 32)));
           const bool valid = static_cast<uint32_t>((j0 + j) * kWave + ln) < wn;
-          const uint32_t at = mine[d];  // every lane of the group reads the count before its first lane moves it
+          const uint32_t at = mine[d[j]];  // every lane of the group reads the count before its first lane moves it
           rk[j0 + j] = at + before;
-          if (valid && before == 0) mine[d] = static_cast<uint16_t>(at + __popc(plo[j]) + __popc(phi[j]));
+          if (valid && before == 0) mine[d[j]] = static_cast<uint16_t>(at + __popc(plo[j]) + __popc(phi[j]));
           __builtin_amdgcn_wave_barrier();
         }
       }
@@ -565,7 +575,7 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
 #pragma unroll
       for (int j = 0; j < I; ++j) {
         rk[j] = 0;
-        if (static_cast<uint32_t>(j * kWave + ln) < wn) rk[j] = atomicAdd(&cnt[digit_of(k[j], shift, fan - 1)], 1u);
+        if (static_cast<uint32_t>(j * kWave + ln) < wn) rk[j] = atomicAdd(&cnt[digit(k[j])], 1u);
       }
     }
     __syncthreads();
@@ -578,7 +588,7 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
 #pragma unroll
     for (int j = 0; j < I; ++j) {
       if (static_cast<uint32_t>(j * kWave + ln) < wn) {
-        const uint32_t d = digit_of(k[j], shift, fan - 1);
+        const uint32_t d = digit(k[j]);
         uint32_t slot;
         if constexpr (Stable) slot = off[d] + mine[d] + rk[j];
         else slot = cnt[d] + rk[j];
@@ -607,7 +617,7 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
       const uint32_t t = static_cast<uint32_t>(j * B) + threadIdx.x;
       if (t < n) {
         const K kk = sk[t];
-        const uint32_t pos = base[digit_of(kk, shift, fan - 1)] + t;
+        const uint32_t pos = base[digit(kk)] + t;
         if (pos < cap) {  // always true for a consistent histogram
           out_keys[pos] = kk;
           if (out_payload) out_payload[pos] = sp[t];
