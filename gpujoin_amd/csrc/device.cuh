@@ -116,6 +116,12 @@ template <class K>
 __device__ __forceinline__ Piece<K> load_piece(const K* p) {
   return piece_of<K>(*reinterpret_cast<const u32x4*>(p));
 }
+// The same from any key's address (a global load asks for four-byte alignment only).
+typedef u32x4 u32x4_at_key __attribute__((aligned(4)));
+template <class K>
+__device__ __forceinline__ Piece<K> load_piece_any(const K* p) {
+  return piece_of<K>(*reinterpret_cast<const u32x4_at_key*>(p));
+}
 
 template <class K>
 __device__ __forceinline__ constexpr K key_max() {

@@ -55,6 +55,12 @@ struct QuadLine {
 #pragma unroll
     for (int t = 0; t < kPieces; ++t) pc[t] = load_piece(p + t * kPiece);
   }
+  // keys at .. at + kKeys - 1 of a column, aligned or not
+  __device__ __forceinline__ void load_keys(const K* lane_base, uint32_t at) {
+    const K* p = lane_base + at;
+#pragma unroll
+    for (int t = 0; t < kPieces; ++t) pc[t] = load_piece_any(p + t * kPiece);
+  }
   // whatever the registers hold, for the rounds that then load nothing and whose count is
   // not looked at; all of a step's calls come before its loads, whose registers these are
   __device__ __forceinline__ void any() {
@@ -114,35 +120,55 @@ __device__ __forceinline__ uint32_t quad_count_less(const K* base, uint32_t line
   return quad_below(ln, q, ql);
 }
 
-// The partial last line of a column of n keys holds fewer keys than a quad reads: the lane
-// walks it by itself, from position `at`.
-template <class K>
-__device__ __forceinline__ uint32_t tail_below(const K* col, uint64_t n, uint64_t at, K x, bool& eq) {
-  uint32_t b = 0;
-  while (at + b < n && col[at + b] < x) ++b;
-  eq = at + b < n && col[at + b] == x;
-  return b;
+// Where the keys of a column's line are read from: a partial last line is read together with
+// the keys before it, as the last kKeys keys of the column (n >= kKeys).  A lane that walked
+// the partial line by itself, key by key, held its wave up: 2^14 probes of 8181 keys, B-tree
+// u32 6.2 us, now 4.6; learned u32 6.6, now 4.6.
+template <int kKeys>
+__device__ __forceinline__ uint32_t line_at(uint32_t line, uint64_t n) {
+  const uint32_t last = static_cast<uint32_t>(n) - kKeys;
+  return line * kKeys < last ? line * kKeys : last;
+}
+
+// Position of each lane's probe in a column of n < QuadLine::kKeys keys, or not found: a
+// quad reads the column once for its four probes, padded with key_max.
+template <class K, int NB>
+__device__ __forceinline__ uint32_t quad_find_short(const K* col, uint64_t n, bool live, const QuadProbes<K>& q,
+                                                    int ql) {
+  using L = QuadLine<K, NB>;
+  const uint32_t valid = static_cast<uint32_t>(n);
+  L ln;
+#pragma unroll
+  for (int t = 0; t < L::kPieces; ++t)
+#pragma unroll
+    for (int j = 0; j < L::kPiece; ++j) {
+      const uint32_t i = static_cast<uint32_t>(ql * L::kLaneKeys + t * L::kPiece + j);
+      ln.pc[t].k[j] = i < valid ? col[i] : key_max<K>();
+    }
+  uint32_t c = 0, e = 0;
+#pragma unroll
+  for (int r = 0; r < kQuad; ++r) {
+    c |= ln.below(q.x[r]) << (8 * r);
+    e |= ln.holds(q.x[r]) ? 1u << r : 0u;
+  }
+  c = (quad_sum(c) >> (8 * ql)) & 0xFFu;
+  e = (quad_or(e) >> ql) & 1u;
+  return (live && e != 0 && c < valid) ? c : kNotFound;  // the padding is no match
 }
 
 // Position of each lane's probe in its NB-byte chunk of the column, or not found.
 template <class K, int NB>
-__device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, uint32_t chunk, bool live, K x,
+__device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, uint32_t chunk, bool live,
                                                     const QuadProbes<K>& q, int ql) {
   using L = QuadLine<K, NB>;
-  const uint64_t at = static_cast<uint64_t>(chunk) * L::kKeys;
-  const bool tail = chunk >= n / L::kKeys;  // the column's partial last chunk
-  const uint32_t whole = tail ? 0u : chunk;
-  uint32_t below = 0;
-  bool eq = false;
-  if (n >= static_cast<uint64_t>(L::kKeys)) {  // kernel-uniform: there is a whole chunk to read
-    L ln[kQuad];
-    const K* lane_base = col + ql * L::kLaneKeys;
-    quad_rounds([&](auto r) { ln[r].load(lane_base, quad_bcast<r>(whole)); });
-    below = quad_below(ln, q, ql);
-    eq = quad_holds(ln, q, ql);
-  }
-  if (tail && live) below = tail_below(col, n, at, x, eq);
-  return (live && eq) ? static_cast<uint32_t>(at + below) : kNotFound;
+  if (n < static_cast<uint64_t>(L::kKeys)) return quad_find_short<K, NB>(col, n, live, q, ql);  // kernel-uniform
+  const uint32_t at = line_at<L::kKeys>(chunk, n);
+  L ln[kQuad];
+  const K* lane_base = col + ql * L::kLaneKeys;
+  quad_rounds([&](auto r) { ln[r].load_keys(lane_base, quad_bcast<r>(at)); });
+  const uint32_t below = quad_below(ln, q, ql);
+  const bool eq = quad_holds(ln, q, ql);
+  return (live && eq) ? at + below : kNotFound;
 }
 
 // ---------------------------------------------------------------------------
@@ -236,8 +262,9 @@ struct BSearchDev {
     return (p < hi && col[p] == x) ? static_cast<uint32_t>(p) : kNotFound;
   }
 
-  // Lines of the bucket [first, last] by quads.  klo, khi: the keys before the bucket (the
-  // column's first key for the first bucket) and at its end, klo < x <= khi.
+  // Whole lines of the bucket [first, last] by quads.  klo, khi: the keys before the bucket
+  // (the column's first key for the first bucket) and at its end, klo < x <= khi.  The
+  // column's partial last line is left to the halving.
   __device__ __forceinline__ void narrow(K x, K klo, K khi, bool inner, bool& open, uint32_t& first, uint32_t& last,
                                          uint32_t& found) const {
     const int ql = lane() & (kQuad - 1);
@@ -247,32 +274,36 @@ struct BSearchDev {
     uint32_t plo = inner && first > 0 ? first - 1 : 0u, phi = last;
     open = open && klo <= x;
     uint32_t line_lo = first / LK, line_hi = last / LK;
+    bool bounded = line_hi < whole;     // x is in no line behind line_hi
+    bool go = open && line_lo < whole;  // lines to look at
+    line_hi -= !bounded && go ? 1u : 0u;
     uint32_t line = guess(x, klo, khi, plo, phi) / LK;
     line = line < line_lo ? line_lo : (line > line_hi ? line_hi : line);
-    for (int t = 1; t <= kGuesses + 1 && ballot(open) != 0; ++t) {  // wave-uniform
-      const bool tail = open && line >= whole;  // the column's partial last line
-      const uint32_t rounds = quad_or(open && !tail ? 1u << ql : 0u);
+    for (int t = 1; t <= kGuesses + 1 && ballot(go) != 0; ++t) {  // wave-uniform
+      const uint32_t rounds = quad_or(go ? 1u << ql : 0u);
       L ln[kQuad];
       quad_rounds([&](auto r) { ln[r].any(); });
       quad_rounds([&](auto r) {
         const uint32_t l = quad_bcast<r>(line);
         if ((rounds >> r) & 1u) ln[r].load(lane_base, l);
       });
-      uint32_t below = quad_below(ln, q, ql);
-      bool eq = quad_holds(ln, q, ql);
-      if (tail) below = tail_below(col, n, static_cast<uint64_t>(line) * LK, x, eq);
-      if (open) {
+      const uint32_t below = quad_below(ln, q, ql);
+      const bool eq = quad_holds(ln, q, ql);
+      if (go) {
         const uint32_t base = line * LK;
-        const bool right = !tail && below == LK;  // every key of the line is below x
+        const bool right = below == LK;  // every key of the line is below x
         if (right) {
-          open = line < line_hi;
+          go = line < line_hi;
+          open = go || !bounded;
           line_lo = line + 1;
         } else {
           found = eq ? base + below : found;
-          open = below == 0 && line > line_lo;
+          go = below == 0 && line > line_lo;
+          open = go;
           line_hi = line - 1;
+          bounded = true;
         }
-        if (open) {
+        if (go) {
           line = right ? line_lo : line_hi;
           if (t < kGuesses) {  // wave-uniform
             const uint32_t at = right ? base + LK - 1 : base;  // the edge of the line on x's side
@@ -289,7 +320,7 @@ struct BSearchDev {
     }
     const uint32_t a = line_lo * LK, z = line_hi * LK + LK - 1;
     first = a > first ? a : first;
-    last = z < last ? z : last;
+    last = bounded && z < last ? z : last;
   }
 };
 
@@ -367,7 +398,7 @@ struct BTreeDev {
     uint32_t lvl = lds_levels;
     for (; lvl < levels; ++lvl)
       descend(node, live, quad_count_less<K, NB>(nodes + level_off[lvl] * NK, node, q, ql), lvl);
-    return quad_find_equal<K, NB>(col, n, node, live, x, q, ql);
+    return quad_find_equal<K, NB>(col, n, node, live, q, ql);
   }
 };
 

@@ -128,9 +128,10 @@ struct HarmoniaDev {
 //
 // A round's line is sorted, so the owning lane only needs how many of its keys are
 // below the probe (the in-line offset of the probe's lower bound) and whether the
-// line holds it.  The owning lane alone holds its probe's state (line, window,
-// direction), which keeps the registers per lane, and hence the waves per SIMD,
-// where a latency-bound search needs them.  Positions are 32-bit (n < 2^32).
+// line holds it.  The owning lane alone holds its probe's state (line and window; a step
+// to one side takes the other side's part of the window away), which keeps the registers
+// per lane, and hence the waves per SIMD, where a latency-bound search needs them.
+// Positions are 32-bit (n < 2^32).
 // ---------------------------------------------------------------------------
 template <class K>
 __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n, uint32_t my_pred, uint32_t my_lo,
@@ -140,40 +141,33 @@ __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n
   const int ql = lane() & (kQuad - 1);
   const QuadProbes<K> q(my_x);
   const K* lane_base = col + ql * L::kLaneKeys;
-  const uint32_t whole = static_cast<uint32_t>(n / LK);  // whole lines of the column
   bool open = my_live && my_lo < my_hi;
+  if (n < LK) return quad_find_short<K, 128>(col, n, open, q, ql);  // kernel-uniform
   uint32_t line = 0, found = kNotFound;
   if (open) {
     const uint32_t p = my_pred < my_lo ? my_lo : (my_pred >= my_hi ? my_hi - 1 : my_pred);
     line = p / LK;
   }
-  const uint32_t first_line = my_lo / LK, last_line = open ? (my_hi - 1) / LK : 0u;
-  int dir = 0;  // 0: first line, -1 walking left, +1 walking right
   while (ballot(open) != 0) {  // wave-uniform exit
-    const bool tail = open && line >= whole;  // the column's partial last line
-    const uint32_t rounds = quad_or(open && !tail ? 1u << ql : 0u);
+    const uint32_t rounds = quad_or(open ? 1u << ql : 0u), base = line_at<LK>(line, n);
     L ln[kQuad];
     quad_rounds([&](auto r) { ln[r].any(); });
     quad_rounds([&](auto r) {
-      const uint32_t l = quad_bcast<r>(line);
-      if ((rounds >> r) & 1u) ln[r].load(lane_base, l);
+      const uint32_t at = quad_bcast<r>(base);
+      if ((rounds >> r) & 1u) ln[r].load_keys(lane_base, at);
     });
-    uint32_t below = quad_below(ln, q, ql);
-    bool eq = quad_holds(ln, q, ql);
-    if (tail) below = tail_below(col, n, static_cast<uint64_t>(line) * LK, my_x, eq);
+    const uint32_t below = quad_below(ln, q, ql);
+    const bool eq = quad_holds(ln, q, ql);
     if (open) {
-      const uint32_t base = line * LK;
-      const uint32_t a = my_lo > base ? my_lo - base : 0u;               // window slots of this line: [a, c)
-      const uint32_t c = my_hi - base < LK ? my_hi - base : LK;
       if (eq) {
         found = base + below;  // the line holds x at its lower-bound offset
         open = false;
-      } else if (below >= c && dir >= 0 && line < last_line) {
-        ++line;  // every window key of the line is below x: only the right can hold it
-        dir = 1;
-      } else if (below <= a && dir <= 0 && line > first_line) {
-        --line;  // no window key of the line is below x: only the left can hold it
-        dir = -1;
+      } else if (below == LK && my_hi - base > LK) {
+        ++line;  // every key of the line is below x, and the window goes on to the right
+        my_lo = 0xFFFFFFFFu;  // and not back to the left
+      } else if (below == 0 && base > my_lo) {
+        --line;  // no key of the line is below x, and the window begins further left
+        my_hi = base;
       } else {
         open = false;  // x falls between two window keys (or past the window): absent
       }
