@@ -148,7 +148,7 @@ __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n
     const uint32_t p = my_pred < my_lo ? my_lo : (my_pred >= my_hi ? my_hi - 1 : my_pred);
     line = p / LK;
   }
-  while (ballot(open) != 0) {  // wave-uniform exit
+  while (const uint64_t lanes = ballot(open)) {  // wave-uniform exit
     const uint32_t rounds = quad_or(open ? 1u << ql : 0u), base = line_at<LK>(line, n);
     L ln[kQuad];
     quad_rounds([&](auto r) { ln[r].any(); });
@@ -156,8 +156,8 @@ __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n
       const uint32_t at = quad_bcast<r>(base);
       if ((rounds >> r) & 1u) ln[r].load_keys(lane_base, at);
     });
-    const uint32_t below = quad_below(ln, q, ql);
-    const bool eq = quad_holds(ln, q, ql);
+    const uint32_t below = quad_below(ln, q, ql, lanes);
+    const bool eq = quad_holds(ln, q, ql, lanes);
     if (open) {
       if (eq) {
         found = base + below;  // the line holds x at its lower-bound offset
