@@ -1231,7 +1231,7 @@ void enqueue_plan(gj_batch_plan& pl, hipStream_t s, GraphLanes* gl = nullptr) {
         }
         if (gl) GJ_HIP_CHECK(gl->join(s));
       }
-    });
+    }, kLinesAggregates);
     return;
   }
   dispatch_key(ix.key_bytes, [&]<class K>() {
@@ -1257,11 +1257,14 @@ void enqueue_plan(gj_batch_plan& pl, hipStream_t s, GraphLanes* gl = nullptr) {
         for (size_t i = 0; i < pl.probe.size(); ++i) {
           const ProbeBatchDev& b = pl.probe[i];
           const hipStream_t ls = lanes ? (*lanes)[i % lanes->size()] : s;
-          launch_plain(d, static_cast<const K*>(b.probes), b.m, b.out, lp, ls, ix.cu);
+          if (few_halvings(ix, b.m))
+            launch_plain(ix.bsearch_dev<K, false>(), static_cast<const K*>(b.probes), b.m, b.out, lp, ls, ix.cu);
+          else
+            launch_plain(d, static_cast<const K*>(b.probes), b.m, b.out, lp, ls, ix.cu);
         }
         if (gl) GJ_HIP_CHECK(gl->join(s));
       }
-    });
+    }, pl.mode == GJ_BATCH_PERSISTENT ? kLinesBatches : kLinesLookups);
   });
 }
 
@@ -1351,7 +1354,7 @@ int gj_join_aggregate(const gj_index* index, const gj_fact_batch* batch, const g
       partial.reserve(agg_partial_cap(index->cu) * sizeof(AggPartial));
       launch_join_agg_strategy(params->strategy, d, b, params->date_lo, params->date_hi, params->d_flag, index->cu,
                                partial.as<AggPartial>(), s);
-    });
+    }, kLinesAggregates);
   });
 }
 
@@ -1369,7 +1372,7 @@ int gj_join_aggregate_noalloc(const gj_index* index, const gj_fact_batch* batch,
     with_index_dev<uint32_t>(*index, [&](auto d) {
       launch_join_agg_strategy(params->strategy, d, b, params->date_lo, params->date_hi, params->d_flag, index->cu,
                                partial, S(stream), kNoAllocPartials);
-    });
+    }, kLinesAggregates);
   });
 }
 

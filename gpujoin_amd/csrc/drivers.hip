@@ -153,7 +153,7 @@ void lookup_partitioned(const gj_index& ix, const K* probes, uint64_t m, uint32_
     with_index_dev<K>(ix, [&](auto d) {
       launch_tuples(d, tkeys, start, together ? static_cast<uint32_t>(nw) : 1u, together ? fan : nw * fan,
                     together ? windows_capacity(std::min(bm, window), window, sizeof(K), bits) : cap_b, res, tp, s, ix.cu);
-    });
+    }, (ix.n >> bits) > kLinesTupleKeys ? kLinesLookups : ~0ull);
     launch_unpartition(inv1, inv2, res, cap_b, bm, out + b0, s, ix.cu);
   }
 }
@@ -176,9 +176,6 @@ void lookup_hash_join(const gj_index& ix, const K* probes, uint64_t m, uint32_t*
 
 }  // namespace
 
-// Binary search goes by lines from this many halvings over all probes on.
-constexpr uint64_t kLinesMinHalvings = 5ull << 18;
-
 void lookup_dispatch(const gj_index& ix, const void* probes, uint64_t m, uint32_t* out, const gj_lookup_params& p,
                      hipStream_t s) {
   dispatch_key(ix.key_bytes, [&]<class K>() {
@@ -195,10 +192,7 @@ void lookup_dispatch(const gj_index& ix, const void* probes, uint64_t m, uint32_
           launch_marked(ix.btree_dev<K>(), pk, m, out, p, s, ix.cu);
           return;
         }
-        // Few probes over small buckets wait for the longest chain of loads, and halving's loads hit
-        // the L1 from the third last on: 2^16 probes of 2^18 u64 keys 5.1 us, by lines 5.5;
-        // 2^17 8.2 and 6.7; 2^16 of 2^22 keys 9.7 and 7.2; 2^17 of 2^18 u32 keys 7.9 and 9.1.
-        if (ix.kind == GJ_BINARY_SEARCH && m * ilog2_ceil(ix.sample_step) < kLinesMinHalvings) {
+        if (few_halvings(ix, m)) {
           launch_plain(ix.bsearch_dev<K, false>(), pk, m, out, p, s, ix.cu);
           return;
         }

@@ -193,10 +193,10 @@ __device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, ui
 // What bounds it: fabric lines (about 52 G/s).  Halving alone touches log2(bucket bytes /
 // 128) + 1 lines per probe, one dependent load each; in a bucket of evenly spread keys the
 // first guess is off by sqrt(bucket) / 3 keys on average and the second finds the line.
-// It stays for buckets of at most kHalve keys (Lines = false: two or three loads of a line
-// that is in reach anyway: 2^24 probes of 2^12 u32 keys 118 us, by quads 170), and for waves whose
-// probes all lie in about one bucket, whose lanes share their loads (sorted probes over
-// 2^22 u64 keys 216 us, by quads 402).
+// It stays for small buckets (Lines = false: two or three loads of a line that is in reach
+// anyway: 2^24 probes of 2^12 u32 keys 118 us, by quads 170; with_index_dev says how small), and
+// for waves whose probes all lie in about one bucket, whose lanes share their loads (sorted
+// probes over 2^22 u64 keys 216 us, by quads 402).
 // 2^24 uniform probes, halving alone -> by lines, us: 2^16 u64 keys 522 -> 220, 2^20 1032 ->
 // 307, 2^22 2357 -> 505, 2^24 3560 -> 667; u32 2^22 1897 -> 329; behind the blockwise sort,
 // 2^22 u64 1261 -> 829.
@@ -206,7 +206,6 @@ struct BSearchDev {
   using L = QuadLine<K, 128>;
   static constexpr uint32_t LK = L::kKeys;
   static constexpr int kGuesses = 2;  // interpolated lines, then one neighbour
-  static constexpr uint32_t kHalve = 8;
   const K* col;
   uint64_t n;
   const K* samples;  // 2^sample_bits bucket maxima (key_max for empty buckets)

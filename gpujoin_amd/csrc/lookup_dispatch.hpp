@@ -116,12 +116,35 @@ void build_index(gj_index& ix, hipStream_t s);
 template <class K> void build_btree(gj_index& ix, hipStream_t s);
 template <class K> void build_extended(gj_index& ix, hipStream_t s);
 
+// Binary search reads lines in buckets of more keys than this, and halves alone in smaller
+// ones.  Lines cost instructions and registers and save dependent loads, so the line lies
+// where a caller's waves are full and wait for those loads (halving -> lines, us):
+//   lookups    2^22 probes, plain: buckets of 9 u32 keys 64 -> 55, of 9 u64 keys 100 -> 56
+//   batches    64 batches of 64 to 70000 probes in one persistent launch: buckets of 65 u32
+//              keys 66 -> 68, of 257 keys 77 -> 68; u64 65 keys 74 -> 63, 9 keys 57 -> 63
+//   aggregates one or two probes a wave (plain strategy, 30 M rows): buckets of 257 u32 keys 203
+//              -> 227, of 1025 keys 239 -> 224; lane_refill, 257 keys, 61 -> 54
+//   tuples     the tuples of a partition share the lines of its keys, so it is the keys per
+//              partition that count: 2^22 probes, windows of 2^20, of 1024 keys (2^18 u32 keys, fan-out
+//              2^8) 116 -> 119, of 4096 keys (2^22, 2^10) 175 -> 158, of 2^16 (2^20, 2^4) 215 -> 111;
+//              u64 of 256 keys (2^18, 2^10) 139 -> 144, of 4096 208 -> 205, of 2^16 234 -> 125
+constexpr uint64_t kLinesLookups = 8, kLinesBatches = 128, kLinesAggregates = 512, kLinesTupleKeys = 1024;
+
+// Few probes over small buckets wait for the longest chain of loads, and halving's loads hit
+// the L1 from the third last on: binary search of one batch goes by lines from this many
+// halvings over all its probes on.  2^16 probes of 2^18 u64 keys 5.1 us, by lines 5.5; 2^17
+// 8.2 and 6.7; 2^16 of 2^22 keys 9.7 and 7.2; 2^17 of 2^18 u32 keys 7.9 and 9.1.
+constexpr uint64_t kLinesMinHalvings = 5ull << 18;
+inline bool few_halvings(const gj_index& ix, uint64_t m) {
+  return ix.kind == GJ_BINARY_SEARCH && m * ilog2_ceil(ix.sample_step) < kLinesMinHalvings;
+}
+
 // Calls f(descriptor) with the device descriptor of the index (every kind).
 template <class K, class F>
-void with_index_dev(const gj_index& ix, F&& f) {
+void with_index_dev(const gj_index& ix, F&& f, uint64_t lines_above = kLinesLookups) {
   switch (ix.kind) {
     case GJ_BINARY_SEARCH:
-      if (ix.sample_step > BSearchDev<K>::kHalve)
+      if (ix.sample_step > lines_above)
         f(ix.bsearch_dev<K, true>());
       else
         f(ix.bsearch_dev<K, false>());
