@@ -147,12 +147,18 @@ void lookup_partitioned(const gj_index& ix, const K* probes, uint64_t m, uint32_
     // u64 keys and probes, fan-out 2^9, windows of 2^16 / 2^18 / 2^20 probes: B-tree 1621 / 1368 /
     // 1267 -> 1245 / 1197 / 1181 us, learned 1187 / 1149 / 1029 -> 957 / 934 / 933).  Denser
     // windows find their lines in L2 either way and go one after the other (2^20 keys, windows
-    // of 2^21: learned 798 us, together 843).
+    // of 2^21: learned 798 us, together 843); so do windows that are less than a workgroup's tile
+    // for each XCD, whose workgroups would be mostly idle (2^20 keys, fan-out 2, windows of 64:
+    // binary search 659 us together, 326 one after the other and without tiles for more padding
+    // than there can be).
     const uint64_t nw = ceil_div(bm, window);
-    const bool together = window <= ix.n * sizeof(K) / 128;
+    const bool together = window <= ix.n * sizeof(K) / 128 && window >= 8 * lookup_block(tp);
     with_index_dev<K>(ix, [&](auto d) {
-      launch_tuples(d, tkeys, start, together ? static_cast<uint32_t>(nw) : 1u, together ? fan : nw * fan,
-                    together ? windows_capacity(std::min(bm, window), window, sizeof(K), bits) : cap_b, res, tp, s, ix.cu);
+      if (together)
+        launch_tuples(d, tkeys, start, static_cast<uint32_t>(nw), fan,
+                      windows_tuples(std::min(bm, window), window, sizeof(K), bits), res, tp, s, ix.cu);
+      else
+        launch_tuples(d, tkeys, start, 1u, nw * fan, windows_tuples(bm, window, sizeof(K), bits), res, tp, s, ix.cu);
     }, (ix.n >> bits) > kLinesTupleKeys ? kLinesLookups : ~0ull);
     launch_unpartition(inv1, inv2, res, cap_b, bm, out + b0, s, ix.cu);
   }

@@ -203,6 +203,8 @@ uint64_t partition_scratch(uint64_t m, int key_bytes, uint32_t bits, uint32_t pa
 // inv2[inv1[i]] its final position (inv2 is null otherwise).  inv1 and inv2 hold m
 // entries each.
 uint64_t windows_capacity(uint64_t m, uint64_t window, int key_bytes, uint32_t bits);
+// what of it the tuples, padding included, can take (each tuple pads one partition at most)
+uint64_t windows_tuples(uint64_t m, uint64_t window, int key_bytes, uint32_t bits);
 uint64_t windows_scratch(uint64_t m, uint64_t window, int key_bytes, uint32_t bits, uint32_t passes);
 bool windows_two_pass(uint32_t bits, uint32_t passes);
 template <class K>

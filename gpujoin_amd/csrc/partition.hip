@@ -957,6 +957,10 @@ uint64_t windows_capacity(uint64_t m, uint64_t window, int key_bytes, uint32_t b
   return m + ceil_div(m, window) * (1ull << bits) * part_align(key_bytes);
 }
 
+uint64_t windows_tuples(uint64_t m, uint64_t window, int key_bytes, uint32_t bits) {
+  return std::min<uint64_t>(windows_capacity(m, window, key_bytes, bits), m * part_align(key_bytes));
+}
+
 uint64_t windows_scratch(uint64_t m, uint64_t window, int key_bytes, uint32_t bits, uint32_t passes) {
   return win_layout(m, window, key_bytes, bits, passes).bytes;
 }
