@@ -13,13 +13,13 @@ namespace gj {
 // reason, :235) with 64-bit indices (the reference uses int, which limits it
 // to 2^31 probes).
 //
-// kMinWaves: waves per SIMD that the registers are cut to.  Binary search by lines over u32
-// keys fits 64 registers without a spill (65 by itself: 7 waves; sorted probes over 2^22 keys
-// 201 -> 183 us), the learned column layout over u32 keys too (2^20 keys: 2^24 uniform
-// probes 218 -> 215 us, sorted 148 -> 138); over u64 keys the cut spills (505 -> 669 and
-// 256 -> 303 us), as it does for RadixSpline and Harmonia.
+// kMinWaves: waves per SIMD that the registers are cut to.  Binary search by lines fits 64
+// registers without a spill (u64 keys 66 by itself: 7 waves, and one more round of workgroups
+// where 8 waves take a million probes in two); the learned column layout over u32 keys fits by
+// itself and is held there.  RadixSpline and Harmonia spill under the cut (405 -> 498 and 391
+// -> 452 us).
 template <class Dev> constexpr int kMinWaves = 1;
-template <> inline constexpr int kMinWaves<BSearchDev<uint32_t, true>> = 8;
+template <class K> inline constexpr int kMinWaves<BSearchDev<K, true>> = 8;
 template <> inline constexpr int kMinWaves<LearnedDev<uint32_t, kLeafNoFallback>> = 8;
 template <class Dev, class K>
 __global__ __launch_bounds__(256, kMinWaves<Dev>) void lookup_plain_kernel(Dev d, const K* __restrict__ probes, uint64_t m,

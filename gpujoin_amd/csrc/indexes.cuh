@@ -205,7 +205,7 @@ template <class K, bool Lines = true>
 struct BSearchDev {
   using L = QuadLine<K, 128>;
   static constexpr uint32_t LK = L::kKeys;
-  static constexpr int kGuesses = 2;  // interpolated lines, then one neighbour
+  static constexpr int kGuesses = 2;  // interpolated lines (the second between the first and the bucket), then one neighbour
   const K* col;
   uint64_t n;
   const K* samples;  // 2^sample_bits bucket maxima (key_max for empty buckets)
@@ -242,18 +242,24 @@ struct BSearchDev {
     } else {
       bool open = active && b < nb && lo < n;
       // x's position is in [first, last], or last + 1 where found holds it already
-      uint32_t first = open ? static_cast<uint32_t>(lo) : 0u;
-      uint32_t last = open ? static_cast<uint32_t>((lo + step < n ? lo + step : n) - 1) : 0u;
+      uint32_t first = open ? bucket_first(b) : 0u, last = open ? bucket_last(b) : 0u;
       uint32_t found = kNotFound;
       const uint32_t b0 = __builtin_amdgcn_readfirstlane(b);
       if (ballot(open && (b > b0 + 1 || b + 1 < b0)) != 0)  // wave-uniform
-        narrow(x, b > 0 ? s[b - 1] : col[0], s[b < nb ? b : nb - 1], b > 0, open, first, last, found);
+        narrow(x, b, s, open, first, last, found);
       if (open) {
         const uint32_t r = halve(x, first, static_cast<uint64_t>(last - first) + 1, static_cast<uint64_t>(last) + 1);
         found = r != kNotFound ? r : found;
       }
       return found;
     }
+  }
+
+  // First and last position of bucket b, which begins inside the column.
+  __device__ __forceinline__ uint32_t bucket_first(uint32_t b) const { return b * static_cast<uint32_t>(step); }
+  __device__ __forceinline__ uint32_t bucket_last(uint32_t b) const {
+    const uint32_t lo = bucket_first(b);
+    return static_cast<uint32_t>(lo + step < n ? lo + step : n) - 1;
   }
 
   // Branch-free lower_bound over len keys from lo on; the row id if the key before hi is x.
@@ -268,24 +274,32 @@ struct BSearchDev {
     return (p < hi && col[p] == x) ? static_cast<uint32_t>(p) : kNotFound;
   }
 
-  // Whole lines of the bucket [first, last] by quads.  klo, khi: the keys before the bucket
-  // (the column's first key for the first bucket) and at its end, klo < x <= khi.  The
-  // column's partial last line is left to the halving.
-  __device__ __forceinline__ void narrow(K x, K klo, K khi, bool inner, bool& open, uint32_t& first, uint32_t& last,
+  // Whole lines of bucket b by quads; what is left of it is [first, last].  The column's
+  // partial last line is left to the halving.  The bucket's bounds are looked up again where
+  // they are needed: kept in registers, they cost u64 keys a wave per SIMD (70 registers, now
+  // 64), which sorted probes, whose waves do not come here, paid for (2^20 of them over 10^6
+  // keys: halving alone 11.4 us, with the bounds in registers 16.4, now 11.6).
+  __device__ __forceinline__ void narrow(K x, uint32_t b, const K* s, bool& open, uint32_t& first, uint32_t& last,
                                          uint32_t& found) const {
     const int ql = lane() & (kQuad - 1);
     const QuadProbes<K> q(x);
     const K* lane_base = col + ql * L::kLaneKeys;
     const uint32_t whole = static_cast<uint32_t>(n / LK);  // whole lines of the column
-    uint32_t plo = inner && first > 0 ? first - 1 : 0u, phi = last;
-    open = open && klo <= x;
-    uint32_t line_lo = first / LK, line_hi = last / LK;
+    if (!open) b = 0;
+    uint32_t line_lo = bucket_first(b) / LK, line_hi = bucket_last(b) / LK, line;
+    // klo < x <= khi: the keys before the bucket (the column's first key for the first one) and at its end
+    {
+      const K klo = b > 0 ? s[b - 1] : col[0];
+      open = open && klo <= x;
+      line = guess(x, klo, s[b], b > 0 ? bucket_first(b) - 1 : 0u, bucket_last(b)) / LK;
+    }
     bool bounded = line_hi < whole;     // x is in no line behind line_hi
     bool go = open && line_lo < whole;  // lines to look at
     line_hi -= !bounded && go ? 1u : 0u;
-    uint32_t line = guess(x, klo, khi, plo, phi) / LK;
     line = line < line_lo ? line_lo : (line > line_hi ? line_hi : line);
-    for (int t = 1; t <= kGuesses + 1 && ballot(go) != 0; ++t) {  // wave-uniform
+    for (int t = 1; t <= kGuesses + 1; ++t) {
+      const uint64_t lanes = ballot(go);
+      if (lanes == 0) break;  // wave-uniform
       const uint32_t rounds = quad_or(go ? 1u << ql : 0u);
       L ln[kQuad];
       quad_rounds([&](auto r) { ln[r].any(); });
@@ -293,8 +307,9 @@ struct BSearchDev {
         const uint32_t l = quad_bcast<r>(line);
         if ((rounds >> r) & 1u) ln[r].load(lane_base, l);
       });
-      const uint32_t below = quad_below(ln, q, ql);
-      const bool eq = quad_holds(ln, q, ql);
+      const uint32_t below = quad_below(ln, q, ql, lanes);
+      const bool eq = quad_holds(ln, q, ql, lanes);
+      asm volatile("" : "+v"(b));  // its bounds are read anew
       if (go) {
         const uint32_t base = line * LK;
         const bool right = below == LK;  // every key of the line is below x
@@ -314,10 +329,8 @@ struct BSearchDev {
           if (t < kGuesses) {  // wave-uniform
             const uint32_t at = right ? base + LK - 1 : base;  // the edge of the line on x's side
             const K edge = col[at];
-            klo = right ? edge : klo;
-            khi = right ? khi : edge;
-            plo = right ? at : plo;
-            phi = right ? phi : at;
+            const K klo = right ? edge : (b > 0 ? s[b - 1] : col[0]), khi = right ? s[b] : edge;
+            const uint32_t plo = right ? at : (b > 0 ? bucket_first(b) - 1 : 0u), phi = right ? bucket_last(b) : at;
             line = guess(x, klo, khi, plo, phi) / LK;
             line = line < line_lo ? line_lo : (line > line_hi ? line_hi : line);
           }
@@ -325,6 +338,8 @@ struct BSearchDev {
       }
     }
     const uint32_t a = line_lo * LK, z = line_hi * LK + LK - 1;
+    first = bucket_first(b);
+    last = bucket_last(b);
     first = a > first ? a : first;
     last = bounded && z < last ? z : last;
   }
