@@ -150,7 +150,7 @@ struct dbuf {
 
 inline hipStream_t S(gj_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
-inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
+constexpr uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 inline uint32_t ilog2_floor(uint64_t v) { return 63u - static_cast<uint32_t>(__builtin_clzll(v)); }
 inline uint32_t ilog2_ceil(uint64_t v) { return v <= 1 ? 0u : 64u - static_cast<uint32_t>(__builtin_clzll(v - 1)); }
 

@@ -29,13 +29,18 @@ inline unsigned lookup_block(const gj_lookup_params& p) {
 // kStageStep bytes of it a wave takes one more step for each (Harmonia's 15.9 KB at 2^20
 // u64 keys: 575 us with one step, 529 with four, 570 strided).  Never fewer workgroups
 // than fit on the chip at once, if there is a step for each.
+// HIP takes fewer than 2^32 threads in a launch, so beyond that many items waves take more steps.
 constexpr uint64_t kStageStep = 8192;
-inline uint64_t cover_blocks(uint64_t items, uint64_t per_block, size_t stage_bytes, uint64_t resident) {
+constexpr uint64_t max_blocks(unsigned threads) { return 0xFFFFFFFFull / threads / 8 * 8; }  // whole XCD rounds
+constexpr uint64_t cover_blocks(uint64_t items, uint64_t per_block, unsigned threads, size_t stage_bytes,
+                                uint64_t resident) {
   const uint64_t cover = ceil_div(items, per_block);
   const uint64_t steps = 1 + stage_bytes / kStageStep;
   const uint64_t blocks = std::max<uint64_t>(ceil_div(cover, steps), std::min<uint64_t>(cover, resident));
-  return std::min<uint64_t>(std::max<uint64_t>(blocks, 1), 0x7FFFFFFFull);
+  return std::min<uint64_t>(std::max<uint64_t>(blocks, 1), max_blocks(threads));
 }
+static_assert(cover_blocks(1ull << 40, 256, 256, 0, 2048) * 256 < 1ull << 32);
+static_assert(cover_blocks(0xFFFFFFFFull, 64, 64, 0, 2048) * 64 < 1ull << 32);
 
 template <class Dev, class K>
 void launch_plain(const Dev& d, const K* probes, uint64_t m, uint32_t* out, const gj_lookup_params& p, hipStream_t s,
@@ -46,7 +51,7 @@ void launch_plain(const Dev& d, const K* probes, uint64_t m, uint32_t* out, cons
   const void* fn = reinterpret_cast<const void*>(&lookup_plain_kernel<Dev, K>);
   const uint64_t blocks = p.grid_blocks
                               ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(m, block)))
-                              : cover_blocks(m, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
+                              : cover_blocks(m, block, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
   hipLaunchKernelGGL((lookup_plain_kernel<Dev, K>), dim3(static_cast<unsigned>(blocks)), dim3(block), lds, s, d,
                      probes, m, out);
   GJ_HIP_CHECK(hipGetLastError());
@@ -81,8 +86,8 @@ void launch_tuples(const Dev& d, const K* keys, const uint64_t* start, uint32_t 
   const uint64_t total = windows * window_max;
   uint64_t blocks = p.grid_blocks
                         ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(total, block)))
-                        : cover_blocks(total, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
-  if (blocks >= 8) blocks = ceil_div(blocks, 8) * 8;  // whole XCD rounds for the XCD-major chunk map
+                        : cover_blocks(total, block, block, lds, static_cast<uint64_t>(blocks_per_cu(fn, block, lds)) * cu);
+  if (blocks >= 8) blocks = std::min(ceil_div(blocks, 8) * 8, max_blocks(block));  // whole XCD rounds for the XCD-major chunk map
   const uint64_t groups = blocks % 8 == 0 ? 8 : 1;
   // a window's share of an XCD is rounded up to whole waves
   const uint64_t tiles = windows * ceil_div(ceil_div(window_max, groups) + kWave, block);
@@ -106,7 +111,7 @@ void launch_bws(const Dev& d, const K* probes, uint64_t m, uint32_t* out, const 
   const void* fn = reinterpret_cast<const void*>(&lookup_bws_kernel<Dev, K, kBwsTile>);
   const uint64_t blocks =
       p.grid_blocks ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(m, kBwsTile)))
-                    : cover_blocks(m, kBwsTile, 0, static_cast<uint64_t>(blocks_per_cu(fn, kBwsBlock, lds)) * cu);
+                    : cover_blocks(m, kBwsTile, kBwsBlock, 0, static_cast<uint64_t>(blocks_per_cu(fn, kBwsBlock, lds)) * cu);
   hipLaunchKernelGGL((lookup_bws_kernel<Dev, K, kBwsTile>), dim3(static_cast<unsigned>(blocks)), dim3(kBwsBlock), lds, s,
                      d, probes, m, shift, out);
   GJ_HIP_CHECK(hipGetLastError());
