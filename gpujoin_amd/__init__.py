@@ -192,6 +192,11 @@ def synchronize():
     check(_lib.call("gj_device_synchronize"))
 
 
+def release_cached():
+    """Gives the device memory kept of dropped indexes back to the device."""
+    check(_lib.call("gj_release_cached"))
+
+
 def index_params(**kw) -> IndexParams:
     p = IndexParams()
     _lib.call("gj_index_params_default", C.byref(p))

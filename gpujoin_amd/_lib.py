@@ -152,6 +152,7 @@ SIGNATURES = {
     "gj_device_info": (_I, [C.c_char_p, C.c_size_t, C.POINTER(_I), C.POINTER(_I)]),
     "gj_malloc": (_I, [C.POINTER(_P), _U64]),
     "gj_free": (_I, [_P]),
+    "gj_release_cached": (_I, []),
     "gj_host_malloc": (_I, [C.POINTER(_P), _U64]),
     "gj_host_free": (_I, [_P]),
     "gj_memcpy_htod": (_I, [_P, _P, _U64, _P]),

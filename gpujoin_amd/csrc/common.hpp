@@ -61,6 +61,9 @@ int guarded(F&& f) {
 // Device blocks that released buffers leave for later ones (runtime.hip).  take: a block of
 // at least `bytes` on the current device, its true size in `cap`; its contents are
 // arbitrary.  give: waits for the device, like hipFree, and keeps or frees the block.
+// alloc: memory from outside the pool, which hipFree frees; the kept blocks go back to the
+// device before it (or take) reports that there is none.
+void* device_alloc(size_t bytes);
 void* device_take(size_t bytes, size_t& cap, int& dev);
 void device_give(void* p, size_t cap, int dev) noexcept;
 
@@ -112,7 +115,7 @@ struct dbuf {
     if (pooled)
       p = device_take(b, cap, dev);
     else
-      GJ_HIP_CHECK(hipMalloc(&p, b));
+      p = device_alloc(b);
     bytes = b;
   }
   // grow-only reallocation for reusable scratch

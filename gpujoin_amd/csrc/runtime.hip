@@ -4,8 +4,8 @@
 #include <mutex>
 #include <string>
 #include <unordered_map>
-#include <vector>
 
+#include "block_pool.hpp"
 #include "common.hpp"
 #include "device.cuh"
 #include "lookup_dispatch.hpp"
@@ -31,10 +31,8 @@ int device_cu_count() {
 // A program that indexes a build side for each query allocates and frees the same sizes
 // over and over, and hipFree of device memory settles at 4.1 ms a call after some hundreds
 // of such calls (0.25 ms before): building, probing once and dropping a learned index over
-// 12.3 M u64 keys took 4.43 ms, and with the pool takes 3.99.
+// 12.3 M u64 keys took 4.43 ms, and with the pool took 3.99.
 //
-// Kept: blocks of up to kPoolBlock bytes, at most kPoolBytes and kPoolBlocks of them in all;
-// the oldest go back to the device first, and all of them do before an allocation fails.
 // A block enters only after the device is idle, so whichever thread and stream takes it
 // next finds nothing in flight on it.  The wait is the one that hipFree makes, on a small
 // allocation (1 us for the pair): hipDeviceSynchronize would end another thread's graph
@@ -42,97 +40,46 @@ int device_cu_count() {
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr size_t kPoolBytes = 512ull << 20;
-constexpr size_t kPoolBlock = kPoolBytes / 2;
-constexpr size_t kPoolBlocks = 64;
-
-struct DevicePool {
-  struct Block {
-    void* p;
-    size_t cap;
-    int dev;
-  };
-  std::mutex mu;
-  std::vector<Block> blocks;  // oldest first
-  size_t held = 0;
-
-  void* find(size_t cap, int dev) {
-    std::lock_guard<std::mutex> g(mu);
-    for (size_t i = blocks.size(); i-- > 0;) {
-      if (blocks[i].cap != cap || blocks[i].dev != dev) continue;
-      void* p = blocks[i].p;
-      blocks.erase(blocks.begin() + static_cast<std::ptrdiff_t>(i));
-      held -= cap;
-      return p;
+struct HipMemory {
+  static bool alloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      return false;
     }
-    return nullptr;
+    GJ_HIP_CHECK(e);
+    return true;
   }
-  // drops the oldest blocks until the pool holds no more than this
-  void trim(size_t max_bytes, size_t max_blocks) {
-    for (;;) {
-      Block b{};
-      {
-        std::lock_guard<std::mutex> g(mu);
-        if (held <= max_bytes && blocks.size() <= max_blocks) return;
-        b = blocks.front();
-        blocks.erase(blocks.begin());
-        held -= b.cap;
-      }
-      (void)hipFree(b.p);
-    }
-  }
+  static void release(void* p) noexcept { (void)hipFree(p); }
 };
-DevicePool& device_pool() {
-  static DevicePool* pool = new DevicePool;  // never destroyed: the device may be gone by then
-  return *pool;
-}
 
-// Sizes in steps of an eighth of their power of two (4 KiB at least), so that builds over
-// columns of about the same size share blocks; larger ones than the pool keeps as they are.
-size_t pool_size(size_t bytes) {
-  if (bytes > kPoolBlock) return bytes;
-  size_t step = 4096;
-  while (step * 16 <= bytes) step *= 2;
-  return (bytes + step - 1) / step * step;
+BlockPool<HipMemory>& device_pool() {
+  static auto* pool = new BlockPool<HipMemory>;  // never destroyed: the device may be gone by then
+  return *pool;
 }
 
 }  // namespace
 
+void* device_alloc(size_t bytes) {
+  void* p = device_pool().alloc(bytes);
+  GJ_REQUIRE(p, GJ_ERR_NOMEM, "device memory: hipMalloc failed: out of memory");
+  return p;
+}
+
 void* device_take(size_t bytes, size_t& cap, int& dev) {
   GJ_HIP_CHECK(hipGetDevice(&dev));
-  cap = pool_size(bytes);
-  if (cap <= kPoolBlock)
-    if (void* p = device_pool().find(cap, dev)) return p;
-  void* p = nullptr;
-  hipError_t e = hipMalloc(&p, cap);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    device_pool().trim(0, 0);
-    e = hipMalloc(&p, cap);
-  }
-  GJ_HIP_CHECK(e);
+  void* p = device_pool().take(bytes, cap, dev);
+  GJ_REQUIRE(p, GJ_ERR_NOMEM, "device memory: hipMalloc failed: out of memory");
   return p;
 }
 
 void device_give(void* p, size_t cap, int dev) noexcept {
   int now = -1;
   void* token = nullptr;
-  if (cap > kPoolBlock || hipGetDevice(&now) != hipSuccess || now != dev || hipMalloc(&token, 256) != hipSuccess ||
-      hipFree(token) != hipSuccess) {
-    (void)hipGetLastError();
-    (void)hipFree(p);
-    return;
-  }
-  DevicePool& pool = device_pool();
-  try {
-    std::lock_guard<std::mutex> g(pool.mu);
-    pool.blocks.push_back({p, cap, dev});
-    pool.held += cap;
-  } catch (...) {
-    (void)hipFree(p);
-    return;
-  }
-  pool.trim(kPoolBytes, kPoolBlocks);
+  const bool idle = cap <= BlockPool<HipMemory>::kBlock && hipGetDevice(&now) == hipSuccess && now == dev &&
+                    hipMalloc(&token, 256) == hipSuccess && hipFree(token) == hipSuccess;
+  if (!idle) (void)hipGetLastError();
+  if (!idle || !device_pool().keep(p, cap, dev)) (void)hipFree(p);
 }
 
 int blocks_per_cu(const void* fn, unsigned block, size_t lds) {
@@ -218,7 +165,7 @@ int gj_malloc(void** d_ptr, uint64_t bytes) {
     GJ_REQUIRE(d_ptr, GJ_ERR_INVALID, "d_ptr is null");
     *d_ptr = nullptr;
     if (bytes == 0) return;
-    GJ_HIP_CHECK(hipMalloc(d_ptr, bytes));
+    *d_ptr = device_alloc(bytes);
   });
 }
 
@@ -226,6 +173,10 @@ int gj_free(void* d_ptr) {
   return guarded([&] {
     if (d_ptr) GJ_HIP_CHECK(hipFree(d_ptr));
   });
+}
+
+int gj_release_cached(void) {
+  return guarded([&] { device_pool().trim(0, 0); });
 }
 
 int gj_host_malloc(void** h_ptr, uint64_t bytes) {

@@ -32,6 +32,10 @@ int gj_device_count(int* count);
 int gj_device_info(char* name, size_t len, int* compute_units, int* gcn_arch_major);
 int gj_malloc(void** d_ptr, uint64_t bytes);
 int gj_free(void* d_ptr);
+/* The library keeps up to 512 MiB of device memory of dropped indexes for later builds, also
+ * after the last index is gone.  It goes back to the device when an allocation of the
+ * library would fail otherwise, and by this call (for programs with an allocator of their own). */
+int gj_release_cached(void);
 /* Page-locked host memory (hipHostMalloc), mapped into every GPU's address space at the
  * same address: kernels may read it in place (e.g. an index column kept in host memory). */
 int gj_host_malloc(void** h_ptr, uint64_t bytes);
