@@ -135,12 +135,22 @@ __global__ __launch_bounds__(256) void lookup_tuples_kernel(Dev d, const K* __re
 // lanes closer.  What bounds it: LDS.  The bitonic network over whole keys (the reference
 // uses CUB's block radix sort) made 66 passes over the tile, 505 us of the 829 that 2^24
 // probes of 2^22 u64 keys took with binary search; now 77 of 625.
+//
+// Over the host link the bound is the link, and what counts is that the tiles in flight on
+// an XCD, which all sweep the column from its start to its end, find each other's lines in its
+// L2.  With every lane of a wave at work (all four rounds of its quads in flight) the
+// queues before the link grow until the tiles have drifted apart; so (Link) only every
+// 2^skip-th lane looks a probe up: one lane of a quad for a column in host memory, two where
+// only the index structures are there.  2^22 probes of 2^22 keys, bitonic network -> all lanes -> now, ms:
+// binary search u32 6.4 -> 10.5 -> 5.9, RadixSpline u64 11.6 -> 18.2 -> 10.7, learned u32 6.9
+// -> 10.3 -> 5.9, B-tree u32 9.6 -> 9.4 -> 7.1; structures alone, B-tree u64 2.04 -> 2.86 ->
+// 1.83, learned u64 0.55 -> 0.68 -> 0.44.
 constexpr uint32_t kBwsBins = 2048;
 constexpr int kBwsBlock = 256;
 
-template <class Dev, class K, int TILE>
+template <class Dev, class K, int TILE, bool Link>
 __global__ __launch_bounds__(kBwsBlock) void lookup_bws_kernel(Dev d, const K* __restrict__ probes, uint64_t m,
-                                                               uint32_t shift, uint32_t* __restrict__ out) {
+                                                               uint32_t shift, uint32_t skip, uint32_t* __restrict__ out) {
   constexpr int kItems = TILE / kBwsBlock;
   constexpr int kWords = static_cast<int>(kBwsBins) / 2 / kBwsBlock;  // words of two 16-bit counts per thread
   static_assert(TILE <= 65535 && kWords == 4, "16-bit counts, 16 bytes of them per thread");
@@ -205,9 +215,10 @@ __global__ __launch_bounds__(kBwsBlock) void lookup_bws_kernel(Dev d, const K* _
       }
     }
     __syncthreads();
-    for (uint32_t base = w * kWave; base < valid; base += kBwsBlock) {
-      const uint32_t t = base + static_cast<uint32_t>(lane());
-      const bool active = t < valid;
+    const uint32_t lk = Link ? skip : 0u;
+    for (uint32_t base = w * (kWave >> lk); base < valid; base += kBwsBlock >> lk) {
+      const uint32_t ln = static_cast<uint32_t>(lane()), t = base + (ln >> lk);
+      const bool active = t < valid && (ln & ((1u << lk) - 1)) == 0;
       const uint32_t r = d.lookup(active ? sk[t] : K(0), active, lds);
       if (active) out[tile + si[t]] = r;
     }

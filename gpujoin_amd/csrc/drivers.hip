@@ -204,7 +204,15 @@ void lookup_dispatch(const gj_index& ix, const void* probes, uint64_t m, uint32_
         }
         with_index_dev<K>(ix, [&](auto d) { launch_plain(d, pk, m, out, p, s, ix.cu); });
         return;
-      case GJ_BWS: with_index_dev<K>(ix, [&](auto d) { launch_bws(d, pk, m, out, p, s, ix.cu); }); return;
+      case GJ_BWS: {
+        // what a lookup reads over the host link: the column, or the structures (binary search's are
+        // staged in LDS; the hash table and the lines layout hold their own copy of the keys)
+        const bool copy = ix.kind == GJ_HASH || ix.kind == GJ_NO_OP || ix.lm_layout == GJ_LAYOUT_LINES;
+        const bool structures = ix.params.placement == GJ_PLACE_HOST && ix.kind != GJ_BINARY_SEARCH;
+        const uint32_t skip = ix.col_in_host && !copy ? 2u : (structures ? 1u : 0u);
+        with_index_dev<K>(ix, [&](auto d) { launch_bws(d, pk, m, out, p, s, ix.cu, skip); });
+        return;
+      }
       case GJ_PARTITIONING: lookup_partitioned<K>(ix, pk, m, out, p, s); return;
       case GJ_HJ: lookup_hash_join<K>(ix, pk, m, out, p, s); return;
     }

@@ -101,20 +101,31 @@ constexpr int kBwsTile = 2048;
 
 template <class Dev, class K>
 void launch_bws(const Dev& d, const K* probes, uint64_t m, uint32_t* out, const gj_lookup_params& p, hipStream_t s,
-                int cu) {
+                int cu, uint32_t skip) {
   if (m == 0) return;
   (void)lookup_block(p);  // a tile is shared by kBwsBlock threads, whatever valid block size is asked for
   const size_t lds = (d.lds_bytes() + 15) / 16 * 16 + kBwsTile * (sizeof(K) + sizeof(uint16_t)) +
                      kBwsBins * sizeof(uint16_t) + kBwsBlock / kWave * sizeof(uint32_t);
   uint32_t shift = 0;  // bins to at most kBwsBins
   while (((d.coarse_bins() - 1) >> shift) >= kBwsBins) ++shift;
-  const void* fn = reinterpret_cast<const void*>(&lookup_bws_kernel<Dev, K, kBwsTile>);
-  const uint64_t blocks =
-      p.grid_blocks ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(m, kBwsTile)))
-                    : cover_blocks(m, kBwsTile, kBwsBlock, 0, static_cast<uint64_t>(blocks_per_cu(fn, kBwsBlock, lds)) * cu);
-  hipLaunchKernelGGL((lookup_bws_kernel<Dev, K, kBwsTile>), dim3(static_cast<unsigned>(blocks)), dim3(kBwsBlock), lds, s,
-                     d, probes, m, shift, out);
-  GJ_HIP_CHECK(hipGetLastError());
+  auto go = [&]<bool Link>() {
+    auto kernel = &lookup_bws_kernel<Dev, K, kBwsTile, Link>;
+    const void* fn = reinterpret_cast<const void*>(kernel);
+    const uint64_t blocks = p.grid_blocks
+                                ? std::max<uint64_t>(1, std::min<uint64_t>(p.grid_blocks, ceil_div(m, kBwsTile)))
+                                : cover_blocks(m, kBwsTile, kBwsBlock, 0,
+                                               static_cast<uint64_t>(blocks_per_cu(fn, kBwsBlock, lds)) * cu);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kBwsBlock), lds, s, d, probes, m, shift, skip, out);
+    GJ_HIP_CHECK(hipGetLastError());
+  };
+  // Up to two tiles in flight on a CU the link's queues stay short by themselves (2^22 probes, grids
+  // of 512: 8.9 ms with all lanes, 9.0 with a quarter; with eight tiles on the chip a quarter of
+  // the lanes takes twice as long).
+  const uint64_t tiles = p.grid_blocks ? std::min<uint64_t>(p.grid_blocks, ceil_div(m, kBwsTile)) : ceil_div(m, kBwsTile);
+  if (skip && tiles > 2ull * cu)
+    go.template operator()<true>();
+  else
+    go.template operator()<false>();
 }
 
 void build_index(gj_index& ix, hipStream_t s);
