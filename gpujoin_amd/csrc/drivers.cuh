@@ -148,6 +148,15 @@ __global__ __launch_bounds__(256) void lookup_tuples_kernel(Dev d, const K* __re
 constexpr uint32_t kBwsBins = 2048;
 constexpr int kBwsBlock = 256;
 
+// A lookup by waves whose lanes are all at work.
+template <class Dev, class K>
+__device__ __forceinline__ uint32_t lookup_full(const Dev& d, K x, bool active, const uint8_t* lds) {
+  if constexpr (requires { d.template lookup<true>(x, active, lds); })
+    return d.template lookup<true>(x, active, lds);
+  else
+    return d.lookup(x, active, lds);
+}
+
 template <class Dev, class K, int TILE, bool Link>
 __global__ __launch_bounds__(kBwsBlock) void lookup_bws_kernel(Dev d, const K* __restrict__ probes, uint64_t m,
                                                                uint32_t shift, uint32_t skip, uint32_t* __restrict__ out) {
@@ -219,7 +228,8 @@ __global__ __launch_bounds__(kBwsBlock) void lookup_bws_kernel(Dev d, const K* _
     for (uint32_t base = w * (kWave >> lk); base < valid; base += kBwsBlock >> lk) {
       const uint32_t ln = static_cast<uint32_t>(lane()), t = base + (ln >> lk);
       const bool active = t < valid && (ln & ((1u << lk) - 1)) == 0;
-      const uint32_t r = d.lookup(active ? sk[t] : K(0), active, lds);
+      const K key = active ? sk[t] : K(0);
+      const uint32_t r = Link ? d.lookup(key, active, lds) : lookup_full(d, key, active, lds);
       if (active) out[tile + si[t]] = r;
     }
     __syncthreads();

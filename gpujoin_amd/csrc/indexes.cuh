@@ -224,13 +224,15 @@ struct BSearchDev {
   }
   __host__ __device__ uint32_t coarse_bins() const { return (1u << sample_bits) + 1; }
 
-  // Where x would sit if the keys between klo (at position plo) and khi (at phi) were
-  // evenly spread; any error only costs lines.
-  __device__ __forceinline__ static uint32_t guess(K x, K klo, K khi, uint32_t plo, uint32_t phi) {
-    const float f = static_cast<float>(x - klo) * __builtin_amdgcn_rcpf(static_cast<float>(khi - klo));
+  // Where x would sit between positions plo and phi, whose keys are `below` and `above` away
+  // from it, if the keys between were evenly spread; any error only costs lines.
+  __device__ __forceinline__ static uint32_t guess(float below, float above, uint32_t plo, uint32_t phi) {
+    const float f = below * __builtin_amdgcn_rcpf(below + above);
     return plo + static_cast<uint32_t>(fminf(fmaxf(f, 0.0f), 1.0f) * static_cast<float>(phi - plo));
   }
 
+  // Full: the wave's lanes are all at work, or about so (see narrow).
+  template <bool Full = false>
   __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
     const K* s = reinterpret_cast<const K*>(lds);
     const uint32_t nb = 1u << sample_bits, b = coarse(x, lds);
@@ -246,7 +248,7 @@ struct BSearchDev {
       uint32_t found = kNotFound;
       const uint32_t b0 = __builtin_amdgcn_readfirstlane(b);
       if (ballot(open && (b > b0 + 1 || b + 1 < b0)) != 0)  // wave-uniform
-        narrow(x, b, s, open, first, last, found);
+        narrow<Full>(x, b, s, open, first, last, found);
       if (open) {
         const uint32_t r = halve(x, first, static_cast<uint64_t>(last - first) + 1, static_cast<uint64_t>(last) + 1);
         found = r != kNotFound ? r : found;
@@ -275,10 +277,14 @@ struct BSearchDev {
   }
 
   // Whole lines of bucket b by quads; what is left of it is [first, last].  The column's
-  // partial last line is left to the halving.  The bucket's bounds are looked up again where
-  // they are needed: kept in registers, they cost u64 keys a wave per SIMD (70 registers, now
-  // 64), which sorted probes, whose waves do not come here, paid for (2^20 of them over 10^6
-  // keys: halving alone 11.4 us, with the bounds in registers 16.4, now 11.6).
+  // partial last line is left to the halving.  Of the bucket's bounds only x's distances from
+  // its keys are kept: the keys and positions themselves cost u64 keys a wave per SIMD (70
+  // registers, now 64), which sorted probes, whose waves do not come here, paid for (2^20 of
+  // them over 10^6 keys: halving alone 11.4 us, with the bounds in registers 16.4, now 11.6).  Rounds whose lanes have nothing left are passed over, but not
+  // in tiles sorted in LDS (Full): there a wave waits for its loads, and the branches between
+  // the rounds keep their work from filling the wait (2^18 probes of 2^20 u32 keys 34.9 us
+  // without them, 37.1 with; unsorted 2^22 of 10^7 u64 keys 186 without, 168 with).
+  template <bool Full>
   __device__ __forceinline__ void narrow(K x, uint32_t b, const K* s, bool& open, uint32_t& first, uint32_t& last,
                                          uint32_t& found) const {
     const int ql = lane() & (kQuad - 1);
@@ -288,11 +294,10 @@ struct BSearchDev {
     if (!open) b = 0;
     uint32_t line_lo = bucket_first(b) / LK, line_hi = bucket_last(b) / LK, line;
     // klo < x <= khi: the keys before the bucket (the column's first key for the first one) and at its end
-    {
-      const K klo = b > 0 ? s[b - 1] : col[0];
-      open = open && klo <= x;
-      line = guess(x, klo, s[b], b > 0 ? bucket_first(b) - 1 : 0u, bucket_last(b)) / LK;
-    }
+    const K klo = b > 0 ? s[b - 1] : col[0];
+    open = open && klo <= x;
+    const float below_x = static_cast<float>(x - klo);
+    line = guess(below_x, static_cast<float>(s[b] - x), b > 0 ? bucket_first(b) - 1 : 0u, bucket_last(b)) / LK;
     bool bounded = line_hi < whole;     // x is in no line behind line_hi
     bool go = open && line_lo < whole;  // lines to look at
     line_hi -= !bounded && go ? 1u : 0u;
@@ -307,9 +312,10 @@ struct BSearchDev {
         const uint32_t l = quad_bcast<r>(line);
         if ((rounds >> r) & 1u) ln[r].load(lane_base, l);
       });
-      const uint32_t below = quad_below(ln, q, ql, lanes);
-      const bool eq = quad_holds(ln, q, ql, lanes);
-      asm volatile("" : "+v"(b));  // its bounds are read anew
+      const uint64_t at_work = Full ? ~0ull : lanes;
+      const uint32_t below = quad_below(ln, q, ql, at_work);
+      const bool eq = quad_holds(ln, q, ql, at_work);
+      asm volatile("" : "+v"(b));  // its positions are computed anew
       if (go) {
         const uint32_t base = line * LK;
         const bool right = below == LK;  // every key of the line is below x
@@ -329,9 +335,10 @@ struct BSearchDev {
           if (t < kGuesses) {  // wave-uniform
             const uint32_t at = right ? base + LK - 1 : base;  // the edge of the line on x's side
             const K edge = col[at];
-            const K klo = right ? edge : (b > 0 ? s[b - 1] : col[0]), khi = right ? s[b] : edge;
-            const uint32_t plo = right ? at : (b > 0 ? bucket_first(b) - 1 : 0u), phi = right ? bucket_last(b) : at;
-            line = guess(x, klo, khi, plo, phi) / LK;
+            const float away = static_cast<float>(right ? x - edge : edge - x);
+            line = right ? guess(away, static_cast<float>(s[b] - x), at, bucket_last(b))
+                         : guess(below_x, away, b > 0 ? bucket_first(b) - 1 : 0u, at);
+            line /= LK;
             line = line < line_lo ? line_lo : (line > line_hi ? line_hi : line);
           }
         }
