@@ -430,7 +430,7 @@ def autotune(index: Index, probes: DeviceArray, scratch: DeviceArray, m: Optiona
 def autotune_index(kind, column: DeviceArray, probes: DeviceArray, scratch: DeviceArray,
                    host_column: Optional[np.ndarray] = None, base: Optional[IndexParams] = None,
                    m: Optional[int] = None, n: Optional[int] = None, stream: Optional[Stream] = None):
-    """Index parameters (threads per lookup, LDS levels, radix bits, error bounds, leaves) of
+    """Index parameters (node size, LDS levels, radix bits, error bounds, leaves) of
     the fastest candidate build of `kind` over `column` (gj_autotune_index); returns (params, rate)."""
     k = INDEX_NAMES[kind] if isinstance(kind, str) else int(kind)
     best = IndexParams()

@@ -89,12 +89,11 @@ extern "C" int gj_autotune_lookup(const gj_index* index, const void* d_probe_sam
 }
 
 // ---- index autotuner -------------------------------------------------------
-// Picks the index's own parameters: threads per lookup (Harmonia's lanes per
-// node search), the B-tree's node size and LDS-resident levels, RadixSpline's radix
-// bits and error bound, the learned index's layout, line load, leaf count and error
-// bound.  Each
-// candidate is built over the caller's column and timed with the plain driver
-// on the probe sample; the candidates are destroyed again.
+// Picks the index's own parameters: the B-tree's node size and LDS-resident levels,
+// RadixSpline's radix bits and error bound, the learned index's layout, line load, leaf
+// count and error bound (Harmonia has one candidate).  Each candidate is built over the
+// caller's column and timed with the plain driver on the probe sample; the candidates are
+// destroyed again.
 namespace {
 
 std::vector<gj_index_params> index_candidates(gj_index_kind kind, uint64_t n, int key_bytes,
@@ -107,8 +106,8 @@ std::vector<gj_index_params> index_candidates(gj_index_kind kind, uint64_t n, in
   };
   switch (kind) {
     case GJ_HARMONIA:
-      for (uint32_t g : {8u, 16u, 32u})
-        if (g != 32 || key_bytes == 4) add([&](gj_index_params& p) { p.harmonia_group_lanes = g; });
+      // the widths of harmonia_group_lanes give one and the same index
+      add([&](gj_index_params& p) { p.harmonia_group_lanes = 8; });
       break;
     case GJ_BTREE:
       // node size (64 B, one 128 B line, 256 B) x the LDS budget of the upper levels

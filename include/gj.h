@@ -394,7 +394,7 @@ int gj_autotune_lookup(const gj_index* index, const void* d_probe_sample, uint64
  * parameters, times the plain lookup of the probe sample on each, and writes
  * the fastest parameter set into *best.  Candidates, starting from *base (or
  * the defaults when base is NULL):
- *   harmonia      harmonia_group_lanes 8 / 16 (/ 32 for 4-byte keys), which time alike
+ *   harmonia      harmonia_group_lanes 8 only: the other widths give the same index
  *   btree         btree_lds_bytes 4096 / 16384 / 32768: the LDS-resident upper levels
  *   radix_spline  rs_radix_bits 12 / 13 (table in LDS) / 16 / 18 (global) x rs_max_error 16 / 32 / 64
  *   learned_plr   learned_leaf_bits 0 (the default: compact 8-byte leaves where the build
