@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("kb,lanes", [(4, 8), (4, 32), (8, 16)])
 def test_one_harmonia_candidate(gj, gpu, kb, lanes):
     print(f"[case] kb={kb} lanes={lanes}", flush=True)
-    keys = gj.gen_build_keys(40001, kb, _lib.KEYS_UNIFORM, 0, 0x51 + kb)
+    keys = gj.gen_build_keys(40000, kb, _lib.KEYS_UNIFORM, 0, 0x51 + kb)  # whole nodes of 32 keys
     col = gj.DeviceArray.from_numpy(keys)
     probes, _ = gj.gen_probes(keys, 20011, _lib.PROBES_UNIFORM, 1.0, 0.0, 0, 0x52)
     dp = gj.DeviceArray.from_numpy(probes)
