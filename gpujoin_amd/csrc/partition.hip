@@ -729,15 +729,15 @@ struct PartPlan {
   uint64_t chunk;
 };
 
-constexpr uint32_t kMaxBlocksPerCu = 4;
+constexpr uint32_t kBlocksPerCu = 2;  // of a pass: two workgroups of 1024 threads are resident
 constexpr size_t kMaxLds = 160 * 1024;
 
-// Whole tiles per block, about per_cu blocks per CU; each block's histogram row
+// Whole tiles per block, about kBlocksPerCu blocks per CU; each block's histogram row
 // lives in scratch.
-PartPlan plan(uint64_t m, uint32_t bits, int cu, uint32_t per_cu) {
+PartPlan plan(uint64_t m, uint32_t bits, int cu) {
   PartPlan p;
   p.fan = 1u << bits;
-  const uint64_t want = static_cast<uint64_t>(cu) * per_cu;
+  const uint64_t want = static_cast<uint64_t>(cu) * kBlocksPerCu;
   uint64_t chunk = std::max<uint64_t>(kPartTile, ceil_div(m, want));
   chunk = ceil_div(chunk, kPartTile) * kPartTile;
   p.chunk = chunk;
@@ -745,10 +745,9 @@ PartPlan plan(uint64_t m, uint32_t bits, int cu, uint32_t per_cu) {
   return p;
 }
 
-// The starts scan's span sums, then the histogram rows for the plan with the most
-// blocks any pass uses.
+// The starts scan's span sums, then the plan's histogram rows.
 uint64_t hist_bytes(uint64_t m, uint32_t bits, int cu) {
-  const PartPlan p = plan(m, bits, cu, kMaxBlocksPerCu);
+  const PartPlan p = plan(m, bits, cu);
   return kScanSumsBytes + ceil_div(static_cast<uint64_t>(p.blocks) * p.fan * 4 + 256, 256) * 256;
 }
 
@@ -848,7 +847,7 @@ void partition_pass(const K* keys, const uint32_t* in_payload, uint32_t payload_
                     uint32_t bits, uint32_t align, bool stable, K* out_keys, uint32_t* out_payload, uint64_t* start,
                     uint64_t* start2, uint64_t* count, uint32_t* hist, uint64_t* sums, unsigned long long* dropped,
                     int cu, hipStream_t s, bool hashed = false) {
-  const PartPlan p = plan(m, bits, cu, 2);
+  const PartPlan p = plan(m, bits, cu);
   auto histogram = hashed ? &part_hist_kernel<K, true> : &part_hist_kernel<K, false>;
   hipLaunchKernelGGL(histogram, dim3(p.blocks), dim3(1024), p.fan * sizeof(uint32_t), s, keys, m, p.chunk, shift, bits,
                      hist, Seg{});
