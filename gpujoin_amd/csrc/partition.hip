@@ -783,10 +783,11 @@ struct Scatter {
 // thread would pad one slot after the other (5.5 k u32 items into 2^11 partitions: two
 // workgroups took 51 us, now 9.6).
 template <class K>
-void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, hipStream_t s, bool hashed = false) {
+void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, int cu, hipStream_t s, bool hashed = false) {
   if (a.align > 1) {
     const uint64_t slots = (static_cast<uint64_t>(a.sg.segs ? a.sg.segs : 1u) << a.bits) * a.align;
-    grid = std::max(grid, static_cast<unsigned>(std::min<uint64_t>(ceil_div(slots, 2 * kTileBlock), 512)));
+    const uint64_t resident = static_cast<uint64_t>(cu) * kBlocksPerCu;
+    grid = std::max(grid, static_cast<unsigned>(std::min<uint64_t>(ceil_div(slots, 2 * kTileBlock), resident)));
   }
   const size_t lds = tile_lds_bytes(1u << a.bits, sizeof(K), a.out_payload != nullptr, stable, kTileBlock, kTileItems);
   GJ_REQUIRE(lds <= kMaxLds - 1024 && (1u << a.bits) <= 8u * kTileBlock, GJ_ERR_INTERNAL,
@@ -859,7 +860,7 @@ void partition_pass(const K* keys, const uint32_t* in_payload, uint32_t payload_
   const uint64_t cap = m + (align > 1 ? static_cast<uint64_t>(p.fan) * align : 0ull);
   launch_scatter<K>({keys, in_payload, payload_base, m, p.chunk, shift, bits, hist, start, count, align, out_keys,
                      out_payload, nullptr, cap, dropped, Seg{}},
-                    stable, p.blocks, s, hashed);
+                    stable, p.blocks, cu, s, hashed);
 }
 
 uint64_t partition_capacity(uint64_t m, int key_bytes, uint32_t bits) {
@@ -876,9 +877,6 @@ uint64_t partition_scratch(uint64_t m, int key_bytes, uint32_t bits, uint32_t pa
 // partitions h * 2^bits + p, with 128-byte aligned starts.  Chunks never straddle
 // segments, so every histogram row and cursor belongs to one segment.
 constexpr uint64_t kSegChunk = 16384;
-// two workgroups for each of 256 CUs (two windows of 262144 u32 probes at fan-out 2^12, the whole
-// lookup: 107 -> 66 us)
-constexpr uint64_t kSegMinChunks = 512;
 // Segments of this many chunks on average scan their histogram columns with a workgroup
 // per 64 partitions; shorter ones take one thread per partition.
 constexpr uint64_t kSegWideChunks = 32;
@@ -888,11 +886,13 @@ void partition_segmented(const K* keys, const uint32_t* payload, uint64_t m, uin
                          uint32_t segs, const uint64_t* start1, const uint64_t* count1, uint64_t* chunk0,
                          uint32_t align, bool stable, K* out_keys, uint32_t* out_payload, uint32_t* inv,
                          uint64_t* start, uint64_t* count, uint32_t* hist, uint64_t* sums,
-                         unsigned long long* dropped, hipStream_t s) {
+                         unsigned long long* dropped, int cu, hipStream_t s) {
   const uint32_t fan = 1u << bits;
   const uint64_t total_fan = static_cast<uint64_t>(segs) * fan;
-  // whole tiles, down to one where longer chunks would leave CUs without a workgroup
-  const uint64_t chunk = std::clamp<uint64_t>(ceil_div(ceil_div(m, kSegMinChunks), kPartTile) * kPartTile, kPartTile, kSegChunk);
+  // whole tiles, down to one where longer chunks would leave CUs without their two workgroups
+  // (256 CUs, two windows of 262144 u32 probes at fan-out 2^12, the whole lookup: 107 -> 66 us)
+  const uint64_t resident = static_cast<uint64_t>(cu) * kBlocksPerCu;
+  const uint64_t chunk = std::clamp<uint64_t>(ceil_div(ceil_div(m, resident), kPartTile) * kPartTile, kPartTile, kSegChunk);
   const uint64_t blocks = ceil_div(m, chunk) + segs;  // an upper bound on the chunks
   GJ_REQUIRE(blocks < (1ull << 31), GJ_ERR_INVALID, "too many partition chunks");
   hipLaunchKernelGGL(seg_chunks_kernel, dim3(1), dim3(1024), 0, s, count1, segs, chunk, chunk0);
@@ -912,7 +912,7 @@ void partition_segmented(const K* keys, const uint32_t* payload, uint64_t m, uin
   const uint64_t cap = m + (align > 1 ? total_fan * align : 0ull);
   launch_scatter<K>({keys, payload, 0u, m, chunk, shift, bits, hist, start, count, align, out_keys, out_payload, inv,
                      cap, dropped, sg},
-                    stable, static_cast<unsigned>(blocks), s);
+                    stable, static_cast<unsigned>(blocks), cu, s);
 }
 
 namespace {
@@ -995,18 +995,19 @@ void partition_windows(const K* keys, uint64_t m, uint64_t window, uint32_t bits
                      wstart, wcount, static_cast<uint32_t>(L.windows), window, m);
   GJ_HIP_CHECK(hipGetLastError());
   const uint32_t align = part_align(sizeof(K));
+  const int cu = device_cu_count();
   if (!L.hb) {
     partition_segmented<K>(keys, nullptr, m, ignore, bits, static_cast<uint32_t>(L.windows), wstart, wcount, chunk0,
-                           align, false, out_keys, nullptr, inv1, start, count, hist, sums, dropped, s);
+                           align, false, out_keys, nullptr, inv1, start, count, hist, sums, dropped, cu, s);
     return;
   }
   K* tk = reinterpret_cast<K*>(scratch + L.o_tk);
   auto* sa = reinterpret_cast<uint64_t*>(scratch + L.o_sa);
   auto* ca = reinterpret_cast<uint64_t*>(scratch + L.o_ca);
   partition_segmented<K>(keys, nullptr, m, ignore + L.lb, L.hb, static_cast<uint32_t>(L.windows), wstart, wcount,
-                         chunk0, 1, false, tk, nullptr, inv1, sa, ca, hist, sums, dropped, s);
+                         chunk0, 1, false, tk, nullptr, inv1, sa, ca, hist, sums, dropped, cu, s);
   partition_segmented<K>(tk, nullptr, m, ignore, L.lb, static_cast<uint32_t>(L.segs_b), sa, ca, chunk0, align, false,
-                         out_keys, nullptr, inv2, start, count, hist, sums, dropped, s);
+                         out_keys, nullptr, inv2, start, count, hist, sums, dropped, cu, s);
 }
 template void partition_windows<uint32_t>(const uint32_t*, uint64_t, uint64_t, uint32_t, uint32_t, uint32_t,
                                           uint32_t*, uint32_t*, uint32_t*, uint64_t*, uint64_t*, uint8_t*,
@@ -1038,7 +1039,7 @@ void partition_keys(const K* keys, uint64_t m, uint32_t payload_base, uint32_t b
     partition_pass<K>(keys, nullptr, payload_base, m, ignore + lb, hb, 1, stable, tk, tp, start1, nullptr, count1, hist,
                       sums, dropped, cu, s, hashed);
     partition_segmented<K>(tk, tp, m, ignore, lb, segs, start1, count1, chunk0, align, stable, out_keys, out_payload,
-                           nullptr, start, count, hist, sums, dropped, s);
+                           nullptr, start, count, hist, sums, dropped, cu, s);
     if (start2) GJ_HIP_CHECK(hipMemcpyAsync(start2, start, (1ull << bits) * 8, hipMemcpyDeviceToDevice, s));
     return;
   }
