@@ -78,10 +78,10 @@ __global__ __launch_bounds__(256) void lookup_marked_kernel(Dev d, const K* __re
 
 // Workgroups are dispatched round-robin over the 8 XCDs (each with its own
 // L2).  This maps the dispatch index to a logical index so that each XCD
-// receives one contiguous eighth of the logical range.
-__device__ __forceinline__ uint32_t xcd_logical_block() {
-  const uint32_t nb = gridDim.x;
-  if (nb % 8 != 0) return blockIdx.x;
+// receives one contiguous eighth of the logical range [0, nb); workgroups from nb on keep
+// their index.
+__device__ __forceinline__ uint32_t xcd_logical_block(uint32_t nb) {
+  if (nb % 8 != 0 || blockIdx.x >= nb) return blockIdx.x;
   return (blockIdx.x % 8) * (nb / 8) + blockIdx.x / 8;
 }
 

@@ -14,10 +14,10 @@
 // Kernels (no cooperative launch, no device-wide barrier):
 //   hist     one block per contiguous chunk, LDS histogram of 2^radix_bits u32 bins
 //   colscan  column prefix over the blocks and the partition totals, 64 partitions a block
-//   starts   one block: aligned exclusive prefix over partitions -> partition starts, and
-//            the padding behind every partition
+//   starts   one block: aligned exclusive prefix over partitions -> partition starts
 //   scatter  one block per chunk (the same chunks as hist): tiles sorted by partition in
-//            LDS, stable or in any order, then stored run by run
+//            LDS, stable or in any order, then stored run by run; all blocks, and more where
+//            the chunks are few, write the padding behind every partition
 #include <algorithm>
 
 #include "common.hpp"
@@ -54,12 +54,13 @@ __device__ __forceinline__ void drop(unsigned long long* dropped) {
 // chunks of `chunk` items; block j handles chunk j - chunk0[h] of the segment h with
 // chunk0[h] <= j < chunk0[h + 1], and partition p of segment h is output partition
 // h * 2^bits + p.  Blocks from chunk0[segs] on have no work.  segs = 0: plain mode,
-// block c handles items [c * chunk, (c + 1) * chunk).
+// block c handles items [c * chunk, (c + 1) * chunk), c < chunks.
 struct Seg {
   const uint64_t* chunk0;  // segs + 1 entries
   const uint64_t* start;   // segs entries
   const uint64_t* count;   // segs entries
   uint32_t segs;
+  uint32_t chunks;  // plain mode
 };
 
 // This block's item range and output partition base; false: the block has no work.
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(1024) void part_hist_kernel(const K* __restrict__ k
   extern __shared__ uint32_t h[];
   const uint32_t fan = 1u << bits;
   // chunk index; the scatter maps blocks the same way
-  const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block();
+  const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block(sg.chunks);
   uint64_t lo, hi, pbase;
   if (!seg_range(sg, c, chunk, m, fan, lo, hi, pbase)) return;  // block-uniform, before any barrier
   const Digit digit(shift, fan);
@@ -435,7 +436,7 @@ __global__ __launch_bounds__(B, 4) void part_scatter_kernel(
   uint16_t* off = rows + static_cast<size_t>(W) * fan;               // [fan] tile offsets (stable)
   // neighbouring chunks run on one XCD, so the partial lines that neighbouring
   // chunks write into a partition's run meet in the same L2
-  const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block();  // as part_hist_kernel
+  const uint64_t c = sg.segs ? static_cast<uint64_t>(blockIdx.x) : xcd_logical_block(sg.chunks);  // as part_hist_kernel
   uint64_t lo, hi, pbase;
   if (!seg_range(sg, c, chunk, m, fan, lo, hi, pbase)) return;  // block-uniform, before any barrier
   const Digit digit(shift, fan);
@@ -781,7 +782,9 @@ struct Scatter {
 
 // Workgroups past the chunks share the padding alone: with few items and many partitions a
 // thread would pad one slot after the other (5.5 k u32 items into 2^11 partitions: two
-// workgroups took 51 us, now 9.6).
+// workgroups took 51 us, now 9.6).  They are no part of the map of chunks to XCDs: counted in,
+// they left the chunks of a few to the first XCDs alone (131072 u32 items into 2^12
+// partitions, whole call: 33.3 us, now 31.3).
 template <class K>
 void launch_scatter(const Scatter<K>& a, bool stable, unsigned grid, int cu, hipStream_t s, bool hashed = false) {
   if (a.align > 1) {
@@ -849,9 +852,10 @@ void partition_pass(const K* keys, const uint32_t* in_payload, uint32_t payload_
                     uint64_t* start2, uint64_t* count, uint32_t* hist, uint64_t* sums, unsigned long long* dropped,
                     int cu, hipStream_t s, bool hashed = false) {
   const PartPlan p = plan(m, bits, cu);
+  const Seg sg{nullptr, nullptr, nullptr, 0, p.blocks};
   auto histogram = hashed ? &part_hist_kernel<K, true> : &part_hist_kernel<K, false>;
   hipLaunchKernelGGL(histogram, dim3(p.blocks), dim3(1024), p.fan * sizeof(uint32_t), s, keys, m, p.chunk, shift, bits,
-                     hist, Seg{});
+                     hist, sg);
   GJ_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(part_colscan_kernel, dim3((p.fan + kWave - 1) / kWave), dim3(kColThreads), 0, s, hist, p.blocks,
                      p.fan, count);
@@ -859,7 +863,7 @@ void partition_pass(const K* keys, const uint32_t* in_payload, uint32_t payload_
   launch_scan_starts(count, p.fan, align, start, start2, sums, s);
   const uint64_t cap = m + (align > 1 ? static_cast<uint64_t>(p.fan) * align : 0ull);
   launch_scatter<K>({keys, in_payload, payload_base, m, p.chunk, shift, bits, hist, start, count, align, out_keys,
-                     out_payload, nullptr, cap, dropped, Seg{}},
+                     out_payload, nullptr, cap, dropped, sg},
                     stable, p.blocks, cu, s, hashed);
 }
 
@@ -897,7 +901,7 @@ void partition_segmented(const K* keys, const uint32_t* payload, uint64_t m, uin
   GJ_REQUIRE(blocks < (1ull << 31), GJ_ERR_INVALID, "too many partition chunks");
   hipLaunchKernelGGL(seg_chunks_kernel, dim3(1), dim3(1024), 0, s, count1, segs, chunk, chunk0);
   GJ_HIP_CHECK(hipGetLastError());
-  const Seg sg{chunk0, start1, count1, segs};
+  const Seg sg{chunk0, start1, count1, segs, 0};
   hipLaunchKernelGGL(part_hist_kernel<K>, dim3(static_cast<unsigned>(blocks)), dim3(kTileBlock),
                      fan * sizeof(uint32_t), s, keys, m, chunk, shift, bits, hist, sg);
   GJ_HIP_CHECK(hipGetLastError());

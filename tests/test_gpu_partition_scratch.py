@@ -13,7 +13,8 @@ GUARD = 4096
 
 
 @pytest.mark.parametrize("kb,bits,passes", [(4, 10, 1), (8, 12, 1), (8, 11, 2), (4, 14, 2)])
-@pytest.mark.parametrize("m", [1, 4097, 3_000_017])
+# 65_530: two chunks for each XCD, fewer than the workgroups that pad
+@pytest.mark.parametrize("m", [1, 4097, 65_530, 3_000_017])
 def test_scratch_is_exact(gj, orc, gpu, kb, bits, passes, m):
     print(f"[case] kb={kb} bits={bits} passes={passes} m={m}", flush=True)
     p = _lib.PartitionParams(bits, 0, passes)
