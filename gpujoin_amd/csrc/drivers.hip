@@ -189,7 +189,7 @@ void lookup_dispatch(const gj_index& ix, const void* probes, uint64_t m, uint32_
     switch (p.approach) {
       case GJ_PLAIN:
         if ((ix.kind == GJ_LEARNED_PLR || ix.kind == GJ_LEARNED_MLP) && ix.lm_layout == GJ_LAYOUT_COLUMN &&
-            ix.lm_fallback_any &&
+            ix.lm_fallback_any && !short_column<K>(ix) &&
             ix.stats.fallback_keys * kMarkFallbackRatio <= ix.n) {
           // few keys in leaves routed to the B-tree: the learned kernel marks their
           // probes, then one B-tree pass over the marks (the hot kernel stays free of
@@ -210,6 +210,10 @@ void lookup_dispatch(const gj_index& ix, const void* probes, uint64_t m, uint32_
         const bool copy = ix.kind == GJ_HASH || ix.kind == GJ_NO_OP || ix.lm_layout == GJ_LAYOUT_LINES;
         const bool structures = ix.params.placement == GJ_PLACE_HOST && ix.kind != GJ_BINARY_SEARCH;
         const uint32_t skip = ix.col_in_host && !copy ? 2u : (structures ? 1u : 0u);
+        if (ix.kind == GJ_BTREE && ix.n * sizeof(K) < ix.bt.node_bytes) {
+          launch_bws(short_dev<K>(ix), pk, m, out, p, s, ix.cu, skip);
+          return;
+        }
         with_index_dev<K>(ix, [&](auto d) { launch_bws(d, pk, m, out, p, s, ix.cu, skip); });
         return;
       }

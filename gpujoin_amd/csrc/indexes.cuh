@@ -137,38 +137,31 @@ __device__ __forceinline__ uint32_t line_at(uint32_t line, uint64_t n) {
   return line * kKeys < last ? line * kKeys : last;
 }
 
-// Position of each lane's probe in a column of n < QuadLine::kKeys keys, or not found: a
-// quad reads the column once for its four probes, padded with key_max.
-template <class K, int NB>
-__device__ __forceinline__ uint32_t quad_find_short(const K* col, uint64_t n, bool live, const QuadProbes<K>& q,
-                                                    int ql) {
-  using L = QuadLine<K, NB>;
-  const uint32_t valid = static_cast<uint32_t>(n);
-  L ln;
-#pragma unroll
-  for (int t = 0; t < L::kPieces; ++t)
-#pragma unroll
-    for (int j = 0; j < L::kPiece; ++j) {
-      const uint32_t i = static_cast<uint32_t>(ql * L::kLaneKeys + t * L::kPiece + j);
-      ln.pc[t].k[j] = i < valid ? col[i] : key_max<K>();
-    }
-  uint32_t c = 0, e = 0;
-#pragma unroll
-  for (int r = 0; r < kQuad; ++r) {
-    c |= ln.below(q.x[r]) << (8 * r);
-    e |= ln.holds(q.x[r]) ? 1u << r : 0u;
+// Branch-free lower_bound over len keys of a column from lo on; the row id if the key before
+// hi is x.
+template <class K>
+__device__ __forceinline__ uint32_t halve(const K* col, K x, uint64_t lo, uint64_t len, uint64_t hi) {
+  const K* base = col + lo;
+  while (len > 1) {
+    const uint64_t half = len >> 1;
+    base = (base[half] < x) ? base + half : base;
+    len -= half;
   }
-  c = (quad_sum(c) >> (8 * ql)) & 0xFFu;
-  e = (quad_or(e) >> ql) & 1u;
-  return (live && e != 0 && c < valid) ? c : kNotFound;  // the padding is no match
+  const uint64_t p = static_cast<uint64_t>(base - col) + ((base[0] < x) ? 1u : 0u);
+  return (p < hi && col[p] == x) ? static_cast<uint32_t>(p) : kNotFound;
 }
 
-// Position of each lane's probe in its NB-byte chunk of the column, or not found.
-template <class K, int NB>
-__device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, uint32_t chunk, bool live,
+// Position of each lane's probe in its NB-byte chunk of the column, or not found.  In a column
+// shorter than a chunk each lane halves for itself: a quad's read of the padded line is so
+// much code that it slows the whole lines down (2^24 probes of 2^22 u32 keys, B-tree: with it
+// 292 us, now 281).  Whole: the column is no shorter (the halving, too, costs sorted tiles 5 %:
+// 2^16 probes of 2^16 u32 keys 23.4 us, now 22.1).
+template <class K, int NB, bool Whole = false>
+__device__ __forceinline__ uint32_t quad_find_equal(const K* col, uint64_t n, uint32_t chunk, bool live, K x,
                                                     const QuadProbes<K>& q, int ql) {
   using L = QuadLine<K, NB>;
-  if (n < static_cast<uint64_t>(L::kKeys)) return quad_find_short<K, NB>(col, n, live, q, ql);  // kernel-uniform
+  if constexpr (!Whole)
+    if (n < static_cast<uint64_t>(L::kKeys)) return live ? halve(col, x, 0, n, n) : kNotFound;  // kernel-uniform
   const uint32_t at = line_at<L::kKeys>(chunk, n);
   L ln[kQuad];
   const K* lane_base = col + ql * L::kLaneKeys;
@@ -240,7 +233,7 @@ struct BSearchDev {
     if constexpr (!Lines) {
       if (!active || b >= nb || lo >= n) return kNotFound;
       const uint64_t hi = (lo + step < n) ? lo + step : n;
-      return halve(x, lo, hi - lo, hi);
+      return halve(col, x, lo, hi - lo, hi);
     } else {
       bool open = active && b < nb && lo < n;
       // x's position is in [first, last], or last + 1 where found holds it already
@@ -250,7 +243,7 @@ struct BSearchDev {
       if (ballot(open && (b > b0 + 1 || b + 1 < b0)) != 0)  // wave-uniform
         narrow<Full>(x, b, s, open, first, last, found);
       if (open) {
-        const uint32_t r = halve(x, first, static_cast<uint64_t>(last - first) + 1, static_cast<uint64_t>(last) + 1);
+        const uint32_t r = halve(col, x, first, static_cast<uint64_t>(last - first) + 1, static_cast<uint64_t>(last) + 1);
         found = r != kNotFound ? r : found;
       }
       return found;
@@ -264,26 +257,15 @@ struct BSearchDev {
     return static_cast<uint32_t>(lo + step < n ? lo + step : n) - 1;
   }
 
-  // Branch-free lower_bound over len keys from lo on; the row id if the key before hi is x.
-  __device__ __forceinline__ uint32_t halve(K x, uint64_t lo, uint64_t len, uint64_t hi) const {
-    const K* base = col + lo;
-    while (len > 1) {
-      const uint64_t half = len >> 1;
-      base = (base[half] < x) ? base + half : base;
-      len -= half;
-    }
-    const uint64_t p = static_cast<uint64_t>(base - col) + ((base[0] < x) ? 1u : 0u);
-    return (p < hi && col[p] == x) ? static_cast<uint32_t>(p) : kNotFound;
-  }
-
   // Whole lines of bucket b by quads; what is left of it is [first, last].  The column's
   // partial last line is left to the halving.  Of the bucket's bounds only x's distances from
   // its keys are kept: the keys and positions themselves cost u64 keys a wave per SIMD (70
   // registers, now 64), which sorted probes, whose waves do not come here, paid for (2^20 of
-  // them over 10^6 keys: halving alone 11.4 us, with the bounds in registers 16.4, now 11.6).  Rounds whose lanes have nothing left are passed over, but not
-  // in tiles sorted in LDS (Full): there a wave waits for its loads, and the branches between
-  // the rounds keep their work from filling the wait (2^18 probes of 2^20 u32 keys 34.9 us
-  // without them, 37.1 with; unsorted 2^22 of 10^7 u64 keys 186 without, 168 with).
+  // them over 10^6 keys: halving alone 11.4 us, with the bounds in registers 16.4, now 11.6).
+  // Rounds whose lanes have nothing left are passed over, but not in tiles sorted in LDS
+  // (Full): there a wave waits for its loads, and the branches between the rounds keep their
+  // work from filling the wait (2^18 probes of 2^20 u32 keys 34.9 us without them, 37.1 with;
+  // unsorted 2^22 of 10^7 u64 keys 186 without, 168 with).
   template <bool Full>
   __device__ __forceinline__ void narrow(K x, uint32_t b, const K* s, bool& open, uint32_t& first, uint32_t& last,
                                          uint32_t& found) const {
@@ -413,6 +395,8 @@ struct BTreeDev {
     node = live ? static_cast<uint32_t>(child) : 0u;
   }
 
+  // Full: by waves whose lanes are all at work, over a column of a chunk and more.
+  template <bool Full = false>
   __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t* lds) const {
     const int ql = lane() & (kQuad - 1);
     const QuadProbes<K> q(x);
@@ -426,7 +410,23 @@ struct BTreeDev {
     uint32_t lvl = lds_levels;
     for (; lvl < levels; ++lvl)
       descend(node, live, quad_count_less<K, NB>(nodes + level_off[lvl] * NK, node, q, ql), lvl);
-    return quad_find_equal<K, NB>(col, n, node, live, q, ql);
+    return quad_find_equal<K, NB, Full>(col, n, node, live, x, q, ql);
+  }
+};
+
+// A column shorter than a line under an index that searches windows (or, blockwise sorted, under
+// a B-tree): each lane halves for itself.  The window search holds no code for it, which slowed it down (2^23 probes of 2^22 u64
+// keys, learned MLP root: with it 171 us, now 165).
+template <class K>
+struct ShortDev {
+  const K* col;
+  uint64_t n;
+  __host__ __device__ size_t lds_bytes() const { return 0; }
+  __device__ void stage(uint8_t*) const {}
+  __device__ __forceinline__ uint32_t coarse(K, const uint8_t*) const { return 0; }
+  __host__ __device__ uint32_t coarse_bins() const { return 1; }
+  __device__ __forceinline__ uint32_t lookup(K x, bool active, const uint8_t*) const {
+    return active ? halve(col, x, 0, n, n) : kNotFound;
   }
 };
 

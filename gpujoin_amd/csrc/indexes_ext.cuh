@@ -131,7 +131,7 @@ struct HarmoniaDev {
 // line holds it.  The owning lane alone holds its probe's state (line and window; a step
 // to one side takes the other side's part of the window away), which keeps the registers
 // per lane, and hence the waves per SIMD, where a latency-bound search needs them.
-// Positions are 32-bit (n < 2^32).
+// Positions are 32-bit (n < 2^32); the column holds a line at least.
 // ---------------------------------------------------------------------------
 template <class K>
 __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n, uint32_t my_pred, uint32_t my_lo,
@@ -142,7 +142,6 @@ __device__ __forceinline__ uint32_t group_window_search(const K* col, uint64_t n
   const QuadProbes<K> q(my_x);
   const K* lane_base = col + ql * L::kLaneKeys;
   bool open = my_live && my_lo < my_hi;
-  if (n < LK) return quad_find_short<K, 128>(col, n, open, q, ql);  // kernel-uniform
   uint32_t line = 0, found = kNotFound;
   if (open) {
     const uint32_t p = my_pred < my_lo ? my_lo : (my_pred >= my_hi ? my_hi - 1 : my_pred);

@@ -155,9 +155,25 @@ inline bool few_halvings(const gj_index& ix, uint64_t m) {
   return ix.kind == GJ_BINARY_SEARCH && m * ilog2_ceil(ix.sample_step) < kLinesMinHalvings;
 }
 
+// Columns shorter than a line are halved (ShortDev) in place of the window search.
+template <class K>
+bool short_column(const gj_index& ix) {
+  const bool learned = ix.kind == GJ_LEARNED_PLR || ix.kind == GJ_LEARNED_MLP;
+  return (ix.kind == GJ_RADIX_SPLINE || (learned && ix.lm_layout == GJ_LAYOUT_COLUMN)) && ix.n * sizeof(K) < 128;
+}
+
+template <class K>
+ShortDev<K> short_dev(const gj_index& ix) {
+  return {static_cast<const K*>(ix.d_col), ix.n};
+}
+
 // Calls f(descriptor) with the device descriptor of the index (every kind).
 template <class K, class F>
 void with_index_dev(const gj_index& ix, F&& f, uint64_t lines_above = kLinesLookups) {
+  if (short_column<K>(ix)) {
+    f(short_dev<K>(ix));
+    return;
+  }
   switch (ix.kind) {
     case GJ_BINARY_SEARCH:
       if (ix.sample_step > lines_above)
