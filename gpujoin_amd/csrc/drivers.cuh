@@ -96,10 +96,10 @@ __device__ __forceinline__ uint32_t xcd_logical_block(uint32_t nb) {
 // column lines its L2 must hold) spans a few partitions, the same ones in all the
 // windows.
 //
-// What bounds it: fabric lines where the tuples are sparse, else the L1 (the B-tree over 2^25
-// u64 keys: 8.6 accesses and 0.23 fabric lines a tuple).  Staging a run's separators in LDS
-// so that a tuple reads its leaf line alone took as long: the run's own chain (bounds,
-// descent, staging) costs what the inner levels do.
+// What bounds it: fabric lines where the tuples are sparse.  Where they are dense that is not
+// settled (the B-tree over 2^25 u64 keys: 8.6 L1 accesses and 0.23 fabric lines a tuple; but
+// staging a run's separators in LDS, so that a tuple reads its leaf line alone, took as
+// long).
 template <class Dev, class K>
 __global__ __launch_bounds__(256) void lookup_tuples_kernel(Dev d, const K* __restrict__ keys,
                                                             const uint64_t* __restrict__ start, uint32_t windows,

@@ -159,7 +159,7 @@ void lookup_partitioned(const gj_index& ix, const K* probes, uint64_t m, uint32_
                       windows_tuples(std::min(bm, window), window, sizeof(K), bits), res, tp, s, ix.cu);
       else
         launch_tuples(d, tkeys, start, 1u, nw * fan, windows_tuples(bm, window, sizeof(K), bits), res, tp, s, ix.cu);
-    }, (ix.n >> bits) > kLinesTupleKeys ? kLinesLookups : ~0ull);
+    });
     launch_unpartition(inv1, inv2, res, cap_b, bm, out + b0, s, ix.cu);
   }
 }

@@ -26,9 +26,10 @@ inline unsigned lookup_block(const gj_lookup_params& p) {
 // over the input ends with the slowest one and runs its waves in lockstep: 2^24 probes of
 // 2^20 u32 keys (learned, column layout) 260 -> 218 us, 2^28 of 2^26 u64 keys (lines)
 // 5.49 -> 5.29 ms.  Every workgroup stages the descriptor's LDS image, though, so above
-// kStageStep bytes of it a wave takes one more step for each (Harmonia's 15.9 KB at 2^20
-// u64 keys: 575 us with one step, 529 with four, 570 strided).  Never fewer workgroups
-// than fit on the chip at once, if there is a step for each.
+// kStageStep bytes of it a wave takes one more step for each (Harmonia, 2^24 probes, one step ->
+// so many -> resident workgroups that stride: 2^22 u32 keys 290 -> 264 -> 280 us, 2^20 u64 345
+// -> 339 -> 367; binary search, 2^20 u32 235 -> 224 -> 243).  Never fewer workgroups than fit
+// on the chip at once, if there is a step for each.
 // HIP takes fewer than 2^32 threads in a launch, so beyond that many items waves take more steps.
 constexpr uint64_t kStageStep = 8192;
 constexpr uint64_t max_blocks(unsigned threads) { return 0xFFFFFFFFull / threads / 8 * 8; }  // whole XCD rounds
@@ -140,11 +141,11 @@ template <class K> void build_extended(gj_index& ix, hipStream_t s);
 //              keys 66 -> 68, of 257 keys 77 -> 68; u64 65 keys 74 -> 63, 9 keys 57 -> 63
 //   aggregates one or two probes a wave (plain strategy, 30 M rows): buckets of 257 u32 keys 203
 //              -> 227, of 1025 keys 239 -> 224; lane_refill, 257 keys, 61 -> 54
-//   tuples     the tuples of a partition share the lines of its keys, so it is the keys per
-//              partition that count: 2^22 probes, windows of 2^20, of 1024 keys (2^18 u32 keys, fan-out
-//              2^8) 116 -> 119, of 4096 keys (2^22, 2^10) 175 -> 158, of 2^16 (2^20, 2^4) 215 -> 111;
-//              u64 of 256 keys (2^18, 2^10) 139 -> 144, of 4096 208 -> 205, of 2^16 234 -> 125
-constexpr uint64_t kLinesLookups = 8, kLinesBatches = 128, kLinesAggregates = 512, kLinesTupleKeys = 1024;
+//   tuples     as lookups, however few keys a partition has: its tuples share the lines of its keys
+//              only where the keys spread evenly over the partitions (2^22 probes, windows of 2^20,
+//              uniform keys of 2^18 u32 and fan-out 2^8 115 -> 119, 2^18 u64 and 2^10 138 -> 138; lognormal
+//              ones 220 -> 127 and 239 -> 131, 2^22 u64 and 2^12 597 -> 224)
+constexpr uint64_t kLinesLookups = 8, kLinesBatches = 128, kLinesAggregates = 512;
 
 // Few probes over small buckets wait for the longest chain of loads, and halving's loads hit
 // the L1 from the third last on: binary search of one batch goes by lines from this many

@@ -1,6 +1,6 @@
 """Binary search on both sides of the rules that choose between halving and reading lines:
-partitions of 1024 keys and a few more, join-aggregate buckets of 512 and 513 keys, batch
-plans over buckets of 128 and 129 keys with batches on both sides of the halvings bound."""
+join-aggregate buckets of 512 and 513 keys, batch plans over buckets of 128 and 129 keys with
+batches on both sides of the halvings bound; partitions of 1024 keys and a few more."""
 import numpy as np
 import pytest
 
