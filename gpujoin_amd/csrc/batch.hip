@@ -1201,6 +1201,8 @@ void enqueue_plan(gj_batch_plan& pl, hipStream_t s, GraphLanes* gl = nullptr) {
   const gj_index& ix = *pl.ix;
   if (pl.aggregate) {
     fill_bytes(pl.results, 0, pl.fact.size() * sizeof(gj_agg_result), s);
+    uint64_t rows = 0;
+    for (const FactBatchDev& b : pl.fact) rows += b.rows;
     with_index_dev<uint32_t>(ix, [&](auto d) {
       using Dev = decltype(d);
       if (pl.mode == GJ_BATCH_PERSISTENT) {
@@ -1231,7 +1233,7 @@ void enqueue_plan(gj_batch_plan& pl, hipStream_t s, GraphLanes* gl = nullptr) {
         }
         if (gl) GJ_HIP_CHECK(gl->join(s));
       }
-    }, kLinesAggregates);
+    }, pl.mode == GJ_BATCH_PERSISTENT ? agg_lines_above(ix, GJ_AGG_LANE_REFILL, rows) : kLinesAggregates);
     return;
   }
   dispatch_key(ix.key_bytes, [&]<class K>() {
@@ -1354,7 +1356,7 @@ int gj_join_aggregate(const gj_index* index, const gj_fact_batch* batch, const g
       partial.reserve(agg_partial_cap(index->cu) * sizeof(AggPartial));
       launch_join_agg_strategy(params->strategy, d, b, params->date_lo, params->date_hi, params->d_flag, index->cu,
                                partial.as<AggPartial>(), s);
-    }, kLinesAggregates);
+    }, agg_lines_above(*index, params->strategy, batch->rows));
   });
 }
 
@@ -1372,7 +1374,7 @@ int gj_join_aggregate_noalloc(const gj_index* index, const gj_fact_batch* batch,
     with_index_dev<uint32_t>(*index, [&](auto d) {
       launch_join_agg_strategy(params->strategy, d, b, params->date_lo, params->date_hi, params->d_flag, index->cu,
                                partial, S(stream), kNoAllocPartials);
-    }, kLinesAggregates);
+    }, agg_lines_above(*index, params->strategy, batch->rows));
   });
 }
 

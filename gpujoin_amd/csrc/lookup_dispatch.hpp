@@ -139,8 +139,13 @@ template <class K> void build_extended(gj_index& ix, hipStream_t s);
 //   lookups    2^22 probes, plain: buckets of 9 u32 keys 64 -> 55, of 9 u64 keys 100 -> 56
 //   batches    64 batches of 64 to 70000 probes in one persistent launch: buckets of 65 u32
 //              keys 66 -> 68, of 257 keys 77 -> 68; u64 65 keys 74 -> 63, 9 keys 57 -> 63
-//   aggregates one or two probes a wave (plain strategy, 30 M rows): buckets of 257 u32 keys 203
-//              -> 227, of 1025 keys 239 -> 224; lane_refill, 257 keys, 61 -> 54
+//   aggregates one or two probes a wave (plain strategy, 30 M rows): buckets of 257 u32 keys 193
+//              -> 206, of 409 keys 210 -> 208.  Whole waves, so agg_lines_above goes by the strategy:
+//              lookup-first, 8 M rows: 17 keys 176 -> 173, 65 keys 198 -> 176, 409 keys 239 -> 184;
+//              partitioned, 257 keys, 112 -> 117; lane refill and sorted by their rows: 257 keys and
+//              1 M rows 12.6 -> 14.0 and 16.5 -> 17.5, 12 M 29.2 -> 28.1 and 41.7 -> 39.9, 30 M 59.5 ->
+//              53.4 and 82.6 -> 83.1; lane refill in one persistent launch, 64 batches of 20000 rows
+//              33.8 -> 35.6, of 300000 94.6 -> 93.6
 //   tuples     as lookups, however few keys a partition has: its tuples share the lines of its keys
 //              only where the keys spread evenly over the partitions (2^22 probes, windows of 2^20,
 //              uniform keys of 2^18 u32 and fan-out 2^8 115 -> 119, 2^18 u64 and 2^10 138 -> 138; lognormal
@@ -166,6 +171,15 @@ bool short_column(const gj_index& ix) {
 template <class K>
 ShortDev<K> short_dev(const gj_index& ix) {
   return {static_cast<const K*>(ix.d_col), ix.n};
+}
+
+// The same for a join-aggregate of `rows` fact rows in one launch.
+constexpr uint64_t kLinesLookupFirst = 16, kLinesRowHalvings = 5ull << 24;
+inline uint64_t agg_lines_above(const gj_index& ix, uint32_t strategy, uint64_t rows) {
+  if (strategy == GJ_AGG_LOOKUP_FIRST) return kLinesLookupFirst;
+  const bool many = ix.kind == GJ_BINARY_SEARCH && rows * ilog2_ceil(ix.sample_step) >= kLinesRowHalvings;
+  const bool refills = strategy == GJ_AGG_LANE_REFILL || strategy == GJ_AGG_SORTED;
+  return refills && many ? kLinesLookups : kLinesAggregates;
 }
 
 // Calls f(descriptor) with the device descriptor of the index (every kind).

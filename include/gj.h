@@ -127,7 +127,8 @@ typedef struct gj_index_params {
  *                     build's measured max_lines.  About 12.8 bytes per 8-byte key at the default
  *                     load, against the column's 8.
  *   GJ_LAYOUT_AUTO    lines for a column of 16 MiB or more (smaller ones are served from the
- *                     caches, where the column's denser lines win) when the build's mean lines per
+ *                     caches, without a second copy of their keys; GJ_LAYOUT_LINES can be the
+ *                     faster one there too) when the build's mean lines per
  *                     present key stays at most 1.10, no key needs more than 4 lines and the line
  *                     copy fits; else column.  Always column with GJ_PLACE_HOST (the line copy
  *                     would put every key read on the host link) */
@@ -145,7 +146,8 @@ void gj_index_params_default(gj_index_params* p);
 /* Lookup parameters.  Zero selects the default / autotuned value. */
 typedef struct gj_lookup_params {
   gj_approach approach;
-  uint32_t block_size;       /* threads per block, default 256 */
+  uint32_t block_size;       /* threads per block: 64, 128, 192 or 256, default 256; the blockwise-sorting
+                                driver checks it and always takes 256 */
   uint32_t grid_blocks;      /* 0 = enough to cover the input (plain) or 4 x CUs (persistent kinds);
                                 the partitioned driver's lookup then uses one workgroup per CU
                                 when the column is page-locked host memory */

@@ -1,6 +1,7 @@
 """Binary search on both sides of the rules that choose between halving and reading lines:
 join-aggregate buckets of 512 and 513 keys, batch plans over buckets of 128 and 129 keys with
-batches on both sides of the halvings bound; partitions of 1024 keys and a few more."""
+batches on both sides of the halvings bound; partitions of 1024 keys and a few more; aggregates
+on both sides of the row bound."""
 import numpy as np
 import pytest
 
@@ -71,5 +72,50 @@ def test_plans(gj, orc, gpu, dt, n, mode):
         plan.run()
         gj.synchronize()
         assert np.array_equal(out.numpy(), want)
+    plan.close()
+    idx.close()
+
+
+@pytest.mark.parametrize("dim", [2048 * 16, 2048 * 17, 300_000])
+@pytest.mark.parametrize("strategy", ["lane_refill", "sorted", "lookup_first"])
+def test_aggregate_by_rows(gj, orc, gpu, dim, strategy):
+    # lane refill and sorted read lines from 5 * 2^24 halvings over their rows on: 9 or 10 a row at
+    # 300000 keys, 4 or 5 at 32768; lookup-first in buckets of 17 keys
+    key, flag = gj.gen_dimension(dim, 5)
+    skey, sflag = gj.sort_dimension(key, flag)
+    fact = gj.gen_fact(21_000_001, dim + dim // 7, 2557, 90000, 10500000, 10, 6)
+    idx = gj.Index("binary_search", gj.DeviceArray.from_numpy(skey))
+    d, dflag = [gj.DeviceArray.from_numpy(a) for a in fact], gj.DeviceArray.from_numpy(sflag)
+    res = gj.DeviceArray(4, np.int64)
+    for rows in (1_000_003, 9_000_001, 21_000_001):
+        res.fill(0)
+        gj.join_aggregate(idx, *d, dflag, 100, 130, res, strategy=strategy, rows=rows)
+        gj.synchronize()
+        want = orc.join_aggregate(skey, sflag, *[a[:rows] for a in fact], 100, 130)
+        assert tuple(int(v) for v in res.numpy()[:3]) == want, rows
+    idx.close()
+
+
+@pytest.mark.parametrize("sizes", [[1000, 70, 30_000], [1000, 9_000_001, 5_000_003]])
+@pytest.mark.parametrize("mode", [_lib.BATCH_LAUNCH, _lib.BATCH_GRAPH, _lib.BATCH_PERSISTENT])
+def test_aggregate_plans(gj, orc, gpu, sizes, mode):
+    dim = 300_000
+    key, flag = gj.gen_dimension(dim, 5)
+    skey, sflag = gj.sort_dimension(key, flag)
+    fact = gj.gen_fact(sum(sizes), dim + dim // 7, 2557, 90000, 10500000, 10, 6)
+    idx = gj.Index("binary_search", gj.DeviceArray.from_numpy(skey))
+    d, dflag = [gj.DeviceArray.from_numpy(a) for a in fact], gj.DeviceArray.from_numpy(sflag)
+    res = gj.DeviceArray(4 * len(sizes), np.int64)
+    starts = np.concatenate([[0], np.cumsum(sizes)]).astype(int)
+    plan = gj.AggregatePlan(idx, [tuple(a.offset(int(s)) for a in d) + (z,) for s, z in zip(starts, sizes)], dflag, 100, 130,
+                            res, mode)
+    for _ in range(2):
+        res.fill(0x5A)
+        plan.run()
+        gj.synchronize()
+        got = res.numpy().reshape(-1, 4)
+        for i, z in enumerate(sizes):
+            want = orc.join_aggregate(skey, sflag, *[a[starts[i]:starts[i] + z] for a in fact], 100, 130)
+            assert tuple(int(v) for v in got[i, :3]) == want, i
     plan.close()
     idx.close()
