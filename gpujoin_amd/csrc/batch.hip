@@ -1236,6 +1236,8 @@ void enqueue_plan(gj_batch_plan& pl, hipStream_t s, GraphLanes* gl = nullptr) {
     }, pl.mode == GJ_BATCH_PERSISTENT ? agg_lines_above(ix, GJ_AGG_LANE_REFILL, rows) : kLinesAggregates);
     return;
   }
+  uint64_t probes = 0;
+  for (const ProbeBatchDev& b : pl.probe) probes += b.m;
   dispatch_key(ix.key_bytes, [&]<class K>() {
     with_index_dev<K>(ix, [&](auto d) {
       using Dev = decltype(d);
@@ -1266,7 +1268,7 @@ void enqueue_plan(gj_batch_plan& pl, hipStream_t s, GraphLanes* gl = nullptr) {
         }
         if (gl) GJ_HIP_CHECK(gl->join(s));
       }
-    }, pl.mode == GJ_BATCH_PERSISTENT ? kLinesBatches : kLinesLookups);
+    }, pl.mode == GJ_BATCH_PERSISTENT ? plan_lines_above(ix, probes) : kLinesLookups);
   });
 }
 

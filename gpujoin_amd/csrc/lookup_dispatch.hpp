@@ -137,8 +137,10 @@ template <class K> void build_extended(gj_index& ix, hipStream_t s);
 // ones.  Lines cost instructions and registers and save dependent loads, so the line lies
 // where a caller's waves are full and wait for those loads (halving -> lines, us):
 //   lookups    2^22 probes, plain: buckets of 9 u32 keys 64 -> 55, of 9 u64 keys 100 -> 56
-//   batches    64 batches of 64 to 70000 probes in one persistent launch: buckets of 65 u32
-//              keys 66 -> 68, of 257 keys 77 -> 68; u64 65 keys 74 -> 63, 9 keys 57 -> 63
+//   batches    in one persistent launch, 64 of 2000 probes: buckets of 64 u32 keys 23.6 -> 32.4, of
+//              256 keys 26.8 -> 33.8; 64 of 64 to 70000: 65 u32 keys 66 -> 68, 257 keys 77 -> 68, 65 u64
+//              keys 74 -> 63, 9 keys 57 -> 63.  As lookups where the launch has many (plan_lines_above):
+//              8 of 2^20, 64 u32 keys 287 -> 138, 32 u64 keys 251 -> 149
 //   aggregates one or two probes a wave (plain strategy, 30 M rows): buckets of 257 u32 keys 193
 //              -> 206, of 409 keys 210 -> 208.  Whole waves, so agg_lines_above goes by the strategy:
 //              lookup-first, 8 M rows: 17 keys 176 -> 173, 65 keys 198 -> 176, 409 keys 239 -> 184;
@@ -171,6 +173,13 @@ bool short_column(const gj_index& ix) {
 template <class K>
 ShortDev<K> short_dev(const gj_index& ix) {
   return {static_cast<const K*>(ix.d_col), ix.n};
+}
+
+// The same for all batches of a persistent launch, `probes` together.
+constexpr uint64_t kLinesPlanHalvings = 5ull << 22;
+inline uint64_t plan_lines_above(const gj_index& ix, uint64_t probes) {
+  const bool many = ix.kind == GJ_BINARY_SEARCH && probes * ilog2_ceil(ix.sample_step) >= kLinesPlanHalvings;
+  return many ? kLinesLookups : kLinesBatches;
 }
 
 // The same for a join-aggregate of `rows` fact rows in one launch.

@@ -119,3 +119,27 @@ def test_aggregate_plans(gj, orc, gpu, sizes, mode):
             assert tuple(int(v) for v in got[i, :3]) == want, i
     plan.close()
     idx.close()
+
+
+@pytest.mark.parametrize("dt", [np.uint32, np.uint64])
+@pytest.mark.parametrize("many", [2_621_439, 2_621_441])
+def test_persistent_plan_by_probes(gj, orc, gpu, dt, many):
+    # persistent plans read lines in smaller buckets from 5 * 2^22 halvings over all their probes
+    # on: 8 a probe over the 256 keys of a bucket here
+    rng = np.random.default_rng(3)
+    keys = _column((1024 if dt == np.uint64 else 2048) * 256 - 5, dt, rng)
+    sizes = [many - 1_000_100, 1_000_000, 100]
+    probes = rng.choice(keys, many)
+    probes[::9] += dt(1)
+    dp, out = gj.DeviceArray.from_numpy(probes), gj.DeviceArray(many, np.uint32)
+    idx = gj.Index("binary_search", gj.DeviceArray.from_numpy(keys))
+    starts = np.concatenate([[0], np.cumsum(sizes)]).astype(int)
+    plan = gj.LookupPlan(idx, [(dp.offset(int(s)), out.offset(int(s)), z) for s, z in zip(starts, sizes)],
+                         _lib.BATCH_PERSISTENT)
+    for _ in range(2):
+        out.fill(0x5A)
+        plan.run()
+        gj.synchronize()
+        assert np.array_equal(out.numpy(), orc.lookup_lower_bound(keys, probes))
+    plan.close()
+    idx.close()
